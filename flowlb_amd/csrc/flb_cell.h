@@ -36,11 +36,44 @@ struct Quotient<float> {
   }
 };
 
+// The collision below is written with its fused multiply-adds explicit and
+// contraction off: which products the compiler fuses by itself depends on the
+// code around the expression, and the kernels that share these functions (one
+// step or several per pass, one domain or a batch) have to agree bit for bit.
+__device__ __forceinline__ float fused(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fused(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
 // Equilibrium minus weights (feq_i - w_i), calculateEquilibriumDDF2Q9
 // (src/cuda/cellCalculations.cuh:32-52) rearranged for shifted storage:
 // feq_i - w_i = w_i * ((rho - 1) + rho * A_i).  R is the arithmetic type.
+// `unit` (here and below) is a power of two that the populations are held
+// times of: it scales them exactly, so the values are those of unit 1.
 template <class R>
-__device__ __forceinline__ void equilibrium_shifted(R rho, R rho1, R ux, R uy, R* fe) {
+__device__ __forceinline__ void equilibrium_shifted(R rho, R rho1, R ux, R uy, R* fe,
+                                                    R unit = R(1)) {
+#pragma clang fp contract(off)
+  const R u2 = R(3) * fused(uy, uy, ux * ux);
+  const R ax = R(3) * ux, ay = R(3) * uy;
+  const R a0 = fused(uy, R(-3), ax), a1 = fused(uy, R(3), ax);
+  const R h = R(0.5f) * u2;
+  const R w0 = wgt_r<R>(0) * unit, w1 = wgt_r<R>(1) * unit, w5 = wgt_r<R>(5) * unit;
+  const R q = R(0.5f);
+  const auto pair = [&](R w, R a, R& plus, R& minus) {
+    const R qa = q * a;
+    plus = w * fused(rho, fused(a, qa, a - h), rho1);
+    minus = w * fused(rho, fused(a, qa, -a - h), rho1);
+  };
+  fe[0] = w0 * fused(-rho, h, rho1);
+  pair(w1, ax, fe[1], fe[2]);
+  pair(w1, ay, fe[3], fe[4]);
+  pair(w5, a1, fe[5], fe[6]);
+  pair(w5, a0, fe[7], fe[8]);
+}
+
+// The same where no other kernel repeats the cell's arithmetic (free-surface
+// passes 1 and 3): contraction left to the compiler.
+template <class R>
+__device__ __forceinline__ void equilibrium_surface(R rho, R rho1, R ux, R uy, R* fe) {
   const R u2 = R(3) * (ux * ux + uy * uy);
   const R ax = R(3) * ux, ay = R(3) * uy;
   const R a0 = ax - ay, a1 = ax + ay;
@@ -58,18 +91,25 @@ __device__ __forceinline__ void equilibrium_shifted(R rho, R rho1, R ux, R uy, R
   fe[8] = w5 * (rho1 + rho * (-a0 - h + q * a0 * a0));
 }
 
+// c_i . v, as a sum (no products with 0 and 1).
+template <class R>
+__device__ __forceinline__ R along(int i, R vx, R vy) {
+  const R a = cx(i) < 0 ? -vx : vx, b = cy(i) < 0 ? -vy : vy;
+  return cx(i) == 0 ? b : (cy(i) == 0 ? a : a + b);
+}
+
 // Guo forcing terms, calculateForcingTerms2D (src/cuda/cellCalculations.cuh:64-73),
 // with the reference's literal 0.33333334f.  The force is a float constant
 // there, so c_i . F is formed in float also in the double path.
 template <class R>
-__device__ __forceinline__ void guo_terms(R ux, R uy, float gx, float gy, R* fi) {
-  const R uF = R(-0.33333334f) * (ux * R(gx) + uy * R(gy));
-  fi[0] = R(9.0f) * wgt_r<R>(0) * uF;
+__device__ __forceinline__ void guo_terms(R ux, R uy, float gx, float gy, R* fi, R unit = R(1)) {
+#pragma clang fp contract(off)
+  const R uF = R(-0.33333334f) * fused(R(gy), uy, ux * R(gx));
+  fi[0] = R(9.0f) * wgt_r<R>(0) * unit * uF;
 #pragma unroll
   for (int i = 1; i < 9; i++) {
-    const float cF = float(cx(i)) * gx + float(cy(i)) * gy;
-    fi[i] = R(9.0f) * wgt_r<R>(i) *
-            (R(cF) * (R(cx(i)) * ux + R(cy(i)) * uy + R(0.33333334f)) + uF);
+    fi[i] = R(9.0f) * wgt_r<R>(i) * unit *
+            fused(R(along(i, gx, gy)), along(i, ux, uy) + R(0.33333334f), uF);
   }
 }
 
@@ -284,6 +324,119 @@ __device__ __forceinline__ void store_outgoing(const Params& p, const uint32_t* 
   }
 }
 
+// Force step of a cell: the velocity shift of Guo's scheme and its terms fi.
+// With Brinkman drag (alpha > 0, no reference counterpart; FP32 and FP64
+// storage only) G = F - alpha rho u with the half-force shift solved for u.
+// Returns whether the collision is forced.
+template <class R>
+__device__ __forceinline__ bool apply_force(const Params& p, bool use_force, bool brinkman, R a,
+                                            R rho, const Quotient<R>& over_rho, R& ux, R& uy,
+                                            R* fi, R unit = R(1)) {
+#pragma clang fp contract(off)
+  if (brinkman) {
+    const R gx0 = R(use_force ? p.fx : 0.0f), gy0 = R(use_force ? p.fy : 0.0f);
+    const R rhol2 = over_rho(R(0.5f));
+    const R s = R(1) / fused(R(0.5f), a, R(1)), ar = a * rho;
+    ux = fused(gx0, rhol2, ux) * s;
+    uy = fused(gy0, rhol2, uy) * s;
+    guo_terms<R>(ux, uy, float(fused(-ar, ux, gx0)), float(fused(-ar, uy, gy0)), fi, unit);
+    return true;
+  }
+  if (use_force) {
+    const R rhol2 = over_rho(R(0.5f));
+    ux = fused(R(p.fx), rhol2, ux);
+    uy = fused(R(p.fy), rhol2, uy);
+    guo_terms<R>(ux, uy, p.fx, p.fy, fi, unit);
+    return true;
+  }
+  return false;
+}
+
+// Relaxation rate of the subgrid model for a cell off equilibrium by g - fe.
+// 1/tau is a float constant in the reference also for PRECISION = 64, and the
+// Smagorinsky correction goes through float sqrtf (lbmKernel2D.cu:414-442).
+template <class R>
+__device__ __forceinline__ float smagorinsky_rate(float inv_tau, R rho, const R* fe, const R* g,
+                                                  R unit) {
+#pragma clang fp contract(off)
+  R hxx = R(0), hyy = R(0), hxy = R(0);
+#pragma unroll
+  for (int i = 1; i < 9; i++) {
+    const R d = g[i] - fe[i];
+    if (cx(i) != 0) hxx += d;
+    if (cy(i) != 0) hyy += d;
+    if (cx(i) * cy(i) > 0) hxy += d;
+    if (cx(i) * cy(i) < 0) hxy -= d;
+  }
+  hxx *= R(1) / unit;
+  hyy *= R(1) / unit;
+  hxy *= R(1) / unit;
+  const R Q = fused(hxy, R(2.0f) * hxy, fused(hxx, hxx, hyy * hyy));
+  const float tau = 1.0f / inv_tau;
+  const R strain = R(0.54037965f * sqrtf(float(Q))) / rho;
+  // The float build fuses tau^2; for doubles tau^2 is a float product.
+  const float sum = sizeof(R) == 4 ? fused(tau, tau, float(strain)) : float(R(tau * tau) + strain);
+  return 2.0f / (tau + sqrtf(sum));
+}
+
+// Collision of a cell's populations g towards the equilibrium fe (inlet and
+// outlet cells, io, take the equilibrium itself): optional Smagorinsky, then
+// SRT or TRT.
+template <class R>
+__device__ __forceinline__ void relax(float inv_tau, int collision, bool smagorinsky, bool io,
+                                      bool forced, R rho, const R* fe, const R* fi, R* g,
+                                      R unit = R(1)) {
+#pragma clang fp contract(off)
+  if (smagorinsky) inv_tau = smagorinsky_rate<R>(inv_tau, rho, fe, g, unit);
+  if (io) {
+#pragma unroll
+    for (int i = 0; i < 9; i++) g[i] = fe[i];
+  } else if (collision == 0) {  // SRT
+    const R omc = R(1.0f - inv_tau), om = R(inv_tau);
+#pragma unroll
+    for (int i = 0; i < 9; i++) g[i] = fused(fe[i], om, omc * g[i]);
+    if (forced) {
+      const R tl = R(1.0f - 0.5f * inv_tau);
+#pragma unroll
+      for (int i = 0; i < 9; i++) g[i] = fused(fi[i], tl, g[i]);
+    }
+  } else if (!forced || collision == 2) {
+    // TRT, magic parameter 1/4 (:475-510).  As written a forced TRT step only
+    // streams; collision 2 (no reference counterpart) defines the forced
+    // branch: Guo terms split into the pair-symmetric part, weighted 1 - w+/2,
+    // and the antisymmetric part, weighted 1 - w-/2 (SRT + Guo when w+ = w-).
+    // The reference keeps these temporaries in float also for PRECISION = 64.
+    const float ip = inv_tau;
+    const float in = 1.0f / (0.25f / (1.0f / inv_tau - 0.5f) + 0.5f);
+    const float hp = 0.5f * ip, hn = 0.5f * in;
+    // a - h * v: one fused step in the float build; for doubles h * v is a
+    // float product.
+    const auto less = [](R a, float h, float v) {
+      return sizeof(R) == 4 ? R(fused(-v, h, float(a))) : a - R(h * v);
+    };
+    g[0] = fused(-(g[0] - fe[0]), R(ip), g[0]);
+#pragma unroll
+    for (int i = 1; i < 9; i += 2) {
+      const float sym = float(g[i] - fe[i] + g[i + 1] - fe[i + 1]);
+      const float fa = float(g[i] - g[i + 1]);
+      const float fea = float(fe[i] - fe[i + 1]);
+      g[i] = less(less(g[i], hp, sym), hn, fa - fea);
+      g[i + 1] = less(less(g[i + 1], hp, sym), hn, fea - fa);
+    }
+    if (forced) {
+      const R ap = R(1.0f - hp), an = R(1.0f - hn);
+      g[0] = fused(fi[0], ap, g[0]);
+#pragma unroll
+      for (int i = 1; i < 9; i += 2) {
+        const R fs = R(0.5f) * (fi[i] + fi[i + 1]), fd = R(0.5f) * (fi[i] - fi[i + 1]);
+        const R anti = fd * an;
+        g[i] = g[i] + fused(fs, ap, anti);
+        g[i + 1] = g[i + 1] + fused(fs, ap, -anti);
+      }
+    }
+  }
+}
+
 // ------------------------------------------------------------- stream-collide
 // d_StreamCollide2D (src/cuda/lbmKernel2D.cu:305-519).  MOM: write the
 // density/velocity readback fields (always done in free-surface runs, where
@@ -468,25 +621,10 @@ __device__ __forceinline__ void stream_collide_cell(const Params& p, const Cell 
     else if ((m_if < -0.001f) || not_fluid) p.flags[n] = (fl & uint8_t(~kFGI)) | kIG;
   }
   R fi[9];
-  bool forced = false;
-  if (!FS && p.alpha && !io) {  // Brinkman drag is offered for monofluid handles only
-    // Brinkman drag G = F - alpha rho u with the Guo half-force shift solved
-    // for u (no reference counterpart; FP32 storage only).
-    const R a = R(p.alpha[n]);
-    const R gx0 = R(p.use_force ? p.fx : 0.0f), gy0 = R(p.use_force ? p.fy : 0.0f);
-    const R rhol2 = over_rho(R(0.5f));
-    const R s = R(1) / (R(1) + R(0.5f) * a);
-    ux = (ux + rhol2 * gx0) * s;
-    uy = (uy + rhol2 * gy0) * s;
-    guo_terms<R>(ux, uy, float(gx0 - a * rho * ux), float(gy0 - a * rho * uy), fi);
-    forced = true;
-  } else if (p.use_force) {
-    const R rhol2 = over_rho(R(0.5f));
-    ux = ux + rhol2 * R(p.fx);
-    uy = uy + rhol2 * R(p.fy);
-    guo_terms<R>(ux, uy, p.fx, p.fy, fi);
-    forced = true;
-  }
+  // Brinkman drag is offered for monofluid handles only.
+  const bool brinkman = !FS && p.alpha && !io;
+  const bool forced = apply_force<R>(p, p.use_force != 0, brinkman, brinkman ? R(p.alpha[n]) : R(0),
+                                     rho, over_rho, ux, uy, fi);
   if (MOM || FS) {
     // Free surface: every cell's density is read by pass 4, but the velocity
     // of a fluid cell only at readback -- pass 1 reads the velocity of
@@ -525,63 +663,7 @@ __device__ __forceinline__ void stream_collide_cell(const Params& p, const Cell 
     // absorbs the weight error instead: sum_i fe_i = rho - 1.
     fe[0] = rho1 - (((fe[1] + fe[2]) + (fe[3] + fe[4])) + ((fe[5] + fe[6]) + (fe[7] + fe[8])));
   }
-  // 1/tau is a float constant in the reference also for PRECISION = 64, and
-  // the Smagorinsky correction goes through float sqrtf (:414-442).
-  float inv_tau = p.inv_tau;
-  if (p.smagorinsky) {
-    R hxx = R(0), hyy = R(0), hxy = R(0);
-#pragma unroll
-    for (int i = 1; i < 9; i++) {
-      const R d = g[i] - fe[i];
-      hxx += R(cx(i) * cx(i)) * d;
-      hyy += R(cy(i) * cy(i)) * d;
-      hxy += R(cx(i) * cy(i)) * d;
-    }
-    const R Q = hxx * hxx + hyy * hyy + R(2.0f) * hxy * hxy;
-    const float tau = 1.0f / inv_tau;
-    inv_tau = 2.0f / (tau + sqrtf(float(R(tau * tau) + R(0.54037965f * sqrtf(float(Q))) / rho)));
-  }
-  if (io) {
-#pragma unroll
-    for (int i = 0; i < 9; i++) g[i] = fe[i];
-  } else if (p.collision == 0) {  // SRT
-    const float omc = 1.0f - inv_tau;
-    if (forced) {
-      const float tl = 1.0f - 0.5f * inv_tau;
-#pragma unroll
-      for (int i = 0; i < 9; i++) g[i] = R(omc) * g[i] + R(inv_tau) * fe[i] + R(tl) * fi[i];
-    } else {
-#pragma unroll
-      for (int i = 0; i < 9; i++) g[i] = R(omc) * g[i] + R(inv_tau) * fe[i];
-    }
-  } else if (!forced || p.collision == 2) {
-    // TRT, magic parameter 1/4 (:475-510).  As written a forced TRT step only
-    // streams; collision 2 (no reference counterpart) defines the forced
-    // branch: Guo terms split into the pair-symmetric part, weighted 1 - w+/2,
-    // and the antisymmetric part, weighted 1 - w-/2 (SRT + Guo when w+ = w-).
-    // The reference keeps these temporaries in float also for PRECISION = 64.
-    const float ip = inv_tau;
-    const float in = 1.0f / (0.25f / (1.0f / inv_tau - 0.5f) + 0.5f);
-    g[0] = g[0] - R(ip) * (g[0] - fe[0]);
-#pragma unroll
-    for (int i = 1; i < 9; i += 2) {
-      const float sym = float(g[i] - fe[i] + g[i + 1] - fe[i + 1]);
-      const float fa = float(g[i] - g[i + 1]);
-      const float fea = float(fe[i] - fe[i + 1]);
-      g[i] = g[i] - R(0.5f * ip * sym) - R(0.5f * in * (fa - fea));
-      g[i + 1] = g[i + 1] - R(0.5f * ip * sym) - R(0.5f * in * (fea - fa));
-    }
-    if (forced) {
-      const R ap = R(1.0f - 0.5f * ip), an = R(1.0f - 0.5f * in);
-      g[0] = g[0] + ap * fi[0];
-#pragma unroll
-      for (int i = 1; i < 9; i += 2) {
-        const R fs = R(0.5f) * (fi[i] + fi[i + 1]), fd = R(0.5f) * (fi[i] - fi[i + 1]);
-        g[i] = g[i] + (ap * fs + an * fd);
-        g[i + 1] = g[i + 1] + (ap * fs - an * fd);
-      }
-    }
-  }
+  relax<R>(p.inv_tau, p.collision, p.smagorinsky != 0, io != 0, forced, rho, fe, fi, g);
   if (!kRounded && S::kBytes == 4 && cons && !(fl & kInlet)) {
     // FP32 storage: the collision's float rounding would make the stored
     // populations carry slightly more or less than rho, which the next step's

@@ -4,7 +4,8 @@
 // of `pitch` cells (Nd = pitch * ny elements per plane of a cell field):
 //   f          9 planes x Np elements of the storage type (Np = Nd rounded up
 //              to 8 KiB plus 4 KiB: flb::plane_stride; every plane starts
-//              256-byte aligned)
+//              256-byte aligned); single phase: a second array of these, which
+//              a pass of several steps writes (prepare_march)
 //   flags[2]   Nd bytes each; free-surface pass 4 writes the second buffer
 //   rho, u     readback fields, 1 and 2 planes
 //   pub_rho[2], pub_u[2]   inlet/outlet neighbour values by step parity
@@ -24,6 +25,7 @@
 #include "flb_device.h"
 
 #include "flb_internal.h"
+#include "flb_march.h"
 
 // Device scratch of flb_flag_histogram_noalloc: its 256 flag counters, one
 // copy per GPU, held for the life of the process (2 KiB).  In host code this
@@ -331,6 +333,84 @@ uint32_t row_pitch(const flb_options* o, uint32_t nx) {
   return (nx + 63u) / 64u * 64u;
 }
 
+bool march_plain(const flb_handle* h) {
+  return h->opt.collision == FLB_SRT && !h->opt.smagorinsky && !h->opt.use_force && !h->alpha;
+}
+
+// Sets a single-phase handle up for the multi-step pass.  It is left to single
+// steps (f_alt null) where the pass's rules do not hold: an inlet cell in the
+// last column or an outlet cell in the first one reads the linear neighbour in
+// another row, and the pass needs as many rows as it does steps; or where the
+// second population array would take more than a quarter of the memory left (a
+// program that fills the device with handles keeps its room).
+int prepare_march(flb_handle* h, const uint8_t* flags) {
+  const uint32_t nx = h->nx, ny = h->ny;
+  if (ny < uint32_t(flb::kMarchMax)) return FLB_OK;
+  std::vector<uint8_t> io(nx, 0);  // columns with an inlet or outlet cell
+  for (uint32_t y = 0; y < ny; ++y) {
+    const uint8_t* row = flags + uint64_t(y) * nx;
+    if ((row[nx - 1] & FLB_INLET) || ((row[0] & FLB_OUTLET) && !(row[0] & FLB_INLET))) return FLB_OK;
+    for (uint32_t x = 0; x < nx; ++x) io[x] |= row[x] & (FLB_INLET | FLB_OUTLET);
+  }
+  const size_t bytes = 9 * h->Np * h->elem_bytes;
+  size_t left = 0, total = 0;
+  void* v = nullptr;
+  if (hipMemGetInfo(&left, &total) != hipSuccess || bytes > left / 4 ||
+      hipMalloc(&v, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return FLB_OK;
+  }
+  h->owned.push_back(v);
+  int rc;
+  for (int T = flb::kMarchMin; T <= flb::kMarchMax; ++T) {
+    const uint32_t cols = flb::march_columns(T), strips = (nx + cols - 1) / cols;
+    std::vector<uint32_t> order(strips);
+    for (uint32_t s = 0; s < strips; ++s) order[s] = s;
+    const auto split = std::stable_partition(order.begin(), order.end(), [&](uint32_t s) {
+      uint8_t any = 0;
+      for (uint32_t l = 0; l < flb::kMarchLanes; ++l)
+        any |= io[(uint64_t(s) * cols + l + uint64_t(T - 1) * (nx - 1)) % nx];
+      return any != 0;
+    });
+    h->march_io[T] = uint32_t(split - order.begin());
+    if ((rc = dev_alloc(h, &h->march_order[T], strips))) return rc;
+    if ((rc = upload(h, h->march_order[T], order.data(), strips * sizeof(uint32_t)))) return rc;
+  }
+  h->f_alt = v;
+  return FLB_OK;
+}
+
+// Shape of the passes of a run of steps.
+//
+// Rows per chunk.  A wavefront's chunk of r rows takes r + 2 (T - 1)
+// iterations and T (r + T - 1) step-rows, so long chunks waste less, while the
+// chip needs wavefronts on its 1024 SIMDs.  Measured with T = 4, us per step: 2048 x 512
+// FP32 (36 strips) 8.3, 7.2, 7.2, 8.6, 9.2 with 4, 8, 12, 16, 24 rows: best near
+// 1.5 wavefronts per SIMD (12 rows).  Where that gives long chunks, the chip
+// runs several rounds of wavefronts anyway and FP32 wants them short, so that
+// fewer rows are in flight: 8192 x 2048 79.8, 83.2, 84.3, 90.5 with 16, 24, 36,
+// 64 rows; FP16S, which is bound by the vector units, 70.6, 68.6, 66.1, 74.6.
+// Below four rows nothing is gained (512 x 128: 3.3 us with 1 to 4).
+//
+// Steps per pass.  T = 4 moves the fewest bytes and was the fastest from
+// 2048 x 512 on (8192 x 2048 FP32 80 us per step, with T = 3 110, with T = 2
+// about 150; single steps 196).  Grids that give less than 1.5 wavefronts per
+// SIMD at four rows are bound by the chain of a wavefront, T (r + T - 1)
+// step-rows: T = 3 takes 3.1 us per step on 512 x 128 and 3.5 on 1024 x 256,
+// T = 4 3.4 and 4.0.
+struct MarchShape {
+  int steps;
+  uint32_t rows;
+};
+MarchShape march_shape(const flb_handle* h) {
+  const uint64_t waves = uint64_t(h->cus) * 6;  // 1.5 per SIMD
+  const uint32_t least = 4, most = h->elem_bytes == 2 ? 36 : 16;
+  const uint32_t cols = flb::march_columns(flb::kMarchMax);
+  const uint64_t strip_rows = uint64_t((h->nx + cols - 1) / cols) * h->ny;
+  const uint64_t rows = (strip_rows + waves - 1) / waves;
+  return MarchShape{rows < least ? 3 : 4, uint32_t(std::min<uint64_t>(std::max<uint64_t>(rows, least), most))};
+}
+
 }  // namespace
 
 extern "C" {
@@ -525,6 +605,7 @@ int flb_create(const flb_options* opt, const uint8_t* flags, uint32_t nx, uint32
     if ((rc = upload(h, h->tile_pub, pub.data(), tiles * sizeof(uint32_t)))) return bail(rc);
     if ((rc = reset_work(h))) return bail(rc);
   }
+  if (!fs && (rc = prepare_march(h, flags))) return bail(rc);
   if ((rc = dev_alloc(h, &h->rho_init, Nd))) return bail(rc);
   if ((rc = dev_alloc(h, &h->u_init, 2 * Nd))) return bail(rc);
   const flb::Params pu = params(h, kUtilBlock);
@@ -724,6 +805,44 @@ static int enqueue_step(flb_handle* h, bool moments, hipEvent_t* ev) {
   return FLB_OK;
 }
 
+// T steps of a single-phase handle in one pass (flb_march.h).
+static int enqueue_march(flb_handle* h, int T, bool moments) {
+  const flb::Params p = params(h, int(flb::kMarchLanes));
+  const int last = int((h->t & 1u) ^ 1u);  // parity the step before published at
+  flb::March a{};
+  a.f_in = h->f;
+  a.f_out = h->f_alt;
+  a.pub_rho_in = h->pub_rho[last];
+  a.pub_u_in = h->pub_u[last];
+  a.pub_rho_out = h->pub_rho[last ^ 1];
+  a.pub_u_out = h->pub_u[last ^ 1];
+  a.odd = int32_t(h->t & 1u);
+  a.moments = moments;
+  const uint32_t cols = flb::march_columns(T);
+  constexpr uint32_t G = flb::kMarchWaves;
+  a.strips = (h->nx + cols - 1) / cols;
+  a.io_strips = h->march_io[T];
+  a.order = h->march_order[T];
+  a.rows = march_shape(h).rows;
+  a.chunks = (h->ny + a.rows - 1) / a.rows;
+  a.io_rows = (a.rows + G - 1) / G;
+  a.groups = (a.strips - a.io_strips + G - 1) / G;
+  a.group_magic = flb::div_magic(a.groups);
+  const uint32_t blocks = a.io_strips * a.chunks + (a.groups * a.chunks + 7u) / 8u * 8u;
+  hipLaunchKernelGGL(flb::get_march(h->opt.storage, T, march_plain(h)), dim3(blocks),
+                     dim3(64 * G), 0, h->stream, p, a);
+  FLB_HIP(h, hipGetLastError());
+  std::swap(h->f, h->f_alt);
+  // The last step published at the other index; after an even number of steps
+  // the next one looks for it at the same parity.
+  if (T % 2 == 0) {
+    std::swap(h->pub_rho[0], h->pub_rho[1]);
+    std::swap(h->pub_u[0], h->pub_u[1]);
+  }
+  h->t += uint64_t(T);
+  return FLB_OK;
+}
+
 }  // extern "C"
 
 namespace flb {
@@ -751,7 +870,17 @@ int flb_step(flb_handle* h, uint64_t nsteps) {
   if (!h) return FLB_ERR_ARGUMENT;
   const bool throttle = h->box_host != nullptr;
   constexpr uint64_t G = flb_handle::kGroup, R = flb_handle::kRing;
-  for (uint64_t k = 0; k < nsteps; ++k) {
+  for (uint64_t k = 0; k < nsteps;) {
+    const uint64_t left = nsteps - k;
+    if (h->f_alt && left > 1) {
+      // Passes of the shape's steps; a single step is not left over.
+      const uint64_t most = uint64_t(march_shape(h).steps);
+      const int T = int(left == most + 1 ? (left + 1) / 2 : std::min(left, most));
+      const int rc = enqueue_march(h, T, left == uint64_t(T));
+      if (rc) return rc;
+      k += uint64_t(T);
+      continue;
+    }
     // Free surface: steps go in groups of G (by lattice time, so across calls
     // too).  Starting group g, wait for the event recorded after group g - 2
     // (a slot never recorded, or recorded by an older group, returns at once),
@@ -764,6 +893,7 @@ int flb_step(flb_handle* h, uint64_t nsteps) {
     if (throttle && t % G == 0 && g >= 2) FLB_HIP(h, hipEventSynchronize(h->in_flight[(g - 2) % R]));
     const int rc = enqueue_step(h, k + 1 == nsteps, nullptr);
     if (rc) return rc;
+    ++k;
     if (throttle && t % G == G - 1) FLB_HIP(h, hipEventRecord(h->in_flight[g % R], h->stream));
   }
   return FLB_OK;

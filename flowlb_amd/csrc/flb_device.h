@@ -81,6 +81,8 @@ struct StoreF32 {
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, int(i * 4u), 0, 0);
   }
   __device__ static float round(float v) { return v; }  // value a store keeps
+  __device__ static float decode(T v) { return v; }
+  __device__ static T encode(float v) { return v; }
 };
 
 struct StoreF64 {
@@ -97,6 +99,8 @@ struct StoreF64 {
     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, int(i * 8u), 0, 0);
   }
   __device__ static double round(double v) { return v; }
+  __device__ static double decode(T v) { return v; }
+  __device__ static T encode(double v) { return v; }
 };
 
 // IEEE binary16, scaled by 2^15 so that the shifted populations (|f - w| < 1)
@@ -119,6 +123,8 @@ struct StoreF16S {
   __device__ static float round(float v) {
     return float(_Float16(v * 32768.0f)) * 3.0517578125e-05f;
   }
+  __device__ static float decode(T v) { return float(v) * 3.0517578125e-05f; }
+  __device__ static T encode(float v) { return _Float16(v * 32768.0f); }
 };
 
 // bfloat16 (upper half of an FP32), round to nearest even on store: gfx950's
@@ -144,6 +150,8 @@ struct StoreBF16S {
   __device__ static float round(float v) {
     return __uint_as_float(uint32_t(bits(v)) << 16);
   }
+  __device__ static float decode(T v) { return __uint_as_float(uint32_t(v) << 16); }
+  __device__ static T encode(float v) { return bits(v); }
 };
 
 // Tile of the fused free-surface passes 2-4: one block of kFsTileW x kFsTileH

@@ -43,6 +43,12 @@ ConvOut64Fn get_pop_to_f64(int storage);
 ConvInFn get_f32_to_pop(int storage);
 ConvIn64Fn get_f64_to_pop(int storage);
 HistFn get_flag_hist();
+
+// The multi-step pass (flb_march.h): `steps` in [kMarchMin, kMarchMax].
+struct March;
+using MarchFn = void (*)(const Params, const March);
+constexpr int kMarchMin = 2, kMarchMax = 4;
+MarchFn get_march(int storage, int steps, bool plain);
 }  // namespace flb
 
 struct flb_handle {
@@ -56,6 +62,12 @@ struct flb_handle {
   int field_bytes = 4;  // bytes per element of the cell fields (8 for FP64)
   hipStream_t stream = nullptr;
   void* f = nullptr;
+  // Single phase, the multi-step pass (flb_march.h): second population array
+  // (null where the pass is not used) and, per number of steps, the strips with
+  // those that hold an inlet or outlet column first and the number of these.
+  void* f_alt = nullptr;
+  uint32_t* march_order[flb::kMarchMax + 1] = {};
+  uint32_t march_io[flb::kMarchMax + 1] = {};
   uint8_t* flags[2] = {nullptr, nullptr};
   int cur = 0;
   float* rho = nullptr;

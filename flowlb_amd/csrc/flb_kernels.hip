@@ -171,7 +171,7 @@ __device__ __forceinline__ void fs1_cell(const Params& p, const Cell c) {
     ux = ux + rhol2 * R(p.fx);
     uy = uy + rhol2 * R(p.fy);
     R fe[9];
-    equilibrium_shifted<R>(R(1), R(0), ux, uy, fe);  // atmospheric equilibrium, rho = 1
+    equilibrium_surface<R>(R(1), R(0), ux, uy, fe);  // atmospheric equilibrium, rho = 1
 #pragma unroll
     for (int i = 1; i < 9; i += 2) {
       R d = R(0);
@@ -348,7 +348,7 @@ __device__ __forceinline__ uint8_t update_cell(const Params& p, const uint8_t* f
     ux = ux + rhol2 * R(p.fx);
     uy = uy + rhol2 * R(p.fy);
     R fe[9];
-    equilibrium_shifted<R>(ar, ar - R(1), ux, uy, fe);
+    equilibrium_surface<R>(ar, ar - R(1), ux, uy, fe);
     store_outgoing<S, ODD, false>(p, nb, fe);  // the update is short of scalar registers
   }
   // A fluid cell carries its mass as the deviation from rho in the

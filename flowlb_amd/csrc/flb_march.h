@@ -1,0 +1,395 @@
+// flb_march.h -- several lattice steps of a single-phase domain in one pass
+// over memory (device code shared by flb_march.hip and flb_batch.hip).
+//
+// A wavefront owns a strip of columns, one column per lane, and marches up a
+// chunk of rows.  In one iteration it loads the next row's populations and
+// runs step 1 on that row, step 2 on the row below it, ... step T on the row
+// T - 1 below, whose populations it stores.  What step s needs of step s - 1
+// comes from registers: the populations along x of the row itself (kept one
+// iteration), those moving up of the row below (kept two) and those moving down
+// of the row above (just computed), each shifted by a lane for its x component
+// (DPP wavefront shift).  No LDS, no barrier; wavefronts are independent.
+//
+// Dependencies reach one cell per step, so of the 64 columns a wavefront loads
+// the 64 - 2 (T - 1) inner ones are its own, and it starts T - 1 rows below its
+// chunk and ends T - 1 above.  Neighbouring wavefronts read those halos from
+// the state before the pass, so the pass reads one population array and
+// writes another.  The cells' results are those of T single steps, bit for
+// bit: the same per-cell arithmetic in the same order, 16-bit storage rounded
+// between the steps as a store and a load would, walls returning what they
+// receive (what they leave in place in the in-place slot layout).
+//
+// What bounds it: a single step moves 18 values per cell (72 bytes in FP32) and is
+// bound by memory on large grids and by the launch on small ones.  T = 4 steps in
+// one pass move 18 x 61 / 58 values in all, a quarter, and the vector units become
+// the bound: about 110 instructions per step and row of 64 columns, 10 % of them
+// for halo columns.  Measured, us per step, single steps / passes: 8192 x 2048
+// FP32 226 / 77 (4.0 TB/s, 0.7 of the vector rate), FP16S 118 / 62, 2001 x 401
+// FP64 16.4 / 10.0; 512 x 128 FP32 3.8 / 3.3 for one handle alone and 3.7 / 1.3 with
+// three handles stepping side by side.
+#pragma once
+
+#include "flb_cell.h"
+
+namespace flb {
+
+constexpr uint32_t kMarchLanes = 64;
+constexpr int kMarchWaves = 4;  // wavefronts per block
+constexpr uint32_t march_columns(int steps) { return kMarchLanes - 2u * uint32_t(steps - 1); }
+
+// One pass of T steps, from time t.
+struct March {
+  const void* f_in;   // populations at time t
+  void* f_out;        // populations at time t + T
+  // Densities and velocities published for inlet/outlet neighbours at the
+  // step before the pass, and by its last step.
+  const float* pub_rho_in;
+  const float* pub_u_in;
+  float* pub_rho_out;
+  float* pub_u_out;
+  int32_t odd;        // t % 2
+  int32_t moments;    // write the readback fields of the last step
+  uint32_t strips, io_strips;  // strips, and those whose 64 columns hold an inlet or outlet cell
+  uint32_t chunks;    // chunks of rows
+  uint32_t rows;      // rows per chunk
+  uint32_t io_rows;   // rows a wavefront takes of a chunk of such a strip
+  uint32_t groups, group_magic;  // blocks per chunk of the other strips, div_magic of it
+  const uint32_t* order;  // strips, the io_strips ones first
+};
+
+// Value of the lane one to the left (lower x) / right.  The lanes at the ends
+// receive zero; their columns are halo.
+__device__ __forceinline__ float from_left(float v) {
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float from_right(float v) {
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x130, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double from_left(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = __builtin_amdgcn_update_dpp(0, int(uint32_t(b)), 0x138, 0xf, 0xf, true);
+  const uint32_t hi = __builtin_amdgcn_update_dpp(0, int(uint32_t(b >> 32)), 0x138, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, uint64_t(hi) << 32 | lo);
+}
+__device__ __forceinline__ double from_right(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = __builtin_amdgcn_update_dpp(0, int(uint32_t(b)), 0x130, 0xf, 0xf, true);
+  const uint32_t hi = __builtin_amdgcn_update_dpp(0, int(uint32_t(b >> 32)), 0x130, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, uint64_t(hi) << 32 | lo);
+}
+
+// How the pass holds populations between memory and the collision: in the
+// arithmetic type, times kUnit.  FP16S keeps the stored scale (2^15), so that a
+// conversion is all that loading, storing and rounding take.  Rounding goes in
+// pairs, one conversion for two values on gfx950.
+template <class S>
+struct Held {
+  using R = typename S::R;
+  using E = typename S::T;
+  static constexpr R kUnit = R(1);
+  __device__ static R in(E v) { return S::decode(v); }
+  __device__ static E out(R v) { return S::encode(v); }
+  __device__ static void round(R* g) {}
+};
+template <>
+struct Held<StoreF16S> {
+  static constexpr float kUnit = 32768.0f;
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+  __device__ static float in(_Float16 v) { return float(v); }
+  // A value is rounded to FP32 before it is to FP16: the empty statement keeps
+  // the compiler from fusing the collision's last multiply-add with the
+  // conversion (v_fma_mixlo_f16), which rounds once.
+  __device__ static void settle(float& v) { asm("" : "+v"(v)); }
+  __device__ static _Float16 out(float v) {
+    settle(v);
+    return _Float16(v);
+  }
+  __device__ static void round(float* g) {
+#pragma unroll
+    for (int i = 0; i < 9; i++) settle(g[i]);
+    g[0] = float(_Float16(g[0]));
+#pragma unroll
+    for (int i = 1; i < 9; i += 2) {
+      const f16x2 h = __builtin_convertvector((f32x2{g[i], g[i + 1]}), f16x2);
+      g[i] = float(h.x);
+      g[i + 1] = float(h.y);
+    }
+  }
+};
+template <>
+struct Held<StoreBF16S> {
+  static constexpr float kUnit = 1.0f;
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  __device__ static float in(uint16_t v) { return StoreBF16S::decode(v); }
+  __device__ static uint16_t out(float v) { return StoreBF16S::encode(v); }
+  __device__ static void round(float* g) {
+    g[0] = StoreBF16S::round(g[0]);
+#pragma unroll
+    for (int i = 1; i < 9; i += 2) {
+      const bf16x2 h = __builtin_convertvector((f32x2{g[i], g[i + 1]}), bf16x2);
+      const uint32_t b = __builtin_bit_cast(uint32_t, h);
+      g[i] = __uint_as_float(b << 16);
+      g[i + 1] = __uint_as_float(b & 0xffff0000u);
+    }
+  }
+};
+
+// Collision models compiled apart: plain SRT (no force, drag or subgrid
+// model), and everything by the handle's options.
+enum : int { kMarchPlain = 0, kMarchGeneral = 1 };
+
+// Previous-step values an inlet or outlet cell reads (stream_collide_cell).
+template <class R>
+struct IoValues {
+  R rho_next;           // published density of the cell at x + 1
+  R ux_prev, uy_prev;   // published velocity of the cell at x - 1
+};
+
+// One step of one cell: g holds its incoming populations and receives the
+// ones it emits; rho, ux, uy are set for cells that collide.
+template <class S, int MODEL, bool IO>
+__device__ __forceinline__ void march_cell(const Params& p, uint8_t fl, uint32_t n,
+                                           const IoValues<typename S::R>& v, typename S::R* g,
+                                           typename S::R& rho, typename S::R& ux,
+                                           typename S::R& uy) {
+#pragma clang fp contract(off)
+  using R = typename S::R;
+  if (fl & (kGas | kWall)) {
+#pragma unroll
+    for (int i = 1; i < 9; i += 2) {
+      const R t = g[i];
+      g[i] = g[i + 1];
+      g[i + 1] = t;
+    }
+    return;
+  }
+  constexpr R unit = Held<S>::kUnit;
+  const uint8_t io = IO ? fl & (kInlet | kOutlet) : 0;
+  R rho1, mx = R(0), my = R(0);
+  if (IO && (io & kInlet)) {
+    rho = v.rho_next;
+    rho1 = rho - R(1);
+    ux = at(fld<R>(p.u), n);
+    uy = at(fld<R>(p.u) + p.N, n);
+  } else if (IO && (io & kOutlet)) {
+    rho = at(fld<R>(p.rho), n);
+    rho1 = rho - R(1);
+    ux = v.ux_prev;
+    uy = v.uy_prev;
+  } else {
+    rho1 = g[0];
+#pragma unroll
+    for (int i = 1; i < 9; i++) rho1 += g[i];
+    rho1 *= R(1) / unit;
+    rho = R(1) + rho1;
+    mx = (g[1] - g[2] + g[5] - g[6] + g[7] - g[8]) * (R(1) / unit);
+    my = (g[3] - g[4] + g[5] - g[6] + g[8] - g[7]) * (R(1) / unit);
+  }
+  const Quotient<R> over_rho(rho);
+  if (!io) {
+    ux = over_rho(mx);
+    uy = over_rho(my);
+  }
+  R fi[9], fe[9];
+  bool forced = false;
+  if (MODEL != kMarchPlain) {
+    const bool brinkman = p.alpha && !io;
+    forced = apply_force<R>(p, p.use_force != 0, brinkman, brinkman ? R(at(p.alpha, n)) : R(0), rho,
+                            over_rho, ux, uy, fi, unit);
+  }
+  equilibrium_shifted<R>(rho, rho1, ux, uy, fe, unit);
+  const bool plain = MODEL == kMarchPlain;
+  relax<R>(p.inv_tau, plain ? 0 : p.collision, !plain && p.smagorinsky != 0, io != 0, forced, rho, fe,
+           fi, g, unit);
+}
+
+struct Fill { static constexpr bool value = false; };
+struct Steady { static constexpr bool value = true; };
+
+// The pass over one chunk of one strip: rows [ya, yb).
+template <class S, int T, int MODEL, bool IO>
+__device__ __forceinline__ void march_rows(const Params& p, const March& a, uint32_t strip,
+                                           uint32_t ya, uint32_t yb) {
+  static_assert(T >= 2 && T <= 4, "a lane keeps the flags of the T rows in one word");
+  using R = typename S::R;
+  using E = typename S::T;
+  constexpr int H = T - 1;  // halo
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t nx = p.nx, ny = p.ny, pitch = p.pitch;
+  const uint32_t xs = strip * march_columns(T) + lane;  // column + H
+  const bool own = lane >= H && lane < 64 - H && xs - H < nx;
+  const uint32_t x = (xs + H * (nx - 1)) % nx;
+  const uint32_t xr = x + 1 == nx ? 0u : x + 1, xl = x == 0 ? nx - 1 : x - 1;
+  // Planes the first step loads from and the last one stores to (pairs i, i + 1
+  // of opposite directions): at the cell, and at its neighbour in direction i.
+  const bool odd = a.odd != 0, odd_last = odd != ((T & 1) == 0);
+  const E* const fi = static_cast<const E*>(a.f_in);
+  E* const fo = static_cast<E*>(a.f_out);
+  const uint64_t Np = p.Np;
+  auto up = [&](uint32_t y) { return y + 1 == ny ? 0u : y + 1; };
+  auto down = [&](uint32_t y) { return y == 0 ? ny - 1 : y - 1; };
+
+  E raw[9];
+  uint8_t raw_fl;
+  auto load_row = [&](uint32_t y) {
+    const uint64_t rc = uint64_t(y) * pitch, ru = uint64_t(up(y)) * pitch,
+                   rd = uint64_t(down(y)) * pitch;
+    auto here = [&](int i) { return fi + (odd ? i : i + 1) * Np; };
+    auto there = [&](int i) { return fi + (odd ? i + 1 : i) * Np; };
+    raw[0] = at(fi + rc, x);
+    raw[1] = at(here(1) + rc, x);
+    raw[2] = at(there(1) + rc, xr);
+    raw[3] = at(here(3) + rc, x);
+    raw[4] = at(there(3) + ru, x);
+    raw[5] = at(here(5) + rc, x);
+    raw[6] = at(there(5) + ru, xr);
+    raw[7] = at(here(7) + rc, x);
+    raw[8] = at(there(7) + rd, xr);
+    raw_fl = at(p.flags + rc, x);
+  };
+  auto store_row = [&](uint32_t y, const R* g) {
+    const uint64_t rc = uint64_t(y) * pitch, ru = uint64_t(up(y)) * pitch,
+                   rd = uint64_t(down(y)) * pitch;
+    auto here = [&](int i) { return fo + (odd_last ? i : i + 1) * Np; };
+    auto there = [&](int i) { return fo + (odd_last ? i + 1 : i) * Np; };
+    at(fo + rc, x) = Held<S>::out(g[0]);
+    at(there(1) + rc, xr) = Held<S>::out(g[1]);
+    at(here(1) + rc, x) = Held<S>::out(g[2]);
+    at(there(3) + ru, x) = Held<S>::out(g[3]);
+    at(here(3) + rc, x) = Held<S>::out(g[4]);
+    at(there(5) + ru, xr) = Held<S>::out(g[5]);
+    at(here(5) + rc, x) = Held<S>::out(g[6]);
+    at(there(7) + rd, xr) = Held<S>::out(g[7]);
+    at(here(7) + rc, x) = Held<S>::out(g[8]);
+  };
+
+  // Between step s and s + 1 (index s - 1), already shifted to the receiving
+  // lane: populations 0, 1, 2 of the row s + 1 takes next; 3, 5, 8 of that row
+  // and of the one below it.
+  R flat[H][3], rise0[H][3], rise1[H][3];
+  R pr[H], pu[H], pv[H];  // values published for inlet/outlet neighbours (IO)
+#pragma unroll
+  for (int s = 0; s < H; s++) {
+#pragma unroll
+    for (int k = 0; k < 3; k++) flat[s][k] = rise0[s][k] = rise1[s][k] = R(0);
+    pr[s] = pu[s] = pv[s] = R(0);
+  }
+  uint32_t fls = 0;  // flags of the rows of steps 1 .. T, a byte each
+
+  uint32_t y1 = ya >= uint32_t(H) ? ya - H : ya + ny - H;  // row of step 1 (ny >= T)
+  load_row(y1);
+  const uint32_t iterations = yb - ya + 2 * H;
+  const auto iterate = [&](uint32_t it, auto steady) {
+    R g[9];
+#pragma unroll
+    for (int i = 0; i < 9; i++) g[i] = Held<S>::in(raw[i]);
+    fls = fls << 8 | raw_fl;
+    const uint32_t y = y1;
+    y1 = up(y1);
+    load_row(y1);  // one row past the last is loaded and not used
+    R rho = R(1), ux = R(0), uy = R(0);
+    R kept_r = R(0), kept_u = R(0), kept_v = R(0);  // published by step s - 1 (IO)
+    uint32_t ys = y;  // row of step s
+#pragma unroll
+    for (int s = 1; s <= T; s++) {
+      if (decltype(steady)::value || it >= 2u * uint32_t(s - 1)) {
+        const uint8_t fl = uint8_t(fls >> (8 * (s - 1)));
+        const uint32_t n = ys * pitch + x;
+        IoValues<R> v{};
+        R own_r = R(0), own_u = R(0), own_v = R(0);  // published at this cell so far
+        if (IO) {
+          if (s == 1) {
+            // From memory: the end lanes are computed too and have no neighbour.
+            const R* const r_in = fld<R>(const_cast<float*>(a.pub_rho_in));
+            const R* const u_in = fld<R>(const_cast<float*>(a.pub_u_in));
+            const uint32_t left = ys * pitch + xl, right = ys * pitch + xr;
+            own_r = at(r_in, n);
+            own_u = at(u_in, n);
+            own_v = at(u_in + p.N, n);
+            v.rho_next = at(r_in, right);
+            v.ux_prev = at(u_in, left);
+            v.uy_prev = at(u_in + p.N, left);
+          } else {
+            own_r = kept_r;
+            own_u = kept_u;
+            own_v = kept_v;
+            v.rho_next = from_right(own_r);
+            v.ux_prev = from_left(own_u);
+            v.uy_prev = from_left(own_v);
+          }
+        }
+        march_cell<S, MODEL, IO>(p, fl, n, v, g, rho, ux, uy);
+        const bool solid = fl & (kGas | kWall);
+        if (s < T) {
+          Held<S>::round(g);
+        } else {
+          if (own) {
+            store_row(ys, g);
+            if (a.moments && !solid) {
+              if (!(IO && (fl & kInlet))) {
+                at(fld<R>(p.u), n) = ux;
+                at(fld<R>(p.u) + p.N, n) = uy;
+              }
+              at(fld<R>(p.rho), n) = rho;
+            }
+          }
+          if (IO) {
+            const uint32_t left = uint32_t(__builtin_amdgcn_update_dpp(0, int(fl), 0x138, 0xf, 0xf, true));
+            const uint32_t right = uint32_t(__builtin_amdgcn_update_dpp(0, int(fl), 0x130, 0xf, 0xf, true));
+            if (own && !solid && (left & kInlet)) at(fld<R>(a.pub_rho_out), n) = rho;
+            if (own && !solid && (right & kOutlet) && !(fl & kInlet)) {
+              at(fld<R>(a.pub_u_out), n) = ux;
+              at(fld<R>(a.pub_u_out) + p.N, n) = uy;
+            }
+          }
+        }
+        if (s < T) {
+          constexpr int last = H - 1;
+          const int b = s - 1 < last ? s - 1 : last;
+          // Incoming populations of step s + 1 on the row below, then this
+          // row's into the registers.
+          R in[9];
+          in[0] = flat[b][0];
+          in[1] = flat[b][1];
+          in[2] = flat[b][2];
+          in[3] = rise1[b][0];
+          in[5] = rise1[b][1];
+          in[8] = rise1[b][2];
+          in[4] = g[4];
+          in[6] = from_right(g[6]);
+          in[7] = from_left(g[7]);
+          flat[b][0] = g[0];
+          flat[b][1] = from_left(g[1]);
+          flat[b][2] = from_right(g[2]);
+#pragma unroll
+          for (int k = 0; k < 3; k++) rise1[b][k] = rise0[b][k];
+          rise0[b][0] = g[3];
+          rise0[b][1] = from_left(g[5]);
+          rise0[b][2] = from_right(g[8]);
+          if (IO) {
+            kept_r = pr[b];
+            kept_u = pu[b];
+            kept_v = pv[b];
+            pr[b] = solid ? own_r : rho;
+            pu[b] = solid || (fl & kInlet) ? own_u : ux;
+            pv[b] = solid || (fl & kInlet) ? own_v : uy;
+          }
+#pragma unroll
+          for (int i = 0; i < 9; i++) g[i] = in[i];
+          ys = down(ys);
+        }
+      }
+    }
+    if (!IO) __builtin_amdgcn_s_barrier();  // a block's strips keep to the same row
+  };
+  // The first 2 H iterations fill the pipeline; from there every step runs.
+  for (uint32_t it = 0; it < 2 * H; ++it) iterate(it, Fill{});
+#pragma unroll 2
+  for (uint32_t it = 2 * H; it < iterations; ++it) iterate(it, Steady{});
+}
+
+}  // namespace flb
