@@ -149,6 +149,7 @@ struct flb_batch {
   int persist_chunk = 100; // persistent mode: steps per cooperative launch
   int ncu = 256;
   hipStream_t stream = nullptr;
+  flb::Staging staging;
   std::vector<flb::Params> host_inst;
   flb::Params* inst = nullptr;
   flb::Tile* tiles = nullptr;
@@ -363,7 +364,8 @@ int flb_batch_create(const flb_instance* in, uint32_t count, int32_t storage, in
   };
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, device) == hipSuccess) b->ncu = prop.multiProcessorCount;
-  if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess)
+  if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess ||
+      b->staging.init() != hipSuccess)
     return bail(FLB_ERR_DEVICE);
   const size_t eb = storage == 0 ? 4 : 2;
   // Offsets of every instance in the shared allocations (elements).
@@ -424,8 +426,8 @@ int flb_batch_create(const flb_instance* in, uint32_t count, int32_t storage, in
     // Host planes of nx * ny cells into pitched device planes (a device plane
     // is exactly ny rows of pitch cells, so `planes` planes are planes * ny rows).
     auto in2d = [&](void* dst, const void* src, size_t elem, int planes) {
-      return hipMemcpy2D(dst, p.pitch * elem, src, s.nx * elem, s.nx * elem, size_t(s.ny) * planes,
-                         hipMemcpyHostToDevice);
+      return b->staging.to_device(b->stream, dst, src, p.pitch * elem, s.nx * elem,
+                                  size_t(s.ny) * planes);
     };
     hipError_t e = in2d(p.flags, s.flags, 1, 1);
     if (e == hipSuccess) e = in2d(p.rho, hr.data(), 4, 1);
@@ -434,7 +436,8 @@ int flb_batch_create(const flb_instance* in, uint32_t count, int32_t storage, in
       e = in2d(p.pub_rho[k], hr.data(), 4, 1);
       if (e == hipSuccess) e = in2d(p.pub_u[k], hu.data(), 4, 2);
     }
-    if (e == hipSuccess) e = hipMemcpy(staging, fs.data(), 9 * N * 4, hipMemcpyHostToDevice);
+    if (e == hipSuccess)
+      e = b->staging.to_device(b->stream, staging, fs.data(), 9 * N * 4, 9 * N * 4, 1);
     if (e == hipSuccess) e = hipMemcpy(b->inst + i, &p, sizeof(p), hipMemcpyHostToDevice);
     if (e == hipSuccess) {
       void (*conv)(const flb::Params*, uint32_t, const float*) =
@@ -620,10 +623,10 @@ int flb_batch_autotune(flb_batch* b, uint32_t steps, int32_t* best_block, int32_
 int flb_batch_read(flb_batch* b, uint32_t i, float* u, float* rho) {
   if (!b || i >= b->host_inst.size()) return FLB_ERR_ARGUMENT;
   const flb::Params& p = b->host_inst[i];
-  BAT_HIP(b, hipStreamSynchronize(b->stream));
   const size_t row = p.nx * sizeof(float), dp = p.pitch * sizeof(float);
-  if (u) BAT_HIP(b, hipMemcpy2D(u, row, p.u, dp, row, 2 * size_t(p.ny), hipMemcpyDeviceToHost));
-  if (rho) BAT_HIP(b, hipMemcpy2D(rho, row, p.rho, dp, row, p.ny, hipMemcpyDeviceToHost));
+  if (u) BAT_HIP(b, b->staging.to_host(b->stream, u, p.u, dp, row, 2 * size_t(p.ny)));
+  if (rho) BAT_HIP(b, b->staging.to_host(b->stream, rho, p.rho, dp, row, p.ny));
+  if (!u && !rho) BAT_HIP(b, hipStreamSynchronize(b->stream));
   return FLB_OK;
 }
 
@@ -638,8 +641,8 @@ int flb_batch_read_populations(flb_batch* b, uint32_t i, float* f) {
                                          : flb::k_batch_to_f32<flb::StoreF32>);
   hipLaunchKernelGGL(conv, dim3(512), dim3(256), 0, b->stream, b->inst, i, tmp);
   hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
-  if (e == hipSuccess) e = hipMemcpy(f, tmp, 9 * p.NL * sizeof(float), hipMemcpyDeviceToHost);
+  const size_t bytes = 9 * p.NL * sizeof(float);
+  if (e == hipSuccess) e = b->staging.to_host(b->stream, f, tmp, bytes, bytes, 1);
   (void)hipFree(tmp);
   BAT_HIP(b, e);
   return FLB_OK;

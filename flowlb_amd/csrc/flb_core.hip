@@ -153,14 +153,12 @@ int dev_alloc(flb_handle* h, T** ptr, size_t count) {
 }
 
 int upload(flb_handle* h, void* dst, const void* src, size_t bytes) {
-  FLB_HIP(h, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, h->stream));
-  FLB_HIP(h, hipStreamSynchronize(h->stream));
+  FLB_HIP(h, h->staging.to_device(h->stream, dst, src, bytes, bytes, 1));
   return FLB_OK;
 }
 
 int download(flb_handle* h, void* dst, const void* src, size_t bytes) {
-  FLB_HIP(h, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, h->stream));
-  FLB_HIP(h, hipStreamSynchronize(h->stream));
+  FLB_HIP(h, h->staging.to_host(h->stream, dst, src, bytes, bytes, 1));
   return FLB_OK;
 }
 
@@ -168,16 +166,14 @@ int download(flb_handle* h, void* dst, const void* src, size_t bytes) {
 // `pitch`: one strided copy over ny * planes rows (a device plane is exactly
 // ny rows of pitch cells).
 int cells_in(flb_handle* h, void* dev, const void* host, size_t elem, int planes) {
-  FLB_HIP(h, hipMemcpy2DAsync(dev, h->pitch * elem, host, h->nx * elem, h->nx * elem,
-                              size_t(h->ny) * planes, hipMemcpyHostToDevice, h->stream));
-  FLB_HIP(h, hipStreamSynchronize(h->stream));
+  FLB_HIP(h, h->staging.to_device(h->stream, dev, host, h->pitch * elem, h->nx * elem,
+                                  size_t(h->ny) * planes));
   return FLB_OK;
 }
 
 int cells_out(flb_handle* h, void* host, const void* dev, size_t elem, int planes) {
-  FLB_HIP(h, hipMemcpy2DAsync(host, h->nx * elem, dev, h->pitch * elem, h->nx * elem,
-                              size_t(h->ny) * planes, hipMemcpyDeviceToHost, h->stream));
-  FLB_HIP(h, hipStreamSynchronize(h->stream));
+  FLB_HIP(h, h->staging.to_host(h->stream, host, dev, h->pitch * elem, h->nx * elem,
+                                size_t(h->ny) * planes));
   return FLB_OK;
 }
 
@@ -512,7 +508,8 @@ int flb_create(const flb_options* opt, const uint8_t* flags, uint32_t nx, uint32
   if (hipDeviceGetAttribute(&h->cus, hipDeviceAttributeMultiprocessorCount, opt->device) !=
           hipSuccess || h->cus <= 0)
     h->cus = 256;
-  if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess)
+  if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess ||
+      h->staging.init() != hipSuccess)
     return bail(FLB_ERR_DEVICE);
 
   int rc = FLB_OK;
@@ -846,6 +843,123 @@ static int enqueue_march(flb_handle* h, int T, bool moments) {
 }  // extern "C"
 
 namespace flb {
+hipError_t Staging::init() {
+  hipError_t e = hipSuccess;
+  for (hipEvent_t& d : done)
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&d, hipEventDisableTiming);
+  return e;
+}
+
+void Staging::release() {
+  for (void*& b : buf) {
+    if (b) (void)hipHostFree(b);
+    b = nullptr;
+  }
+  size = 0;
+}
+
+Staging::~Staging() {
+  release();
+  for (hipEvent_t d : done)
+    if (d) (void)hipEventDestroy(d);
+}
+
+// Buffers for a copy of `bytes`: one of that size, or two of kBytes.
+bool Staging::reserve(size_t bytes) {
+  const size_t want = std::min(bytes, kBytes);
+  if (size < want) release();
+  const int count = bytes > kBytes ? 2 : 1;
+  for (int k = 0; k < count; ++k)
+    if (!buf[k] && hipHostMalloc(&buf[k], std::max(want, size), hipHostMallocPortable) != hipSuccess) {
+      (void)hipGetLastError();
+      buf[k] = nullptr;
+      release();
+      return false;
+    }
+  size = std::max(want, size);
+  return true;
+}
+
+// One piece of a copy: rows [first, first + count) or, for contiguous rows,
+// bytes of a single row.
+namespace {
+struct Piece {
+  size_t host, dev, bytes, rows;
+};
+Piece piece(size_t k, size_t per, size_t pitch, size_t row_bytes, size_t rows) {
+  if (pitch == row_bytes) {
+    const size_t total = row_bytes * rows, at = k * per;
+    return Piece{at, at, std::min(per, total - at), 1};
+  }
+  const size_t first = k * per, count = std::min(per, rows - first);
+  return Piece{first * row_bytes, first * pitch, count * row_bytes, count};
+}
+}  // namespace
+
+hipError_t Staging::to_host(hipStream_t s, void* host, const void* dev, size_t pitch,
+                            size_t row_bytes, size_t rows) {
+  const size_t total = row_bytes * rows;
+  if (!total) return hipStreamSynchronize(s);
+  const bool flat = pitch == row_bytes;
+  if ((!flat && row_bytes > kBytes) || !reserve(total)) {  // rows longer than a buffer
+    const hipError_t e =
+        flat ? hipMemcpyAsync(host, dev, total, hipMemcpyDeviceToHost, s)
+             : hipMemcpy2DAsync(host, row_bytes, dev, pitch, row_bytes, rows, hipMemcpyDeviceToHost, s);
+    return e == hipSuccess ? hipStreamSynchronize(s) : e;
+  }
+  hipError_t e = hipSuccess;
+  const size_t per = flat ? kBytes : kBytes / row_bytes;
+  const size_t pieces = ((flat ? total : rows) + per - 1) / per;
+  auto start = [&](size_t k) {
+    const Piece q = piece(k, per, pitch, row_bytes, rows);
+    const char* from = static_cast<const char*>(dev) + q.dev;
+    hipError_t r = flat ? hipMemcpyAsync(buf[k & 1], from, q.bytes, hipMemcpyDeviceToHost, s)
+                        : hipMemcpy2DAsync(buf[k & 1], row_bytes, from, pitch, row_bytes, q.rows,
+                                           hipMemcpyDeviceToHost, s);
+    return r == hipSuccess ? hipEventRecord(done[k & 1], s) : r;
+  };
+  e = start(0);
+  for (size_t k = 0; k < pieces && e == hipSuccess; ++k) {
+    if (k + 1 < pieces) e = start(k + 1);
+    const hipError_t w = hipEventSynchronize(done[k & 1]);
+    if (e == hipSuccess) e = w;
+    if (e != hipSuccess) break;
+    const Piece q = piece(k, per, pitch, row_bytes, rows);
+    std::memcpy(static_cast<char*>(host) + q.host, buf[k & 1], q.bytes);
+  }
+  if (e != hipSuccess) (void)hipStreamSynchronize(s);
+  return e;
+}
+
+hipError_t Staging::to_device(hipStream_t s, void* dev, const void* host, size_t pitch,
+                              size_t row_bytes, size_t rows) {
+  const size_t total = row_bytes * rows;
+  if (!total) return hipStreamSynchronize(s);
+  const bool flat = pitch == row_bytes;
+  if ((!flat && row_bytes > kBytes) || !reserve(total)) {
+    const hipError_t e =
+        flat ? hipMemcpyAsync(dev, host, total, hipMemcpyHostToDevice, s)
+             : hipMemcpy2DAsync(dev, pitch, host, row_bytes, row_bytes, rows, hipMemcpyHostToDevice, s);
+    return e == hipSuccess ? hipStreamSynchronize(s) : e;
+  }
+  hipError_t e = hipSuccess;
+  const size_t per = flat ? kBytes : kBytes / row_bytes;
+  const size_t pieces = ((flat ? total : rows) + per - 1) / per;
+  for (size_t k = 0; k < pieces && e == hipSuccess; ++k) {
+    if (k >= 2) e = hipEventSynchronize(done[k & 1]);  // the piece two back has left the buffer
+    if (e != hipSuccess) break;
+    const Piece q = piece(k, per, pitch, row_bytes, rows);
+    std::memcpy(buf[k & 1], static_cast<const char*>(host) + q.host, q.bytes);
+    char* to = static_cast<char*>(dev) + q.dev;
+    e = flat ? hipMemcpyAsync(to, buf[k & 1], q.bytes, hipMemcpyHostToDevice, s)
+             : hipMemcpy2DAsync(to, pitch, buf[k & 1], row_bytes, row_bytes, q.rows,
+                                hipMemcpyHostToDevice, s);
+    if (e == hipSuccess) e = hipEventRecord(done[k & 1], s);
+  }
+  const hipError_t w = hipStreamSynchronize(s);
+  return e == hipSuccess ? w : e;
+}
+
 void host_initial_populations(uint32_t nx, uint32_t ny, const float* rho0, const float* u0,
                               std::vector<float>& fs) {
   initial_populations<float>(nx, ny, rho0, u0, fs);
