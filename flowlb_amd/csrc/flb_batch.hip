@@ -27,6 +27,7 @@
 
 #include "flb_cell.h"
 #include "flb_internal.h"
+#include "flb_march.h"
 
 namespace flb {
 
@@ -90,6 +91,59 @@ __global__ void __launch_bounds__(1024) k_batch_persistent(const Tile* __restric
   }
 }
 
+// A block of a multi-step pass over the batch: rows [ya, yb) of up to
+// kMarchWaves strips of an instance, or (io) of one strip with inlet or outlet
+// columns, split by rows between the wavefronts, as in k_march.
+struct MarchBlock {
+  static constexpr uint32_t kNone = ~0u;
+  uint32_t inst, ya, yb, io;
+  uint32_t strip[kMarchWaves];  // kNone: no strip
+};
+
+// inst: the instances with the populations the pass reads, out: those it writes.
+template <class S, int T, int MODEL>
+__global__ void __launch_bounds__(64 * kMarchWaves)
+__attribute__((amdgpu_waves_per_eu(march_occupancy<S, MODEL>())))
+k_batch_march(const MarchBlock* __restrict__ blocks, const Params* __restrict__ inst,
+              const Params* __restrict__ out, int odd, int moments) {
+  const MarchBlock* const d = blocks + blockIdx.x;
+  const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(threadIdx.x / 64u));
+  const uint32_t i = d->inst;
+  if (i == MarchBlock::kNone) return;
+  // What the pass uses of the instance, held in scalar registers.
+  const Params& q = inst[i];
+  Params p{};
+  p.nx = q.nx;
+  p.ny = q.ny;
+  p.pitch = q.pitch;
+  p.N = q.N;
+  p.Np = q.Np;
+  p.inv_tau = q.inv_tau;
+  p.fx = q.fx;
+  p.fy = q.fy;
+  p.use_force = q.use_force;
+  p.flags = q.flags;
+  p.rho = q.rho;
+  p.u = q.u;
+  March a{};
+  a.f_in = q.f;
+  a.f_out = out[i].f;
+  a.pub_rho_in = q.pub_rho[odd ^ 1];
+  a.pub_u_in = q.pub_u[odd ^ 1];
+  a.pub_rho_out = q.pub_rho[odd];
+  a.pub_u_out = q.pub_u[odd];
+  a.odd = odd;
+  a.moments = moments;
+  if (d->io) {
+    const uint32_t rows = (d->yb - d->ya + uint32_t(kMarchWaves) - 1u) / uint32_t(kMarchWaves);
+    const uint32_t ya = d->ya + wave * rows, yb = min(ya + rows, d->yb);
+    if (ya < yb) march_rows<S, T, MODEL, true>(p, a, d->strip[0], ya, yb);
+    return;
+  }
+  const uint32_t strip = d->strip[wave];
+  if (strip != MarchBlock::kNone) march_rows<S, T, MODEL, false>(p, a, strip, d->ya, d->yb);
+}
+
 // Populations of instance i to / from nx * ny host-ordered float planes
 // (unshifted), through the pitched device planes.
 template <class S>
@@ -127,6 +181,26 @@ BatchFn get_batch(int storage, int odd, bool mom) {
     default: return batch_fn<StoreF32>(odd, mom);
   }
 }
+using BatchMarchFn = void (*)(const MarchBlock*, const Params*, const Params*, int, int);
+template <class S, int T>
+BatchMarchFn batch_march_fn(bool forced) {
+  return forced ? k_batch_march<S, T, kMarchGeneral> : k_batch_march<S, T, kMarchPlain>;
+}
+template <class S>
+BatchMarchFn batch_march_steps(int steps, bool forced) {
+  switch (steps) {
+    case 2: return batch_march_fn<S, 2>(forced);
+    case 3: return batch_march_fn<S, 3>(forced);
+    default: return batch_march_fn<S, 4>(forced);
+  }
+}
+BatchMarchFn get_batch_march(int storage, int steps, bool forced) {
+  switch (storage) {
+    case 1: return batch_march_steps<StoreF16S>(steps, forced);
+    case 2: return batch_march_steps<StoreBF16S>(steps, forced);
+    default: return batch_march_steps<StoreF32>(steps, forced);
+  }
+}
 using PersistFn = void (*)(const Tile*, uint32_t, const Params*, uint32_t, uint32_t);
 PersistFn get_persistent(int storage) {
   switch (storage) {
@@ -151,12 +225,23 @@ struct flb_batch {
   hipStream_t stream = nullptr;
   flb::Staging staging;
   std::vector<flb::Params> host_inst;
+  // The instances' parameters, four sets of count: bit 0 of the set says which
+  // of the two population arrays they name, bit 1 whether the publication
+  // buffers are exchanged (a pass of an even number of steps leaves what it
+  // published at the other parity).  inst is the current set.
+  flb::Params* inst_sets = nullptr;
   flb::Params* inst = nullptr;
+  int set = 0;
+  // Blocks of the multi-step passes by number of steps; no passes if shape.steps is 0.
+  flb::MarchBlock* march[flb::kMarchMax + 1] = {};
+  uint32_t march_blocks[flb::kMarchMax + 1] = {};
+  flb::MarchShape shape{0, 0};
+  bool forced = false;
   flb::Tile* tiles = nullptr;
   uint32_t ntiles = 0;
   std::vector<void*> owned;
-  hipGraphExec_t graph = nullptr;
-  int graph_steps = 0;
+  hipGraphExec_t graph[4] = {};  // by the set it starts from
+  int graph_set[4] = {};         // the set it ends at
   uint64_t t = 0;
   std::string err;
 };
@@ -264,9 +349,104 @@ int build_tiles(flb_batch* b, int bx) {
 }
 
 void drop_graph(flb_batch* b) {
-  if (b->graph) (void)hipGraphExecDestroy(b->graph);
-  b->graph = nullptr;
-  b->graph_steps = 0;
+  for (hipGraphExec_t& g : b->graph) {
+    if (g) (void)hipGraphExecDestroy(g);
+    g = nullptr;
+  }
+}
+
+void use_set(flb_batch* b, int set) {
+  b->set = set;
+  b->inst = b->inst_sets + size_t(set) * b->host_inst.size();
+}
+
+// Block list of the passes of T steps: the inlet/outlet strips first (they take
+// longest), the others in an order that gives each XCD (block index mod 8)
+// consecutive groups of strips.
+int build_march(flb_batch* b, int T, const std::vector<std::vector<uint8_t>>& io) {
+  constexpr uint32_t G = flb::kMarchWaves;
+  std::vector<flb::MarchBlock> first, rest;
+  std::vector<uint32_t> order;
+  for (uint32_t i = 0; i < b->host_inst.size(); ++i) {
+    const flb::Params& p = b->host_inst[i];
+    const uint32_t nio = flb::march_strips(p.nx, T, io[i], order);
+    for (uint32_t ya = 0; ya < p.ny; ya += b->shape.rows) {
+      flb::MarchBlock d{};
+      d.inst = i;
+      d.ya = ya;
+      d.yb = std::min(ya + b->shape.rows, p.ny);
+      d.io = 1;
+      for (uint32_t k = 0; k < nio; ++k) {
+        d.strip[0] = order[k];
+        first.push_back(d);
+      }
+      d.io = 0;
+      for (uint32_t k = nio; k < order.size(); k += G) {
+        for (uint32_t w = 0; w < G; ++w)
+          d.strip[w] = k + w < order.size() ? order[k + w] : flb::MarchBlock::kNone;
+        rest.push_back(d);
+      }
+    }
+  }
+  const size_t per = (rest.size() + 7) / 8;
+  flb::MarchBlock none{};
+  none.inst = flb::MarchBlock::kNone;
+  for (size_t q = 0; q < 8 * per; ++q) {
+    const size_t w = (q % 8) * per + q / 8;
+    first.push_back(w < rest.size() ? rest[w] : none);
+  }
+  int rc = balloc(b, &b->march[T], first.size());
+  if (rc) return rc;
+  const size_t bytes = first.size() * sizeof(flb::MarchBlock);
+  BAT_HIP(b, b->staging.to_device(b->stream, b->march[T], first.data(), bytes, bytes, 1));
+  b->march_blocks[T] = uint32_t(first.size());
+  return FLB_OK;
+}
+
+// The second population array, the four sets of parameters and the block lists
+// of the passes; single steps only where an instance does not fit the passes'
+// rules or the array would take more than a quarter of the memory left.
+int prepare_march(flb_batch* b, const flb_instance* in, size_t f_bytes) {
+  const size_t count = b->host_inst.size();
+  int rc;
+  std::vector<std::vector<uint8_t>> io(count);
+  uint64_t strip_rows = 0;
+  bool fits = true;
+  const uint32_t cols = flb::march_columns(flb::kMarchMax);
+  for (size_t i = 0; i < count && fits; ++i) {
+    fits = flb::march_columns_io(in[i].flags, in[i].nx, in[i].ny, io[i]);
+    strip_rows += uint64_t((in[i].nx + cols - 1) / cols) * in[i].ny;
+    b->forced = b->forced || in[i].use_force;
+  }
+  size_t left = 0, total = 0;
+  void* alt = nullptr;
+  if (fits && (hipMemGetInfo(&left, &total) != hipSuccess || f_bytes > left / 4 ||
+               hipMalloc(&alt, f_bytes) != hipSuccess)) {
+    (void)hipGetLastError();
+    alt = nullptr;
+  }
+  if (alt) b->owned.push_back(alt);
+  const uint8_t* const base = static_cast<const uint8_t*>(b->host_inst[0].f);
+  std::vector<flb::Params> sets;
+  sets.reserve(4 * count);
+  for (int s = 0; s < 4; ++s)
+    for (flb::Params p : b->host_inst) {
+      if ((s & 1) && alt)
+        p.f = static_cast<uint8_t*>(alt) + (static_cast<const uint8_t*>(p.f) - base);
+      if (s & 2) {
+        std::swap(p.pub_rho[0], p.pub_rho[1]);
+        std::swap(p.pub_u[0], p.pub_u[1]);
+      }
+      sets.push_back(p);
+    }
+  const size_t bytes = sets.size() * sizeof(flb::Params);
+  BAT_HIP(b, b->staging.to_device(b->stream, b->inst_sets, sets.data(), bytes, bytes, 1));
+  if (!alt) return FLB_OK;
+  const flb::MarchShape shape = flb::march_shape(b->ncu, strip_rows, b->storage == 0 ? 4 : 2);
+  b->shape = shape;
+  for (int T = flb::kMarchMin; T <= flb::kMarchMax; ++T)
+    if ((rc = build_march(b, T, io))) return rc;
+  return FLB_OK;
 }
 
 int launch_step(flb_batch* b, int odd, bool mom) {
@@ -275,6 +455,25 @@ int launch_step(flb_batch* b, int odd, bool mom) {
                      b->stream, b->tiles + (odd ? b->ntiles : 0u), b->ntiles, b->inst);
   BAT_HIP(b, hipGetLastError());
   return FLB_OK;
+}
+
+// A pass of T steps from time parity odd; moves on to the set it leaves.
+int launch_march(flb_batch* b, int T, int odd, bool mom) {
+  const flb::Params* const out = b->inst_sets + size_t(b->set ^ 1) * b->host_inst.size();
+  hipLaunchKernelGGL(flb::get_batch_march(b->storage, T, b->forced), dim3(b->march_blocks[T]),
+                     dim3(64 * flb::kMarchWaves), 0, b->stream, b->march[T], b->inst, out, odd,
+                     int(mom));
+  BAT_HIP(b, hipGetLastError());
+  use_set(b, b->set ^ (T % 2 == 0 ? 3 : 1));
+  return FLB_OK;
+}
+
+// The next steps of a run with `left` to go: a pass, or a single step.
+int advance(flb_batch* b, uint64_t t, uint64_t left, bool mom, int* done) {
+  const int T = b->shape.steps ? flb::march_steps_next(left, b->shape.steps) : 0;
+  *done = T ? T : 1;
+  const bool last = mom && left == uint64_t(*done);
+  return T ? launch_march(b, T, int(t & 1), last) : launch_step(b, int(t & 1), last);
 }
 
 // Resident blocks per CU the persistent kernel can have at block size bx.
@@ -300,23 +499,26 @@ int launch_persistent(flb_batch* b, uint32_t nsteps, uint32_t odd0) {
   return FLB_OK;
 }
 
-// Graph of graph_chunk steps starting at an even t (parities alternate).
+// Graph of graph_chunk steps starting at an even t from the current set.
 int ensure_graph(flb_batch* b) {
-  if (b->graph || b->graph_chunk <= 0) return FLB_OK;
+  const int from = b->set;
+  if (b->graph[from] || b->graph_chunk <= 0) return FLB_OK;
   hipGraph_t g = nullptr;
   BAT_HIP(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-  int rc = FLB_OK;
-  for (int s = 0; s < b->graph_chunk && !rc; ++s) rc = launch_step(b, s & 1, false);
+  int rc = FLB_OK, done = 0;
+  for (int s = 0; s < b->graph_chunk && !rc; s += done)
+    rc = advance(b, uint64_t(s), uint64_t(b->graph_chunk - s), false, &done);
   hipError_t e = hipStreamEndCapture(b->stream, &g);
+  b->graph_set[from] = b->set;
+  use_set(b, from);
   if (rc) {
     if (g) (void)hipGraphDestroy(g);
     return rc;
   }
   BAT_HIP(b, e);
-  e = hipGraphInstantiate(&b->graph, g, nullptr, nullptr, 0);
+  e = hipGraphInstantiate(&b->graph[from], g, nullptr, nullptr, 0);
   (void)hipGraphDestroy(g);
   BAT_HIP(b, e);
-  b->graph_steps = b->graph_chunk;
   return FLB_OK;
 }
 
@@ -387,13 +589,14 @@ int flb_batch_create(const flb_instance* in, uint32_t count, int32_t storage, in
       (rc = balloc(b, &rho, tot_c)) || (rc = balloc(b, &u, 2 * tot_c)) ||
       (rc = balloc(b, &pr0, tot_c)) || (rc = balloc(b, &pr1, tot_c)) ||
       (rc = balloc(b, &pu0, 2 * tot_c)) || (rc = balloc(b, &pu1, 2 * tot_c)) ||
-      (rc = balloc(b, &b->inst, count)))
+      (rc = balloc(b, &b->inst_sets, 4 * size_t(count))))
     return bail(rc);
   float* staging = nullptr;
   size_t max_n = 0;
   for (uint32_t i = 0; i < count; ++i) max_n = std::max(max_n, size_t(in[i].nx) * in[i].ny);
   if (hipMalloc(&staging, 9 * max_n * sizeof(float)) != hipSuccess) return bail(FLB_ERR_MEMORY);
   b->host_inst.resize(count);
+  use_set(b, 0);
   std::vector<float> fs, hr, hu;
   for (uint32_t i = 0; i < count && !rc; ++i) {
     const flb_instance& s = in[i];
@@ -455,6 +658,7 @@ int flb_batch_create(const flb_instance* in, uint32_t count, int32_t storage, in
   }
   (void)hipFree(staging);
   if (rc) return bail(rc);
+  if ((rc = prepare_march(b, in, tot_f * eb))) return bail(rc);
   b->grid = 8 * b->ncu;
   if ((rc = build_tiles(b, 256))) return bail(rc);
   *out = b;
@@ -519,13 +723,15 @@ int flb_batch_step(flb_batch* b, uint64_t nsteps) {
     // Graph replays need an even start; the last step writes the readback fields.
     if (b->graph_chunk > 0 && (b->t & 1) == 0 && left > uint64_t(b->graph_chunk)) {
       if ((rc = ensure_graph(b))) break;
-      BAT_HIP(b, hipGraphLaunch(b->graph, b->stream));
-      b->t += uint64_t(b->graph_steps);
-      left -= uint64_t(b->graph_steps);
+      BAT_HIP(b, hipGraphLaunch(b->graph[b->set], b->stream));
+      use_set(b, b->graph_set[b->set]);
+      b->t += uint64_t(b->graph_chunk);
+      left -= uint64_t(b->graph_chunk);
     } else {
-      rc = launch_step(b, int(b->t & 1), left == 1);
-      b->t += 1;
-      left -= 1;
+      int done = 0;
+      rc = advance(b, b->t, left, true, &done);
+      b->t += uint64_t(done);
+      left -= uint64_t(done);
     }
   }
   return rc;

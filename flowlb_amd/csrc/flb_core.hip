@@ -329,25 +329,18 @@ uint32_t row_pitch(const flb_options* o, uint32_t nx) {
   return (nx + 63u) / 64u * 64u;
 }
 
-bool march_plain(const flb_handle* h) {
-  return h->opt.collision == FLB_SRT && !h->opt.smagorinsky && !h->opt.use_force && !h->alpha;
+int march_model(const flb_handle* h) {
+  if (h->opt.collision != FLB_SRT || h->opt.smagorinsky || h->alpha) return flb::kMarchGeneral;
+  return h->opt.use_force ? flb::kMarchForced : flb::kMarchPlain;
 }
 
 // Sets a single-phase handle up for the multi-step pass.  It is left to single
-// steps (f_alt null) where the pass's rules do not hold: an inlet cell in the
-// last column or an outlet cell in the first one reads the linear neighbour in
-// another row, and the pass needs as many rows as it does steps; or where the
-// second population array would take more than a quarter of the memory left (a
-// program that fills the device with handles keeps its room).
+// steps (f_alt null) where the pass's rules do not hold (march_columns_io) or
+// the second population array would take more than a quarter of the memory
+// left (a program that fills the device with handles keeps its room).
 int prepare_march(flb_handle* h, const uint8_t* flags) {
-  const uint32_t nx = h->nx, ny = h->ny;
-  if (ny < uint32_t(flb::kMarchMax)) return FLB_OK;
-  std::vector<uint8_t> io(nx, 0);  // columns with an inlet or outlet cell
-  for (uint32_t y = 0; y < ny; ++y) {
-    const uint8_t* row = flags + uint64_t(y) * nx;
-    if ((row[nx - 1] & FLB_INLET) || ((row[0] & FLB_OUTLET) && !(row[0] & FLB_INLET))) return FLB_OK;
-    for (uint32_t x = 0; x < nx; ++x) io[x] |= row[x] & (FLB_INLET | FLB_OUTLET);
-  }
+  std::vector<uint8_t> io;
+  if (!flb::march_columns_io(flags, h->nx, h->ny, io)) return FLB_OK;
   const size_t bytes = 9 * h->Np * h->elem_bytes;
   size_t left = 0, total = 0;
   void* v = nullptr;
@@ -359,52 +352,18 @@ int prepare_march(flb_handle* h, const uint8_t* flags) {
   h->owned.push_back(v);
   int rc;
   for (int T = flb::kMarchMin; T <= flb::kMarchMax; ++T) {
-    const uint32_t cols = flb::march_columns(T), strips = (nx + cols - 1) / cols;
-    std::vector<uint32_t> order(strips);
-    for (uint32_t s = 0; s < strips; ++s) order[s] = s;
-    const auto split = std::stable_partition(order.begin(), order.end(), [&](uint32_t s) {
-      uint8_t any = 0;
-      for (uint32_t l = 0; l < flb::kMarchLanes; ++l)
-        any |= io[(uint64_t(s) * cols + l + uint64_t(T - 1) * (nx - 1)) % nx];
-      return any != 0;
-    });
-    h->march_io[T] = uint32_t(split - order.begin());
-    if ((rc = dev_alloc(h, &h->march_order[T], strips))) return rc;
-    if ((rc = upload(h, h->march_order[T], order.data(), strips * sizeof(uint32_t)))) return rc;
+    std::vector<uint32_t> order;
+    h->march_io[T] = flb::march_strips(h->nx, T, io, order);
+    if ((rc = dev_alloc(h, &h->march_order[T], order.size()))) return rc;
+    if ((rc = upload(h, h->march_order[T], order.data(), order.size() * sizeof(uint32_t)))) return rc;
   }
   h->f_alt = v;
   return FLB_OK;
 }
 
-// Shape of the passes of a run of steps.
-//
-// Rows per chunk.  A wavefront's chunk of r rows takes r + 2 (T - 1)
-// iterations and T (r + T - 1) step-rows, so long chunks waste less, while the
-// chip needs wavefronts on its 1024 SIMDs.  Measured with T = 4, us per step: 2048 x 512
-// FP32 (36 strips) 8.3, 7.2, 7.2, 8.6, 9.2 with 4, 8, 12, 16, 24 rows: best near
-// 1.5 wavefronts per SIMD (12 rows).  Where that gives long chunks, the chip
-// runs several rounds of wavefronts anyway and FP32 wants them short, so that
-// fewer rows are in flight: 8192 x 2048 79.8, 83.2, 84.3, 90.5 with 16, 24, 36,
-// 64 rows; FP16S, which is bound by the vector units, 70.6, 68.6, 66.1, 74.6.
-// Below four rows nothing is gained (512 x 128: 3.3 us with 1 to 4).
-//
-// Steps per pass.  T = 4 moves the fewest bytes and was the fastest from
-// 2048 x 512 on (8192 x 2048 FP32 80 us per step, with T = 3 110, with T = 2
-// about 150; single steps 196).  Grids that give less than 1.5 wavefronts per
-// SIMD at four rows are bound by the chain of a wavefront, T (r + T - 1)
-// step-rows: T = 3 takes 3.1 us per step on 512 x 128 and 3.5 on 1024 x 256,
-// T = 4 3.4 and 4.0.
-struct MarchShape {
-  int steps;
-  uint32_t rows;
-};
-MarchShape march_shape(const flb_handle* h) {
-  const uint64_t waves = uint64_t(h->cus) * 6;  // 1.5 per SIMD
-  const uint32_t least = 4, most = h->elem_bytes == 2 ? 36 : 16;
+flb::MarchShape march_shape(const flb_handle* h) {
   const uint32_t cols = flb::march_columns(flb::kMarchMax);
-  const uint64_t strip_rows = uint64_t((h->nx + cols - 1) / cols) * h->ny;
-  const uint64_t rows = (strip_rows + waves - 1) / waves;
-  return MarchShape{rows < least ? 3 : 4, uint32_t(std::min<uint64_t>(std::max<uint64_t>(rows, least), most))};
+  return flb::march_shape(h->cus, uint64_t((h->nx + cols - 1) / cols) * h->ny, h->elem_bytes);
 }
 
 }  // namespace
@@ -826,7 +785,7 @@ static int enqueue_march(flb_handle* h, int T, bool moments) {
   a.groups = (a.strips - a.io_strips + G - 1) / G;
   a.group_magic = flb::div_magic(a.groups);
   const uint32_t blocks = a.io_strips * a.chunks + (a.groups * a.chunks + 7u) / 8u * 8u;
-  hipLaunchKernelGGL(flb::get_march(h->opt.storage, T, march_plain(h)), dim3(blocks),
+  hipLaunchKernelGGL(flb::get_march(h->opt.storage, T, march_model(h)), dim3(blocks),
                      dim3(64 * G), 0, h->stream, p, a);
   FLB_HIP(h, hipGetLastError());
   std::swap(h->f, h->f_alt);
@@ -843,6 +802,57 @@ static int enqueue_march(flb_handle* h, int T, bool moments) {
 }  // extern "C"
 
 namespace flb {
+bool march_columns_io(const uint8_t* flags, uint32_t nx, uint32_t ny, std::vector<uint8_t>& io) {
+  if (ny < uint32_t(kMarchMax)) return false;
+  io.assign(nx, 0);
+  for (uint32_t y = 0; y < ny; ++y) {
+    const uint8_t* row = flags + uint64_t(y) * nx;
+    if ((row[nx - 1] & FLB_INLET) || ((row[0] & FLB_OUTLET) && !(row[0] & FLB_INLET))) return false;
+    for (uint32_t x = 0; x < nx; ++x) io[x] |= row[x] & (FLB_INLET | FLB_OUTLET);
+  }
+  return true;
+}
+
+uint32_t march_strips(uint32_t nx, int steps, const std::vector<uint8_t>& io,
+                      std::vector<uint32_t>& order) {
+  const uint32_t cols = march_columns(steps);
+  order.resize((nx + cols - 1) / cols);
+  for (uint32_t s = 0; s < order.size(); ++s) order[s] = s;
+  const auto split = std::stable_partition(order.begin(), order.end(), [&](uint32_t s) {
+    uint8_t any = 0;
+    for (uint32_t l = 0; l < kMarchLanes; ++l)
+      any |= io[(uint64_t(s) * cols + l + uint64_t(steps - 1) * (nx - 1)) % nx];
+    return any != 0;
+  });
+  return uint32_t(split - order.begin());
+}
+
+// Shape of the passes of a run of steps.
+//
+// Rows per chunk.  A wavefront's chunk of r rows takes r + 2 (T - 1)
+// iterations and T (r + T - 1) step-rows, so long chunks waste less, while the
+// chip needs wavefronts on its 1024 SIMDs.  Measured with T = 4, us per step: 2048 x 512
+// FP32 (36 strips) 8.3, 7.2, 7.2, 8.6, 9.2 with 4, 8, 12, 16, 24 rows: best near
+// 1.5 wavefronts per SIMD (12 rows).  Where that gives long chunks, the chip
+// runs several rounds of wavefronts anyway and FP32 wants them short, so that
+// fewer rows are in flight: 8192 x 2048 79.8, 83.2, 84.3, 90.5 with 16, 24, 36,
+// 64 rows; FP16S, which is bound by the vector units, 70.6, 68.6, 66.1, 74.6.
+// Below four rows nothing is gained (512 x 128: 3.3 us with 1 to 4).
+//
+// Steps per pass.  T = 4 moves the fewest bytes and was the fastest from
+// 2048 x 512 on (8192 x 2048 FP32 80 us per step, with T = 3 110, with T = 2
+// about 150; single steps 196).  Grids that give less than 1.5 wavefronts per
+// SIMD at four rows are bound by the chain of a wavefront, T (r + T - 1)
+// step-rows: T = 3 takes 3.1 us per step on 512 x 128 and 3.5 on 1024 x 256,
+// T = 4 3.4 and 4.0.
+MarchShape march_shape(int cus, uint64_t strip_rows, int elem_bytes) {
+  const uint64_t waves = uint64_t(cus) * 6;  // 1.5 per SIMD
+  const uint32_t least = 4, most = elem_bytes == 2 ? 36 : 16;
+  const uint64_t rows = (strip_rows + waves - 1) / waves;
+  return MarchShape{rows < least ? 3 : 4,
+                    uint32_t(std::min<uint64_t>(std::max<uint64_t>(rows, least), most))};
+}
+
 hipError_t Staging::init() {
   hipError_t e = hipSuccess;
   for (hipEvent_t& d : done)
@@ -988,8 +998,7 @@ int flb_step(flb_handle* h, uint64_t nsteps) {
     const uint64_t left = nsteps - k;
     if (h->f_alt && left > 1) {
       // Passes of the shape's steps; a single step is not left over.
-      const uint64_t most = uint64_t(march_shape(h).steps);
-      const int T = int(left == most + 1 ? (left + 1) / 2 : std::min(left, most));
+      const int T = flb::march_steps_next(left, march_shape(h).steps);
       const int rc = enqueue_march(h, T, left == uint64_t(T));
       if (rc) return rc;
       k += uint64_t(T);

@@ -48,7 +48,27 @@ HistFn get_flag_hist();
 struct March;
 using MarchFn = void (*)(const Params, const March);
 constexpr int kMarchMin = 2, kMarchMax = 4;
-MarchFn get_march(int storage, int steps, bool plain);
+// Shape of the passes of a run of steps: steps per pass and rows per chunk.
+struct MarchShape {
+  int steps;
+  uint32_t rows;
+};
+MarchShape march_shape(int cus, uint64_t strip_rows, int elem_bytes);
+// Steps of the next pass of a run with `left` steps to go; 0: a single step.
+inline int march_steps_next(uint64_t left, int most) {
+  if (left < 2) return 0;
+  return int(left == uint64_t(most) + 1 ? (left + 1) / 2 : (left < uint64_t(most) ? left : most));
+}
+// Strips of a domain of nx columns for passes of `steps` steps, those whose 64
+// columns hold a column marked in io (inlet or outlet cells) first; returns
+// the number of these.
+uint32_t march_strips(uint32_t nx, int steps, const std::vector<uint8_t>& io,
+                      std::vector<uint32_t>& order);
+// Columns with an inlet or outlet cell; false where passes are not used: an
+// inlet cell in the last column or an outlet cell in the first one reads the
+// linear neighbour in another row, and a pass needs as many rows as steps.
+bool march_columns_io(const uint8_t* flags, uint32_t nx, uint32_t ny, std::vector<uint8_t>& io);
+MarchFn get_march(int storage, int steps, int model);
 }  // namespace flb
 
 namespace flb {

@@ -139,8 +139,13 @@ struct Held<StoreBF16S> {
 };
 
 // Collision models compiled apart: plain SRT (no force, drag or subgrid
-// model), and everything by the handle's options.
-enum : int { kMarchPlain = 0, kMarchGeneral = 1 };
+// model), SRT with a body force, and everything by the handle's options.
+enum : int { kMarchPlain = 0, kMarchForced = 1, kMarchGeneral = 2 };
+// Wavefronts per SIMD the pass is compiled for (its registers: 128, 168, 256).
+template <class S, int MODEL>
+constexpr int march_occupancy() {
+  return S::kBytes > 4 ? 2 : (MODEL == kMarchGeneral ? 3 : 4);
+}
 
 // Previous-step values an inlet or outlet cell reads (stream_collide_cell).
 template <class R>
@@ -197,14 +202,14 @@ __device__ __forceinline__ void march_cell(const Params& p, uint8_t fl, uint32_t
   R fi[9], fe[9];
   bool forced = false;
   if (MODEL != kMarchPlain) {
-    const bool brinkman = p.alpha && !io;
-    forced = apply_force<R>(p, p.use_force != 0, brinkman, brinkman ? R(at(p.alpha, n)) : R(0), rho,
-                            over_rho, ux, uy, fi, unit);
+    const bool brinkman = MODEL == kMarchGeneral && p.alpha && !io;
+    forced = apply_force<R>(p, MODEL == kMarchForced || p.use_force != 0, brinkman,
+                            brinkman ? R(at(p.alpha, n)) : R(0), rho, over_rho, ux, uy, fi, unit);
   }
   equilibrium_shifted<R>(rho, rho1, ux, uy, fe, unit);
-  const bool plain = MODEL == kMarchPlain;
-  relax<R>(p.inv_tau, plain ? 0 : p.collision, !plain && p.smagorinsky != 0, io != 0, forced, rho, fe,
-           fi, g, unit);
+  const bool general = MODEL == kMarchGeneral;
+  relax<R>(p.inv_tau, general ? p.collision : 0, general && p.smagorinsky != 0, io != 0, forced, rho,
+           fe, fi, g, unit);
 }
 
 struct Fill { static constexpr bool value = false; };

@@ -14,7 +14,7 @@ namespace flb {
 // Block b runs on XCD b mod 8; one XCD's blocks take consecutive groups of strips.
 template <class S, int T, int MODEL>
 __global__ void __launch_bounds__(64 * kMarchWaves)
-__attribute__((amdgpu_waves_per_eu(MODEL == kMarchPlain && S::kBytes <= 4 ? 4 : (S::kBytes <= 4 ? 3 : 2))))
+__attribute__((amdgpu_waves_per_eu(march_occupancy<S, MODEL>())))
 k_march(const Params p, const March a) {
   const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(threadIdx.x / 64u));
   const uint32_t io_blocks = a.io_strips * a.chunks;
@@ -36,26 +36,27 @@ k_march(const Params p, const March a) {
 
 namespace {
 template <class S, int T>
-MarchFn march_fn(bool plain) {
-  return plain ? k_march<S, T, kMarchPlain> : k_march<S, T, kMarchGeneral>;
+MarchFn march_fn(int model) {
+  if (model == kMarchPlain) return k_march<S, T, kMarchPlain>;
+  return model == kMarchForced ? k_march<S, T, kMarchForced> : k_march<S, T, kMarchGeneral>;
 }
 template <class S>
-MarchFn march_steps(int steps, bool plain) {
+MarchFn march_steps(int steps, int model) {
   switch (steps) {
-    case 2: return march_fn<S, 2>(plain);
-    case 3: return march_fn<S, 3>(plain);
-    case 4: return march_fn<S, 4>(plain);
+    case 2: return march_fn<S, 2>(model);
+    case 3: return march_fn<S, 3>(model);
+    case 4: return march_fn<S, 4>(model);
     default: return nullptr;
   }
 }
 }  // namespace
 
-MarchFn get_march(int storage, int steps, bool plain) {
+MarchFn get_march(int storage, int steps, int model) {
   switch (storage) {
-    case 1: return march_steps<StoreF16S>(steps, plain);
-    case 2: return march_steps<StoreBF16S>(steps, plain);
-    case 3: return march_steps<StoreF64>(steps, plain);
-    default: return march_steps<StoreF32>(steps, plain);
+    case 1: return march_steps<StoreF16S>(steps, model);
+    case 2: return march_steps<StoreBF16S>(steps, model);
+    case 3: return march_steps<StoreF64>(steps, model);
+    default: return march_steps<StoreF32>(steps, model);
   }
 }
 

@@ -100,3 +100,49 @@ def test_inlet_in_the_last_column_keeps_single_steps():
     many = _run(fl.ravel(), nx, ny, rho0, u0.ravel(), [9])
     for k in ("f", "u", "rho"):
         assert np.array_equal(one[k], many[k]), k
+
+
+@pytest.mark.parametrize("storage", ["fp32", "fp16s", "bf16s"])
+@pytest.mark.parametrize("force", [False, True])
+def test_batch_passes_equal_single_steps(storage, force):
+    """A batch of uneven instances: passes, graphs of passes (8 steps, so that a
+    replay starts from each of the two population arrays) and single steps."""
+    rng = np.random.default_rng(10)
+    inst = []
+    for k, (nx, ny) in enumerate([(65, 9), (130, 41), (57, 4), (300, 33), (64, 64)]):
+        fl, rho0, u0 = _domain(nx, ny, "channel" if k % 2 else "scattered", rng)
+        fl[-1] = core.WALL
+        fl[0] = core.WALL
+        inst.append(dict(nx=nx, ny=ny, tau=0.6 + 0.05 * k, flags=fl, rho0=rho0, u0=u0,
+                         use_force=int(force and k != 2), fx=1e-5 * k, fy=-1e-5))
+
+    def run(calls, chunk):
+        with core.Batch(inst, storage=storage) as b:
+            b.configure(block_x=128, grid=0, graph_chunk=chunk)
+            for n in calls:
+                b.step(n)
+            assert b.time == sum(calls)
+            return [dict(f=b.populations(i), **b.read(i)) for i in range(len(inst))]
+
+    one = run([1] * 48, 0)
+    for calls, chunk in (([48], 0), ([7, 20, 21], 0), ([26, 1, 21], 4), ([3, 45], 10)):
+        for i, (a, g) in enumerate(zip(one, run(calls, chunk))):
+            for k in a:
+                assert np.array_equal(a[k], g[k], equal_nan=True), (calls, chunk, i, k)
+
+
+def test_batch_with_an_unfit_instance():
+    """One instance under four rows: the whole batch keeps single steps."""
+    rng = np.random.default_rng(11)
+    inst = []
+    for nx, ny in [(65, 9), (70, 3)]:
+        fl, rho0, u0 = _domain(nx, ny, "channel", rng)
+        inst.append(dict(nx=nx, ny=ny, tau=0.7, flags=fl, rho0=rho0, u0=u0))
+    got = []
+    for calls in ([1] * 9, [9]):
+        with core.Batch(inst) as b:
+            for n in calls:
+                b.step(n)
+            got.append([b.populations(i) for i in range(2)])
+    for a, g in zip(*got):
+        assert np.array_equal(a, g)
