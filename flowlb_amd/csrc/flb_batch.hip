@@ -119,6 +119,8 @@ k_batch_march(const MarchBlock* __restrict__ blocks, const Params* __restrict__ 
   p.N = q.N;
   p.Np = q.Np;
   p.inv_tau = q.inv_tau;
+  p.tau = q.tau;
+  p.trt_minus = q.trt_minus;
   p.fx = q.fx;
   p.fy = q.fy;
   p.use_force = q.use_force;
@@ -442,7 +444,7 @@ int prepare_march(flb_batch* b, const flb_instance* in, size_t f_bytes) {
   const size_t bytes = sets.size() * sizeof(flb::Params);
   BAT_HIP(b, b->staging.to_device(b->stream, b->inst_sets, sets.data(), bytes, bytes, 1));
   if (!alt) return FLB_OK;
-  const flb::MarchShape shape = flb::march_shape(b->ncu, strip_rows, b->storage == 0 ? 4 : 2);
+  const flb::MarchShape shape = flb::march_shape(b->ncu, strip_rows, b->storage == 0 ? 4 : 2, false);
   b->shape = shape;
   for (int T = flb::kMarchMin; T <= flb::kMarchMax; ++T)
     if ((rc = build_march(b, T, io))) return rc;
@@ -609,7 +611,7 @@ int flb_batch_create(const flb_instance* in, uint32_t count, int32_t storage, in
     p.N = size_t(p.pitch) * s.ny;  // device plane of a cell field
     p.NL = N;                      // host plane
     p.Np = flb::plane_stride(p.N, uint32_t(eb));
-    p.inv_tau = 1.0f / s.tau;
+    flb::set_relaxation(p, 1.0f / s.tau);
     p.use_force = s.use_force;
     p.fx = s.use_force ? s.fx : 0.0f;
     p.fy = s.use_force ? s.fy : 0.0f;

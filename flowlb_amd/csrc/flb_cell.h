@@ -352,12 +352,27 @@ __device__ __forceinline__ bool apply_force(const Params& p, bool use_force, boo
   return false;
 }
 
+// Square root, correctly rounded (as sqrtf) for zero and normal x above 2^-100:
+// the hardware's value s is within one unit in the last place, and the sign of
+// x - s t for its neighbours t, exact in a fused multiply-add, tells which of the
+// three is nearest.  Nine instructions; sqrtf takes fifteen, scaling x first
+// for the sake of smaller ones.
+__device__ __forceinline__ float root(float x) {
+  const float s = __builtin_amdgcn_sqrtf(x);
+  const float down = __uint_as_float(__float_as_uint(s) - 1u);
+  const float up = __uint_as_float(__float_as_uint(s) + 1u);
+  const float below = fused(-down, s, x), above = fused(-up, s, x);
+  float r = below <= 0.0f ? down : s;
+  r = above > 0.0f ? up : r;
+  return r;
+}
+
 // Relaxation rate of the subgrid model for a cell off equilibrium by g - fe.
 // 1/tau is a float constant in the reference also for PRECISION = 64, and the
 // Smagorinsky correction goes through float sqrtf (lbmKernel2D.cu:414-442).
 template <class R>
-__device__ __forceinline__ float smagorinsky_rate(float inv_tau, R rho, const R* fe, const R* g,
-                                                  R unit) {
+__device__ __forceinline__ float smagorinsky_rate(float tau, const Quotient<R>& over_rho,
+                                                  const R* fe, const R* g, R unit) {
 #pragma clang fp contract(off)
   R hxx = R(0), hyy = R(0), hxy = R(0);
 #pragma unroll
@@ -372,22 +387,24 @@ __device__ __forceinline__ float smagorinsky_rate(float inv_tau, R rho, const R*
   hyy *= R(1) / unit;
   hxy *= R(1) / unit;
   const R Q = fused(hxy, R(2.0f) * hxy, fused(hxx, hxx, hyy * hyy));
-  const float tau = 1.0f / inv_tau;
-  const R strain = R(0.54037965f * sqrtf(float(Q))) / rho;
+  // Below 2^-100 the root of Q is under 2^-50 and does not reach tau^2.
+  const float q = float(Q);
+  const R strain = over_rho(R(0.54037965f * root(q < 0x1p-100f ? 0.0f : q)));
   // The float build fuses tau^2; for doubles tau^2 is a float product.
   const float sum = sizeof(R) == 4 ? fused(tau, tau, float(strain)) : float(R(tau * tau) + strain);
-  return 2.0f / (tau + sqrtf(sum));
+  return Quotient<float>(tau + root(sum))(2.0f);
 }
 
 // Collision of a cell's populations g towards the equilibrium fe (inlet and
 // outlet cells, io, take the equilibrium itself): optional Smagorinsky, then
 // SRT or TRT.
 template <class R>
-__device__ __forceinline__ void relax(float inv_tau, int collision, bool smagorinsky, bool io,
-                                      bool forced, R rho, const R* fe, const R* fi, R* g,
-                                      R unit = R(1)) {
+__device__ __forceinline__ void relax(const Params& p, int collision, bool smagorinsky, bool io,
+                                      bool forced, const Quotient<R>& over_rho, const R* fe,
+                                      const R* fi, R* g, R unit = R(1)) {
 #pragma clang fp contract(off)
-  if (smagorinsky) inv_tau = smagorinsky_rate<R>(inv_tau, rho, fe, g, unit);
+  float inv_tau = p.inv_tau;
+  if (smagorinsky) inv_tau = smagorinsky_rate<R>(p.tau, over_rho, fe, g, unit);
   if (io) {
 #pragma unroll
     for (int i = 0; i < 9; i++) g[i] = fe[i];
@@ -407,7 +424,11 @@ __device__ __forceinline__ void relax(float inv_tau, int collision, bool smagori
     // and the antisymmetric part, weighted 1 - w-/2 (SRT + Guo when w+ = w-).
     // The reference keeps these temporaries in float also for PRECISION = 64.
     const float ip = inv_tau;
-    const float in = 1.0f / (0.25f / (1.0f / inv_tau - 0.5f) + 0.5f);
+    float in = p.trt_minus;
+    if (smagorinsky) {
+      const float lambda = Quotient<float>(Quotient<float>(inv_tau)(1.0f) - 0.5f)(0.25f);
+      in = Quotient<float>(lambda + 0.5f)(1.0f);
+    }
     const float hp = 0.5f * ip, hn = 0.5f * in;
     // a - h * v: one fused step in the float build; for doubles h * v is a
     // float product.
@@ -663,7 +684,7 @@ __device__ __forceinline__ void stream_collide_cell(const Params& p, const Cell 
     // absorbs the weight error instead: sum_i fe_i = rho - 1.
     fe[0] = rho1 - (((fe[1] + fe[2]) + (fe[3] + fe[4])) + ((fe[5] + fe[6]) + (fe[7] + fe[8])));
   }
-  relax<R>(p.inv_tau, p.collision, p.smagorinsky != 0, io != 0, forced, rho, fe, fi, g);
+  relax<R>(p, p.collision, p.smagorinsky != 0, io != 0, forced, over_rho, fe, fi, g);
   if (!kRounded && S::kBytes == 4 && cons && !(fl & kInlet)) {
     // FP32 storage: the collision's float rounding would make the stored
     // populations carry slightly more or less than rho, which the next step's

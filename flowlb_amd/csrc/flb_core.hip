@@ -91,7 +91,7 @@ flb::Params params(const flb_handle* h, int bx) {
   p.N = h->Nd;
   p.NL = h->N;
   p.Np = h->Np;
-  p.inv_tau = h->inv_tau;
+  flb::set_relaxation(p, h->inv_tau);
   const bool force = h->opt.use_force != 0;
   p.fx = force ? h->opt.fx : 0.0f;
   p.fy = force ? h->opt.fy : 0.0f;
@@ -330,7 +330,8 @@ uint32_t row_pitch(const flb_options* o, uint32_t nx) {
 }
 
 int march_model(const flb_handle* h) {
-  if (h->opt.collision != FLB_SRT || h->opt.smagorinsky || h->alpha) return flb::kMarchGeneral;
+  if (h->opt.collision != FLB_SRT || h->opt.smagorinsky || h->alpha)
+    return h->opt.use_force || h->alpha ? flb::kMarchGeneral : flb::kMarchUnforced;
   return h->opt.use_force ? flb::kMarchForced : flb::kMarchPlain;
 }
 
@@ -363,7 +364,8 @@ int prepare_march(flb_handle* h, const uint8_t* flags) {
 
 flb::MarchShape march_shape(const flb_handle* h) {
   const uint32_t cols = flb::march_columns(flb::kMarchMax);
-  return flb::march_shape(h->cus, uint64_t((h->nx + cols - 1) / cols) * h->ny, h->elem_bytes);
+  return flb::march_shape(h->cus, uint64_t((h->nx + cols - 1) / cols) * h->ny, h->elem_bytes,
+                          h->opt.smagorinsky != 0);
 }
 
 }  // namespace
@@ -836,7 +838,8 @@ uint32_t march_strips(uint32_t nx, int steps, const std::vector<uint8_t>& io,
 // 1.5 wavefronts per SIMD (12 rows).  Where that gives long chunks, the chip
 // runs several rounds of wavefronts anyway and FP32 wants them short, so that
 // fewer rows are in flight: 8192 x 2048 79.8, 83.2, 84.3, 90.5 with 16, 24, 36,
-// 64 rows; FP16S, which is bound by the vector units, 70.6, 68.6, 66.1, 74.6.
+// 64 rows; FP16S, which is bound by the vector units, 70.6, 68.6, 66.1, 74.6
+// (5001 x 1001: 32 rows 2 to 10 % ahead of 36 or 40, which end a round short).
 // Below four rows nothing is gained (512 x 128: 3.3 us with 1 to 4).
 //
 // Steps per pass.  T = 4 moves the fewest bytes and was the fastest from
@@ -844,11 +847,17 @@ uint32_t march_strips(uint32_t nx, int steps, const std::vector<uint8_t>& io,
 // about 150; single steps 196).  Grids that give less than 1.5 wavefronts per
 // SIMD at four rows are bound by the chain of a wavefront, T (r + T - 1)
 // step-rows: T = 3 takes 3.1 us per step on 512 x 128 and 3.5 on 1024 x 256,
-// T = 4 3.4 and 4.0.
-MarchShape march_shape(int cus, uint64_t strip_rows, int elem_bytes) {
+// T = 4 3.4 and 4.0.  The subgrid model (heavy) adds two thirds to the
+// instructions of a step; in 16-bit storage, where the bytes were never the bound,
+// the halo then costs more than the bytes saved: 5001 x 1001 BF16S 30.7, 33.8, 34.4
+// with T = 2, 3, 4 (with TRT 36.6 with T = 2, single steps 42; FP32 keeps T = 4:
+// 46.9, 33.9, 33.2).
+MarchShape march_shape(int cus, uint64_t strip_rows, int elem_bytes, bool heavy) {
   const uint64_t waves = uint64_t(cus) * 6;  // 1.5 per SIMD
-  const uint32_t least = 4, most = elem_bytes == 2 ? 36 : 16;
+  const uint32_t least = 4, most = elem_bytes == 2 && !heavy ? 32 : 16;
   const uint64_t rows = (strip_rows + waves - 1) / waves;
+  if (elem_bytes == 2 && heavy)
+    return MarchShape{2, uint32_t(std::min<uint64_t>(std::max<uint64_t>(rows, least), most))};
   return MarchShape{rows < least ? 3 : 4,
                     uint32_t(std::min<uint64_t>(std::max<uint64_t>(rows, least), most))};
 }

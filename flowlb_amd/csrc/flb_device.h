@@ -173,6 +173,8 @@ struct Params {
   uint64_t NL;           // cells of the domain (nx * ny): host arrays, staging
   uint64_t Np;           // plane stride of the population array (elements)
   float inv_tau, fx, fy;
+  float tau;             // 1 / inv_tau, rounded
+  float trt_minus;       // TRT's antisymmetric rate for inv_tau (magic parameter 1/4)
   int32_t use_force, collision, smagorinsky, gas_check_corrected, mass_mode;
   void* f;               // populations, 9 planes of Np elements of the storage type
   uint8_t* flags;        // current flags
@@ -236,6 +238,12 @@ struct Params {
   // divide on the scalar unit (0 = divide instead).
   uint32_t band_magic, win_magic, last_magic;
 };
+
+inline void set_relaxation(Params& p, float inv_tau) {
+  p.inv_tau = inv_tau;
+  p.tau = 1.0f / inv_tau;
+  p.trt_minus = 1.0f / (0.25f / (p.tau - 0.5f) + 0.5f);
+}
 
 enum : int { kListFS1 = 0 };
 constexpr int kListThreads = 256;  // block size of the list-driven pass 1

@@ -53,7 +53,7 @@ struct MarchShape {
   int steps;
   uint32_t rows;
 };
-MarchShape march_shape(int cus, uint64_t strip_rows, int elem_bytes);
+MarchShape march_shape(int cus, uint64_t strip_rows, int elem_bytes, bool heavy);
 // Steps of the next pass of a run with `left` steps to go; 0: a single step.
 inline int march_steps_next(uint64_t left, int most) {
   if (left < 2) return 0;

@@ -139,19 +139,24 @@ struct Held<StoreBF16S> {
 };
 
 // Collision models compiled apart: plain SRT (no force, drag or subgrid
-// model), SRT with a body force, and everything by the handle's options.
-enum : int { kMarchPlain = 0, kMarchForced = 1, kMarchGeneral = 2 };
+// model), SRT with a body force, any collision and subgrid model without force
+// or drag, and everything by the handle's options.
+enum : int { kMarchPlain = 0, kMarchForced = 1, kMarchUnforced = 2, kMarchGeneral = 3 };
 // Wavefronts per SIMD the pass is compiled for (its registers: 128, 168, 256).
 template <class S, int MODEL>
 constexpr int march_occupancy() {
-  return S::kBytes > 4 ? 2 : (MODEL == kMarchGeneral ? 3 : 4);
+  return S::kBytes > 4 ? 2 : (MODEL >= kMarchUnforced ? 3 : 4);
 }
 
-// Previous-step values an inlet or outlet cell reads (stream_collide_cell).
+// What an inlet or outlet cell reads (stream_collide_cell): the published
+// density of the cell at x + 1 and velocity of the cell at x - 1, of the step
+// before, and its own published values.  An inlet cell never publishes a
+// velocity and an outlet cell's density never changes, so these hold the
+// velocity the inlet prescribes and the density the outlet keeps.
 template <class R>
 struct IoValues {
-  R rho_next;           // published density of the cell at x + 1
-  R ux_prev, uy_prev;   // published velocity of the cell at x - 1
+  R rho, ux, uy;
+  R rho_next, ux_prev, uy_prev;
 };
 
 // One step of one cell: g holds its incoming populations and receives the
@@ -178,10 +183,10 @@ __device__ __forceinline__ void march_cell(const Params& p, uint8_t fl, uint32_t
   if (IO && (io & kInlet)) {
     rho = v.rho_next;
     rho1 = rho - R(1);
-    ux = at(fld<R>(p.u), n);
-    uy = at(fld<R>(p.u) + p.N, n);
+    ux = v.ux;
+    uy = v.uy;
   } else if (IO && (io & kOutlet)) {
-    rho = at(fld<R>(p.rho), n);
+    rho = v.rho;
     rho1 = rho - R(1);
     ux = v.ux_prev;
     uy = v.uy_prev;
@@ -201,15 +206,15 @@ __device__ __forceinline__ void march_cell(const Params& p, uint8_t fl, uint32_t
   }
   R fi[9], fe[9];
   bool forced = false;
-  if (MODEL != kMarchPlain) {
+  if (MODEL == kMarchForced || MODEL == kMarchGeneral) {
     const bool brinkman = MODEL == kMarchGeneral && p.alpha && !io;
     forced = apply_force<R>(p, MODEL == kMarchForced || p.use_force != 0, brinkman,
                             brinkman ? R(at(p.alpha, n)) : R(0), rho, over_rho, ux, uy, fi, unit);
   }
   equilibrium_shifted<R>(rho, rho1, ux, uy, fe, unit);
-  const bool general = MODEL == kMarchGeneral;
-  relax<R>(p.inv_tau, general ? p.collision : 0, general && p.smagorinsky != 0, io != 0, forced, rho,
-           fe, fi, g, unit);
+  const bool any = MODEL >= kMarchUnforced;
+  relax<R>(p, any ? p.collision : 0, any && p.smagorinsky != 0, io != 0, forced, over_rho, fe,
+           fi, g, unit);
 }
 
 struct Fill { static constexpr bool value = false; };
@@ -240,6 +245,7 @@ __device__ __forceinline__ void march_rows(const Params& p, const March& a, uint
 
   E raw[9];
   uint8_t raw_fl;
+  IoValues<R> raw_io{};
   auto load_row = [&](uint32_t y) {
     const uint64_t rc = uint64_t(y) * pitch, ru = uint64_t(up(y)) * pitch,
                    rd = uint64_t(down(y)) * pitch;
@@ -255,6 +261,16 @@ __device__ __forceinline__ void march_rows(const Params& p, const March& a, uint
     raw[7] = at(here(7) + rc, x);
     raw[8] = at(there(7) + rd, xr);
     raw_fl = at(p.flags + rc, x);
+    if (IO) {  // the neighbours' too: the end lanes have none to take them from
+      const R* const r = fld<R>(const_cast<float*>(a.pub_rho_in)) + rc;
+      const R* const u = fld<R>(const_cast<float*>(a.pub_u_in)) + rc;
+      raw_io.rho = at(r, x);
+      raw_io.ux = at(u, x);
+      raw_io.uy = at(u + p.N, x);
+      raw_io.rho_next = at(r, xr);
+      raw_io.ux_prev = at(u, xl);
+      raw_io.uy_prev = at(u + p.N, xl);
+    }
   };
   auto store_row = [&](uint32_t y, const R* g) {
     const uint64_t rc = uint64_t(y) * pitch, ru = uint64_t(up(y)) * pitch,
@@ -293,11 +309,12 @@ __device__ __forceinline__ void march_rows(const Params& p, const March& a, uint
 #pragma unroll
     for (int i = 0; i < 9; i++) g[i] = Held<S>::in(raw[i]);
     fls = fls << 8 | raw_fl;
+    const IoValues<R> io_now = raw_io;
     const uint32_t y = y1;
     y1 = up(y1);
     load_row(y1);  // one row past the last is loaded and not used
     R rho = R(1), ux = R(0), uy = R(0);
-    R kept_r = R(0), kept_u = R(0), kept_v = R(0);  // published by step s - 1 (IO)
+    IoValues<R> kept = io_now;  // published by step s - 1 (IO)
     uint32_t ys = y;  // row of step s
 #pragma unroll
     for (int s = 1; s <= T; s++) {
@@ -305,26 +322,12 @@ __device__ __forceinline__ void march_rows(const Params& p, const March& a, uint
         const uint8_t fl = uint8_t(fls >> (8 * (s - 1)));
         const uint32_t n = ys * pitch + x;
         IoValues<R> v{};
-        R own_r = R(0), own_u = R(0), own_v = R(0);  // published at this cell so far
         if (IO) {
-          if (s == 1) {
-            // From memory: the end lanes are computed too and have no neighbour.
-            const R* const r_in = fld<R>(const_cast<float*>(a.pub_rho_in));
-            const R* const u_in = fld<R>(const_cast<float*>(a.pub_u_in));
-            const uint32_t left = ys * pitch + xl, right = ys * pitch + xr;
-            own_r = at(r_in, n);
-            own_u = at(u_in, n);
-            own_v = at(u_in + p.N, n);
-            v.rho_next = at(r_in, right);
-            v.ux_prev = at(u_in, left);
-            v.uy_prev = at(u_in + p.N, left);
-          } else {
-            own_r = kept_r;
-            own_u = kept_u;
-            own_v = kept_v;
-            v.rho_next = from_right(own_r);
-            v.ux_prev = from_left(own_u);
-            v.uy_prev = from_left(own_v);
+          v = kept;
+          if (s > 1) {
+            v.rho_next = from_right(v.rho);
+            v.ux_prev = from_left(v.ux);
+            v.uy_prev = from_left(v.uy);
           }
         }
         march_cell<S, MODEL, IO>(p, fl, n, v, g, rho, ux, uy);
@@ -376,12 +379,12 @@ __device__ __forceinline__ void march_rows(const Params& p, const March& a, uint
           rise0[b][1] = from_left(g[5]);
           rise0[b][2] = from_right(g[8]);
           if (IO) {
-            kept_r = pr[b];
-            kept_u = pu[b];
-            kept_v = pv[b];
-            pr[b] = solid ? own_r : rho;
-            pu[b] = solid || (fl & kInlet) ? own_u : ux;
-            pv[b] = solid || (fl & kInlet) ? own_v : uy;
+            kept.rho = pr[b];
+            kept.ux = pu[b];
+            kept.uy = pv[b];
+            pr[b] = solid ? v.rho : rho;
+            pu[b] = solid || (fl & kInlet) ? v.ux : ux;
+            pv[b] = solid || (fl & kInlet) ? v.uy : uy;
           }
 #pragma unroll
           for (int i = 0; i < 9; i++) g[i] = in[i];

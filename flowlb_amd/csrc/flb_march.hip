@@ -37,8 +37,12 @@ k_march(const Params p, const March a) {
 namespace {
 template <class S, int T>
 MarchFn march_fn(int model) {
-  if (model == kMarchPlain) return k_march<S, T, kMarchPlain>;
-  return model == kMarchForced ? k_march<S, T, kMarchForced> : k_march<S, T, kMarchGeneral>;
+  switch (model) {
+    case kMarchPlain: return k_march<S, T, kMarchPlain>;
+    case kMarchForced: return k_march<S, T, kMarchForced>;
+    case kMarchUnforced: return k_march<S, T, kMarchUnforced>;
+    default: return k_march<S, T, kMarchGeneral>;
+  }
 }
 template <class S>
 MarchFn march_steps(int steps, int model) {
