@@ -46,20 +46,105 @@ struct AdjParams {
   double qbar;          // 1 / number of averaged steps
 };
 
-// Equilibrium and its velocity derivatives with the weights of the forward
-// arithmetic T (float weights for FP32, exact ones for FP64).
+// Equilibrium derivatives with respect to the velocity at x, with the weights
+// of the forward arithmetic T (float weights for FP32, exact ones for FP64).
 template <class T>
-__device__ __forceinline__ void feq_grad(double rho, double ux, double uy, double* fe,
-                                         double* dfx, double* dfy) {
-  const double usq = ux * ux + uy * uy;
+__device__ __forceinline__ double feq_dx(double rho, double ux, double uy, int i) {
+  const double ex = double(cx(i)), cu = ex * ux + double(cy(i)) * uy;
+  return double(wgt_r<T>(i)) * rho * (3.0 * ex + 9.0 * cu * ex - 3.0 * ux);
+}
+
+// Weighted moments of nine adjoint values.  The collision's derivatives contract
+// them with polynomials of the velocities c_i of degree two at most, so six
+// moments replace three sums over the nine directions (equilibrium, and its two
+// velocity derivatives) and four more with a force: about 500 FP64 instructions
+// per cell became 130.
+struct Moments {
+  double s, x, y, xx, yy, xy;
+};
+template <class T>
+__device__ __forceinline__ Moments moments(const double* v) {
+  const double w0 = double(wgt_r<T>(0)), w1 = double(wgt_r<T>(1)), w5 = double(wgt_r<T>(5));
+  const double h = v[1] + v[2], k = v[3] + v[4], p = v[5] + v[6], m = v[7] + v[8];
+  const double d = p + m;
+  Moments r;
+  r.s = w0 * v[0] + w1 * (h + k) + w5 * d;
+  r.x = w1 * (v[1] - v[2]) + w5 * ((v[5] - v[6]) + (v[7] - v[8]));
+  r.y = w1 * (v[3] - v[4]) + w5 * ((v[5] - v[6]) + (v[8] - v[7]));
+  r.xx = w1 * h + w5 * d;
+  r.yy = w1 * k + w5 * d;
+  r.xy = w5 * (p - m);
+  return r;
+}
+
+// Adjoint of feq(rho, u) from the moments of the adjoints of its nine values.
+__device__ __forceinline__ void feq_adjoint(const Moments& m, double rho, double ux, double uy,
+                                            double& rb, double& ubx, double& uby) {
+  const double qx = ux * m.xx + uy * m.xy, qy = ux * m.xy + uy * m.yy;
+  rb = m.s * (1.0 - 1.5 * (ux * ux + uy * uy)) + 3.0 * (ux * m.x + uy * m.y) +
+       4.5 * (ux * qx + uy * qy);
+  ubx = rho * (3.0 * (m.x - ux * m.s) + 9.0 * qx);
+  uby = rho * (3.0 * (m.y - uy * m.s) + 9.0 * qy);
+}
+
+// Reverse of one cell's step.  v: adjoints of the populations it emitted;
+// rb, ubx, uby: adjoints of its density and velocity as published (0 where none);
+// t0, t1, t2: its trace.  gb: adjoints of the populations it received; ab: of
+// its solid fraction.  For an inlet or outlet cell (io) gb is zero and rb, ubx,
+// uby become the adjoints of the density and velocity it read.  `in_window`:
+// the objective takes the discharge here at this step.
+template <class T>
+__device__ __forceinline__ void adjoint_cell(const Params& p, bool io, double al, double t0,
+                                             double t1, double t2, bool in_window, double qbar,
+                                             const double* v, double* gb, double& rb, double& ubx,
+                                             double& uby, double& ab) {
+  const double Fx = p.use_force ? p.fx : 0.0f, Fy = p.use_force ? p.fy : 0.0f;
+  const Moments m = moments<T>(v);
+  double r, x, y;
+  const double rho = t0, inv = 1.0 / rho;
+  if (io) {
+    // populations = feq(rho, u_read + F/(2 rho)): no dependence on the loaded ones
+    const double ux = t1 + 0.5 * inv * Fx, uy = t2 + 0.5 * inv * Fy;
+    feq_adjoint(m, rho, ux, uy, r, x, y);
+    ubx += x;
+    uby += y;
+    rb += r - (ubx * Fx + uby * Fy) * 0.5 * inv * inv;
 #pragma unroll
-  for (int i = 0; i < 9; i++) {
-    const double w = double(wgt_r<T>(i)), ex = double(cx(i)), ey = double(cy(i));
-    const double cu = ex * ux + ey * uy;
-    fe[i] = w * rho * (1.0 + 3.0 * cu + 4.5 * cu * cu - 1.5 * usq);
-    dfx[i] = w * rho * (3.0 * ex + 9.0 * cu * ex - 3.0 * ux);
-    dfy[i] = w * rho * (3.0 * ey + 9.0 * cu * ey - 3.0 * uy);
+    for (int i = 0; i < 9; i++) gb[i] = 0.0;
+    ab = 0.0;
+    return;
   }
+  const double sa = 1.0 / (1.0 + 0.5 * al), si = sa * inv;
+  const double ux = (t1 + 0.5 * Fx) * si, uy = (t2 + 0.5 * Fy) * si;
+  // The forward's SRT weights are float constants (also in FP64).
+  const double om = p.inv_tau, omc = 1.0f - p.inv_tau, tl = 1.0f - 0.5f * p.inv_tau;
+  feq_adjoint(m, rho, ux, uy, r, x, y);
+  rb += om * r;
+  ubx += om * x;
+  uby += om * y;
+  ab = 0.0;
+  if (p.use_force || p.alpha) {
+    const double k3 = double(0.33333334f), f = 9.0 * tl;
+    const double Gx = Fx - al * rho * ux, Gy = Fy - al * rho * uy;
+    ubx += f * (Gx * m.xx + Gy * m.xy - k3 * Gx * m.s);
+    uby += f * (Gx * m.xy + Gy * m.yy - k3 * Gy * m.s);
+    const double Gbx = f * (ux * m.xx + uy * m.xy + k3 * (m.x - ux * m.s));
+    const double Gby = f * (ux * m.xy + uy * m.yy + k3 * (m.y - uy * m.s));
+    const double uG = ux * Gbx + uy * Gby;
+    ubx += -al * rho * Gbx;
+    uby += -al * rho * Gby;
+    rb += -al * uG;
+    ab = -rho * uG;
+  }
+  if (in_window) {  // J += qbar * rho * u_x
+    rb += qbar * ux;
+    ubx += qbar * rho;
+  }
+  const double mbx = ubx * si, mby = uby * si, ubu = ubx * ux + uby * uy;
+  rb += -ubu * inv;
+  ab += -0.5 * sa * ubu;
+#pragma unroll
+  for (int i = 0; i < 9; i++) gb[i] = omc * v[i] + (rb + along(i, mbx, mby));
 }
 
 __device__ __forceinline__ uint32_t cell_neighbour(const Params& p, uint32_t x, uint32_t y, int i) {
@@ -137,78 +222,19 @@ __global__ void __launch_bounds__(256) k_adjoint_step(const Params p, const AdjP
         a.ubar[ODD][n] = 0.0;
         a.ubar[ODD][N + n] = 0.0;
       }
-      const double Fx = p.use_force ? p.fx : 0.0f, Fy = p.use_force ? p.fy : 0.0f;
       const T* const tr = static_cast<const T*>(a.trace);
-      const double t0 = tr[n], t1 = tr[N + n], t2 = tr[2 * N + n];
       const uint8_t io = fl & (kInlet | kOutlet);
-      double gb[9];
-      if (io) {
-        // populations = feq(rho, u_read + F/(2 rho)): no dependence on the loaded ones
-        const double rho = t0;
-        const double ux = t1 + 0.5 / rho * Fx, uy = t2 + 0.5 / rho * Fy;
-        double fe[9], dfx[9], dfy[9];
-        feq_grad<T>(rho, ux, uy, fe, dfx, dfy);
-#pragma unroll
-        for (int i = 0; i < 9; i++) {
-          rb += v[i] * fe[i] / rho;
-          ubx += v[i] * dfx[i];
-          uby += v[i] * dfy[i];
-          gb[i] = 0.0;
-        }
-        rb += -(ubx * Fx + uby * Fy) * 0.5 / (rho * rho);
-        if (io & kInlet) {
-          a.rbar[ODD ^ 1][lin.next] += rb;
-          duin = ubx;
-        } else {
-          a.ubar[ODD ^ 1][lin.prev] += ubx;
-          a.ubar[ODD ^ 1][N + lin.prev] += uby;
-        }
-      } else {
-        const double rho = t0, mx = t1, my = t2;
-        const double al = p.alpha ? p.alpha[n] : 0.0f;
-        const double sa = 1.0 / (1.0 + 0.5 * al);
-        const double ux = (mx + 0.5 * Fx) * sa / rho, uy = (my + 0.5 * Fy) * sa / rho;
-        const double Gx = Fx - al * rho * ux, Gy = Fy - al * rho * uy;
-        const bool forced = p.use_force || p.alpha;
-        // The forward's SRT weights are float constants (also in FP64).
-        const double om = p.inv_tau, omc = 1.0f - p.inv_tau, tl = 1.0f - 0.5f * p.inv_tau;
-        const double k3 = double(0.33333334f);
-        double fe[9], dfx[9], dfy[9];
-        feq_grad<T>(rho, ux, uy, fe, dfx, dfy);
-        double Gbx = 0.0, Gby = 0.0;
-#pragma unroll
-        for (int i = 0; i < 9; i++) {
-          const double ex = double(cx(i)), ey = double(cy(i));
-          gb[i] = omc * v[i];
-          const double feb = om * v[i];
-          rb += feb * fe[i] / rho;
-          ubx += feb * dfx[i];
-          uby += feb * dfy[i];
-          if (forced) {
-            const double Fb = tl * v[i] * 9.0 * double(wgt_r<T>(i));
-            const double cG = ex * Gx + ey * Gy;
-            const double cu = ex * ux + ey * uy;
-            ubx += Fb * (cG * ex - k3 * Gx);
-            uby += Fb * (cG * ey - k3 * Gy);
-            Gbx += Fb * (ex * (cu + k3) - k3 * ux);
-            Gby += Fb * (ey * (cu + k3) - k3 * uy);
-          }
-        }
-        ubx += -al * rho * Gbx;
-        uby += -al * rho * Gby;
-        rb += -al * (ux * Gbx + uy * Gby);
-        double ab = -rho * (ux * Gbx + uy * Gby);
-        if (a.in_window && x == a.column) {  // J += qbar * rho * u_x
-          rb += a.qbar * ux;
-          ubx += a.qbar * rho;
-        }
-        const double mbx = ubx * sa / rho, mby = uby * sa / rho;
-        const double ubu = ubx * ux + uby * uy;
-        rb += -ubu / rho;
-        ab += -0.5 * sa * ubu;
-#pragma unroll
-        for (int i = 0; i < 9; i++) gb[i] += rb + double(cx(i)) * mbx + double(cy(i)) * mby;
-        if (a.galpha) a.galpha[n] += ab;
+      double gb[9], ab;
+      adjoint_cell<T>(p, io != 0, p.alpha ? p.alpha[n] : 0.0f, tr[n], tr[N + n], tr[2 * N + n],
+                      a.in_window && x == a.column, a.qbar, v, gb, rb, ubx, uby, ab);
+      if (io & kInlet) {
+        a.rbar[ODD ^ 1][lin.next] += rb;
+        duin = ubx;
+      } else if (io) {
+        a.ubar[ODD ^ 1][lin.prev] += ubx;
+        a.ubar[ODD ^ 1][N + lin.prev] += uby;
+      } else if (a.galpha) {
+        a.galpha[n] += ab;
       }
 #pragma unroll
       for (int i = 0; i < 9; i++) a.abar[load_index<ODD>(p, n, nb, i)] = gb[i];
@@ -233,10 +259,10 @@ __global__ void __launch_bounds__(256) k_adjoint_inlet_init(const Params p, cons
       nb[0] = n;
 #pragma unroll
       for (int i = 1; i < 9; i++) nb[i] = cell_neighbour(p, x, y, i);
-      double fe[9], dfx[9], dfy[9];
-      feq_grad<double>(a.rho_init[n], a.u_init[n], a.u_init[p.N + n], fe, dfx, dfy);
 #pragma unroll
-      for (int i = 0; i < 9; i++) acc += a.abar[store_index<1>(p, n, nb, i)] * dfx[i];
+      for (int i = 0; i < 9; i++)
+        acc += a.abar[store_index<1>(p, n, nb, i)] *
+               feq_dx<double>(a.rho_init[n], a.u_init[n], a.u_init[p.N + n], i);
     }
   }
   block_add(acc, a.duin);
@@ -271,20 +297,18 @@ namespace {
       return flb::set_error((h), FLB_ERR_DEVICE, std::string(#call) + ": " + hipGetErrorString(e_)); \
   } while (0)
 
-struct DevBuf {
-  std::vector<void*> ptrs;
-  ~DevBuf() {
-    for (void* p : ptrs) (void)hipFree(p);
-  }
-  template <class T>
-  T* get(size_t count) {
-    void* v = nullptr;
-    if (hipMalloc(&v, std::max<size_t>(count, 1) * sizeof(T)) != hipSuccess) {
+// Bounds what a handle keeps of its buffers after a call, a sixteenth of the
+// device's memory (18 GB of 288; a gradient of 2000 steps of 1024 x 256 takes
+// 6.3 GB in FP32, 12.6 GB in FP64).
+struct TrimWork {
+  flb_handle* h;
+  ~TrimWork() {
+    size_t left = 0, total = 0;
+    if (hipMemGetInfo(&left, &total) != hipSuccess) {
       (void)hipGetLastError();
-      return nullptr;
+      total = 0;
     }
-    ptrs.push_back(v);
-    return static_cast<T*>(v);
+    h->work.trim(total / 16);
   }
 };
 
@@ -381,9 +405,10 @@ int flb_set_brinkman(flb_handle* h, const float* alpha) {
 int flb_objective(flb_handle* h, const flb_adjoint_spec* sp, double* J) {
   int rc = check_adjoint_state(h, sp);
   if (rc) return rc;
-  DevBuf mem;
-  uint8_t* saved = mem.get<uint8_t>(state_bytes(h, true));
-  double* d_j = mem.get<double>(1);
+  using W = flb::Workspace;
+  TrimWork trim{h};
+  uint8_t* saved = h->work.get<uint8_t>(W::kState, state_bytes(h, true));
+  double* d_j = h->work.get<double>(W::kSums, 2);
   if (!saved || !d_j) return flb::set_error(h, FLB_ERR_MEMORY, "objective buffers");
   if ((rc = copy_state(h, saved, false, true))) return rc;
   ADJ_HIP(h, hipMemsetAsync(d_j, 0, sizeof(double), h->stream));
@@ -415,23 +440,31 @@ int flb_adjoint(flb_handle* h, const flb_adjoint_spec* sp, double* J, float* dj_
   if (budget == 0) {
     size_t free_b = 0, total_b = 0;
     ADJ_HIP(h, hipMemGetInfo(&free_b, &total_b));
-    budget = free_b / 2;
+    budget = (free_b + h->work.held()) / 2;  // what the handle kept counts as free
   }
   const uint64_t resident = std::min<uint64_t>(nseg, budget / seg_bytes);
   const uint64_t first_res = nseg - resident;  // segments [0, first_res) are recomputed
-  DevBuf mem;
-  uint8_t* ckpt = first_res ? mem.get<uint8_t>(first_res * ck_bytes) : nullptr;
-  uint8_t* fields0 = mem.get<uint8_t>(state_bytes(h, true));
-  uint8_t* trace_res = resident ? mem.get<uint8_t>(resident * seg_bytes) : nullptr;
-  uint8_t* trace_tmp = first_res ? mem.get<uint8_t>(seg_bytes) : nullptr;
-  double* abar = mem.get<double>(9 * Np);
-  double* rbar = mem.get<double>(2 * N);
-  double* ubar = mem.get<double>(4 * N);
-  double* galpha = h->alpha ? mem.get<double>(N) : nullptr;
-  double* d_acc = mem.get<double>(2);  // J, dJ/du_in
-  if ((first_res && (!ckpt || !trace_tmp)) || (resident && !trace_res) || !fields0 || !abar ||
-      !rbar || !ubar || (h->alpha && !galpha) || !d_acc)
-    return flb::set_error(h, FLB_ERR_MEMORY, "adjoint buffers (checkpoints, trace, adjoint state)");
+  using W = flb::Workspace;
+  TrimWork trim{h};
+  uint8_t *ckpt = nullptr, *fields0 = nullptr, *trace_res = nullptr, *trace_tmp = nullptr;
+  double *abar = nullptr, *rbar = nullptr, *ubar = nullptr, *galpha = nullptr, *d_acc = nullptr;
+  auto buffers = [&]() {
+    flb::Workspace& w = h->work;
+    return (!first_res || ((ckpt = w.get<uint8_t>(W::kCheckpoints, first_res * ck_bytes)) &&
+                           (trace_tmp = w.get<uint8_t>(W::kTraceOnce, seg_bytes)))) &&
+           (!resident || (trace_res = w.get<uint8_t>(W::kTrace, resident * seg_bytes))) &&
+           (fields0 = w.get<uint8_t>(W::kState, state_bytes(h, true))) &&
+           (abar = w.get<double>(W::kAdjoint, 9 * Np)) &&
+           (rbar = w.get<double>(W::kDensity, 2 * N)) &&
+           (ubar = w.get<double>(W::kVelocity, 4 * N)) &&
+           (!h->alpha || (galpha = w.get<double>(W::kAlpha, N))) &&
+           (d_acc = w.get<double>(W::kSums, 2));  // J, dJ/du_in
+  };
+  if (!buffers()) {
+    h->work.trim(0);  // buffers of an earlier call may be what is in the way
+    if (!buffers())
+      return flb::set_error(h, FLB_ERR_MEMORY, "adjoint buffers (checkpoints, trace, adjoint state)");
+  }
   auto seg_trace = [&](uint64_t s) {
     return s >= first_res ? trace_res + (s - first_res) * seg_bytes : trace_tmp;
   };

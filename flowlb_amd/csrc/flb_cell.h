@@ -94,6 +94,7 @@ __device__ __forceinline__ void equilibrium_surface(R rho, R rho1, R ux, R uy, R
 // c_i . v, as a sum (no products with 0 and 1).
 template <class R>
 __device__ __forceinline__ R along(int i, R vx, R vy) {
+  if (i == 0) return R(0);
   const R a = cx(i) < 0 ? -vx : vx, b = cy(i) < 0 ? -vy : vy;
   return cx(i) == 0 ? b : (cy(i) == 0 ? a : a + b);
 }
