@@ -283,7 +283,36 @@ __global__ void __launch_bounds__(256) k_discharge(const Params p, uint32_t colu
   for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
   if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = s;
   __syncthreads();
-  if (threadIdx.x == 0) acc[0] += scale * (lds[0] + lds[1] + lds[2] + lds[3]);
+  if (threadIdx.x == 0) acc[0] = fma(scale, lds[0] + lds[1] + lds[2] + lds[3], acc[0]);
+}
+
+// The same of `steps` steps recorded by passes, ny values each: the sums of
+// k_discharge in its order, and the steps in theirs, so that neither the length
+// of the passes nor that of the segments changes a bit.
+constexpr uint32_t kDischargeSteps = 256;
+__global__ void __launch_bounds__(1024) k_discharge_rows(const double* rows, uint32_t steps,
+                                                         uint32_t ny, double scale, double* acc) {
+  __shared__ double q[kDischargeSteps];
+  const uint32_t lane = threadIdx.x & 63u;
+  for (uint32_t k = threadIdx.x >> 6; k < steps; k += blockDim.x >> 6) {
+    const double* const r = rows + uint64_t(k) * ny;
+    double sum[4];
+#pragma unroll
+    for (uint32_t w = 0; w < 4; w++) {
+      double s = 0.0;
+      for (uint32_t y = w * 64u + lane; y < ny; y += 256u) s += r[y];
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
+      sum[w] = s;
+    }
+    if (lane == 0) q[k] = sum[0] + sum[1] + sum[2] + sum[3];
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double s = acc[0];
+    for (uint32_t k = 0; k < steps; k++) s = fma(scale, q[k], s);
+    acc[0] = s;
+  }
 }
 
 }  // namespace flb
@@ -355,29 +384,78 @@ int check_adjoint_state(flb_handle* h, const flb_adjoint_spec* sp) {
   return FLB_OK;
 }
 
+using flb::kDischargeSteps;
+
 // Forward steps [t, t+count) with the objective accumulated into d_j; with a
-// trace buffer, step t + k records its trace at trace + k * 3 N values.
+// trace buffer, step t + k records its trace at trace + k * 3 N values.  In
+// passes of several steps where the handle has them: the averaged steps record
+// the column's discharge, summed every kDischargeSteps steps and at the end,
+// which takes the place of a reduction of one block after each step.  600 steps of
+// 1024 x 256 in FP32 with the trace: 4.31 ms step by step, 3.29 ms (the trace's
+// 1.9 GB take 0.4 ms at the rate of a copy; the rest is the passes' arithmetic
+// on a domain of one wavefront per SIMD).
 int run_forward(flb_handle* h, uint64_t count, const flb_adjoint_spec* sp, double qscale,
                 double* d_j, uint8_t* trace = nullptr) {
   const bool fp64 = h->opt.storage == FLB_STORAGE_FP64;
   const int bx = flb::handle_block_x(h);
-  for (uint64_t k = 0; k < count; ++k) {
+  const int most = flb::march_most(h);
+  double* q = nullptr;
+  if (most && d_j) {
+    q = h->work.get<double>(flb::Workspace::kColumn, uint64_t(kDischargeSteps) * h->ny);
+    if (!q) return flb::set_error(h, FLB_ERR_MEMORY, "discharge of the averaged steps");
+  }
+  uint64_t held = 0;  // steps in q
+  auto flush = [&]() -> int {
+    if (held)
+      hipLaunchKernelGGL(flb::k_discharge_rows, dim3(1), dim3(1024), 0, h->stream, q,
+                         uint32_t(held), h->ny, qscale, d_j);
+    held = 0;
+    ADJ_HIP(h, hipGetLastError());
+    return FLB_OK;
+  };
+  int rc = FLB_OK;
+  for (uint64_t k = 0; k < count && !rc;) {
     const uint64_t t = h->t;
+    uint8_t* const to = trace ? trace + k * 3 * h->Nd * h->field_bytes : nullptr;
     const bool win = d_j && t >= sp->t0 && t <= sp->t1;
+    // A pass lies in the averaged steps as a whole or not at all.
+    uint64_t left = count - k;
+    if (d_j && t < sp->t0) left = std::min(left, sp->t0 - t);
+    if (win) left = std::min(left, sp->t1 + 1 - t);
+    const int T = most ? flb::march_steps_next(left, most) : 0;
+    if (T && (trace || win)) {
+      if (win && held + uint64_t(T) > kDischargeSteps && (rc = flush())) break;
+      flb::MarchTrace m{};
+      m.trace = to;
+      m.discharge = win ? q + held * h->ny : nullptr;
+      m.column = sp->column;
+      m.window = win ? (1u << T) - 1u : 0u;
+      if (win) held += uint64_t(T);
+      rc = flb::enqueue_march_ex(h, T, false, &m);
+      k += uint64_t(T);
+      continue;
+    }
+    if (T) {
+      rc = flb::enqueue_march_ex(h, T, false, nullptr);
+      k += uint64_t(T);
+      continue;
+    }
     flb::Params p = flb::make_params(h, bx);
-    p.trace = trace ? reinterpret_cast<float*>(trace + k * 3 * h->Nd * h->field_bytes) : nullptr;
+    p.trace = reinterpret_cast<float*>(to);
     hipLaunchKernelGGL(trace ? flb::get_stream_collide_trace(h->opt.storage, int(t & 1), win)
                              : flb::get_stream_collide(h->opt.storage, int(t & 1), false, win),
                        dim3(p.nblocks), dim3(bx), 0, h->stream, p);
     ADJ_HIP(h, hipGetLastError());
     if (win) {
+      if ((rc = flush())) break;
       hipLaunchKernelGGL(fp64 ? flb::k_discharge<double> : flb::k_discharge<float>, dim3(1),
                          dim3(256), 0, h->stream, p, sp->column, qscale, d_j);
       ADJ_HIP(h, hipGetLastError());
     }
     h->t += 1;
+    ++k;
   }
-  return FLB_OK;
+  return rc ? rc : flush();
 }
 
 }  // namespace

@@ -330,8 +330,10 @@ uint32_t row_pitch(const flb_options* o, uint32_t nx) {
 }
 
 int march_model(const flb_handle* h) {
-  if (h->opt.collision != FLB_SRT || h->opt.smagorinsky || h->alpha)
-    return h->opt.use_force || h->alpha ? flb::kMarchGeneral : flb::kMarchUnforced;
+  const bool srt = h->opt.collision == FLB_SRT && !h->opt.smagorinsky;
+  if (h->alpha)
+    return srt && h->elem_bytes >= 4 ? flb::kMarchDrag : flb::kMarchGeneral;
+  if (!srt) return h->opt.use_force ? flb::kMarchGeneral : flb::kMarchUnforced;
   return h->opt.use_force ? flb::kMarchForced : flb::kMarchPlain;
 }
 
@@ -764,7 +766,7 @@ static int enqueue_step(flb_handle* h, bool moments, hipEvent_t* ev) {
 }
 
 // T steps of a single-phase handle in one pass (flb_march.h).
-static int enqueue_march(flb_handle* h, int T, bool moments) {
+static int enqueue_march(flb_handle* h, int T, bool moments, const flb::MarchTrace* trace = nullptr) {
   const flb::Params p = params(h, int(flb::kMarchLanes));
   const int last = int((h->t & 1u) ^ 1u);  // parity the step before published at
   flb::March a{};
@@ -776,19 +778,15 @@ static int enqueue_march(flb_handle* h, int T, bool moments) {
   a.pub_u_out = h->pub_u[last ^ 1];
   a.odd = int32_t(h->t & 1u);
   a.moments = moments;
-  const uint32_t cols = flb::march_columns(T);
-  constexpr uint32_t G = flb::kMarchWaves;
-  a.strips = (h->nx + cols - 1) / cols;
-  a.io_strips = h->march_io[T];
-  a.order = h->march_order[T];
-  a.rows = march_shape(h).rows;
-  a.chunks = (h->ny + a.rows - 1) / a.rows;
-  a.io_rows = (a.rows + G - 1) / G;
-  a.groups = (a.strips - a.io_strips + G - 1) / G;
-  a.group_magic = flb::div_magic(a.groups);
-  const uint32_t blocks = a.io_strips * a.chunks + (a.groups * a.chunks + 7u) / 8u * 8u;
-  hipLaunchKernelGGL(flb::get_march(h->opt.storage, T, march_model(h)), dim3(blocks),
-                     dim3(64 * G), 0, h->stream, p, a);
+  a.grid = flb::march_grid(h, T);
+  if (trace) {
+    a.trace = trace->trace;
+    a.discharge = trace->discharge;
+    a.column = trace->column;
+    a.window = trace->window;
+  }
+  hipLaunchKernelGGL(flb::get_march(h->opt.storage, T, march_model(h), trace != nullptr),
+                     dim3(a.grid.blocks), dim3(64 * flb::kMarchWaves), 0, h->stream, p, a);
   FLB_HIP(h, hipGetLastError());
   std::swap(h->f, h->f_alt);
   // The last step published at the other index; after an even number of steps
@@ -988,6 +986,25 @@ Params make_params(const flb_handle* h, int bx) { return params(h, bx); }
 int handle_block_x(const flb_handle* h) { return block_x(h); }
 int enqueue_step_ex(flb_handle* h, bool moments, hipEvent_t* ev) {
   return enqueue_step(h, moments, ev);
+}
+int enqueue_march_ex(flb_handle* h, int T, bool moments, const MarchTrace* trace) {
+  return enqueue_march(h, T, moments, trace);
+}
+int march_most(const flb_handle* h) { return h->f_alt ? ::march_shape(h).steps : 0; }
+MarchGrid march_grid(const flb_handle* h, int T) {
+  const uint32_t cols = march_columns(T);
+  constexpr uint32_t G = kMarchWaves;
+  MarchGrid g{};
+  g.strips = (h->nx + cols - 1) / cols;
+  g.io_strips = h->march_io[T];
+  g.order = h->march_order[T];
+  g.rows = ::march_shape(h).rows;
+  g.chunks = (h->ny + g.rows - 1) / g.rows;
+  g.io_rows = (g.rows + G - 1) / G;
+  g.groups = (g.strips - g.io_strips + G - 1) / G;
+  g.group_magic = div_magic(g.groups);
+  g.blocks = g.io_strips * g.chunks + (g.groups * g.chunks + 7u) / 8u * 8u;
+  return g;
 }
 int copy_cells_in(flb_handle* h, void* dev, const void* host, size_t elem, int planes) {
   return cells_in(h, dev, host, elem, planes);

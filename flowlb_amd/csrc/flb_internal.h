@@ -46,6 +46,7 @@ HistFn get_flag_hist();
 
 // The multi-step pass (flb_march.h): `steps` in [kMarchMin, kMarchMax].
 struct March;
+struct MarchGrid;
 using MarchFn = void (*)(const Params, const March);
 constexpr int kMarchMin = 2, kMarchMax = 4;
 // Shape of the passes of a run of steps: steps per pass and rows per chunk.
@@ -68,7 +69,8 @@ uint32_t march_strips(uint32_t nx, int steps, const std::vector<uint8_t>& io,
 // inlet cell in the last column or an outlet cell in the first one reads the
 // linear neighbour in another row, and a pass needs as many rows as steps.
 bool march_columns_io(const uint8_t* flags, uint32_t nx, uint32_t ny, std::vector<uint8_t>& io);
-MarchFn get_march(int storage, int steps, int model);
+// trace: record the trace (SRT with or without drag; FP32 and FP64).
+MarchFn get_march(int storage, int steps, int model, bool trace);
 }  // namespace flb
 
 namespace flb {
@@ -108,7 +110,7 @@ namespace flb {
 // trim() gives back what exceeds its bound.
 struct Workspace {
   enum Slot { kCheckpoints, kState, kTrace, kTraceOnce, kAdjoint, kAdjointAlt, kDensity, kVelocity,
-              kAlpha, kSums, kSlots };
+              kAlpha, kSums, kColumn, kSlots };
   void* ptr[kSlots] = {};
   size_t size[kSlots] = {};
   Workspace() = default;
@@ -226,7 +228,16 @@ namespace flb {
 int set_error(flb_handle* h, int code, const std::string& msg);
 Params make_params(const flb_handle* h, int bx);
 int handle_block_x(const flb_handle* h);
-int enqueue_step_ex(flb_handle* h, bool moments, hipEvent_t* ev);
+// A pass of T steps.  trace: as March::trace, with the window bits and the
+// buffer for the discharge of `column` (nullptr: no trace).
+struct MarchTrace {
+  void* trace;
+  double* discharge;
+  uint32_t column, window;
+};
+int enqueue_march_ex(flb_handle* h, int T, bool moments, const MarchTrace* trace);
+MarchGrid march_grid(const flb_handle* h, int T);
+int march_most(const flb_handle* h);  // steps per pass of a long run, 0: no passes
 // Copies `planes` planes of cells of `elem` bytes between a host array
 // (planes of nx * ny, row-major) and a pitched device array (planes of Nd),
 // on the handle's stream, and waits for the copy.

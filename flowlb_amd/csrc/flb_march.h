@@ -37,6 +37,49 @@ constexpr uint32_t kMarchLanes = 64;
 constexpr int kMarchWaves = 4;  // wavefronts per block
 constexpr uint32_t march_columns(int steps) { return kMarchLanes - 2u * uint32_t(steps - 1); }
 
+// Blocks of a pass over a single domain.  The first io_strips * chunks blocks take
+// a chunk of an inlet/outlet strip each, split by rows between their wavefronts
+// (such a strip costs two to three times the others: with whole chunks these
+// wavefronts ended last, alone).  The others take a chunk of kMarchWaves adjacent
+// strips, which stay within a row of each other (a barrier per row), so that
+// the lines two strips share are read and written while they are in the L2.
+// Block b runs on XCD b mod 8; one XCD's blocks take consecutive groups of strips.
+struct MarchGrid {
+  uint32_t strips, io_strips;  // strips, and those whose 64 columns hold an inlet or outlet cell
+  uint32_t chunks;             // chunks of rows
+  uint32_t rows;               // rows per chunk
+  uint32_t io_rows;            // rows a wavefront takes of a chunk of such a strip
+  uint32_t groups, group_magic;  // blocks per chunk of the other strips, div_magic of it
+  uint32_t blocks;
+  const uint32_t* order;       // strips, the io_strips ones first
+};
+struct MarchWork {
+  uint32_t strip, ya, yb;  // nothing to do where ya >= yb
+  bool io;
+};
+__device__ __forceinline__ MarchWork march_work(const MarchGrid& g, uint32_t ny) {
+  const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(threadIdx.x / 64u));
+  const uint32_t io_blocks = g.io_strips * g.chunks;
+  MarchWork w{};
+  if (blockIdx.x < io_blocks) {
+    const uint32_t chunk = blockIdx.x / g.io_strips;
+    w.io = true;
+    w.strip = g.order[blockIdx.x - chunk * g.io_strips];
+    w.ya = chunk * g.rows + wave * g.io_rows;
+    w.yb = min(w.ya + g.io_rows, min((chunk + 1u) * g.rows, ny));
+    return w;
+  }
+  const uint32_t b = blockIdx.x - io_blocks, per = (gridDim.x - io_blocks) / 8u;
+  const uint32_t i = (b % 8u) * per + b / 8u;
+  const uint32_t chunk = div_by(i, g.groups, g.group_magic);
+  const uint32_t k = g.io_strips + (i - chunk * g.groups) * uint32_t(kMarchWaves) + wave;
+  if (k >= g.strips) return w;
+  w.strip = g.order[k];
+  w.ya = chunk * g.rows;
+  w.yb = min(w.ya + g.rows, ny);
+  return w;
+}
+
 // One pass of T steps, from time t.
 struct March {
   const void* f_in;   // populations at time t
@@ -49,12 +92,13 @@ struct March {
   float* pub_u_out;
   int32_t odd;        // t % 2
   int32_t moments;    // write the readback fields of the last step
-  uint32_t strips, io_strips;  // strips, and those whose 64 columns hold an inlet or outlet cell
-  uint32_t chunks;    // chunks of rows
-  uint32_t rows;      // rows per chunk
-  uint32_t io_rows;   // rows a wavefront takes of a chunk of such a strip
-  uint32_t groups, group_magic;  // blocks per chunk of the other strips, div_magic of it
-  const uint32_t* order;  // strips, the io_strips ones first
+  // TRACE: the trace of step t + k at trace + k * 3 N elements of R; and, where
+  // bit k of window is set, rho u_x of the cells of `column` (0 for walls) at
+  // discharge + k * ny, for the objective.
+  void* trace;
+  double* discharge;
+  uint32_t column, window;
+  MarchGrid grid;
 };
 
 // Value of the lane one to the left (lower x) / right.  The lanes at the ends
@@ -140,8 +184,9 @@ struct Held<StoreBF16S> {
 
 // Collision models compiled apart: plain SRT (no force, drag or subgrid
 // model), SRT with a body force, any collision and subgrid model without force
-// or drag, and everything by the handle's options.
-enum : int { kMarchPlain = 0, kMarchForced = 1, kMarchUnforced = 2, kMarchGeneral = 3 };
+// or drag, everything by the handle's options, and SRT with drag (TRACE too).
+enum : int { kMarchPlain = 0, kMarchForced = 1, kMarchUnforced = 2, kMarchGeneral = 3,
+             kMarchDrag = 4 };
 // Wavefronts per SIMD the pass is compiled for (its registers: 128, 168, 256).
 template <class S, int MODEL>
 constexpr int march_occupancy() {
@@ -161,11 +206,13 @@ struct IoValues {
 
 // One step of one cell: g holds its incoming populations and receives the
 // ones it emits; rho, ux, uy are set for cells that collide.
+// `alpha` is the cell's solid fraction (kMarchDrag); tr receives its trace
+// (stream_collide_cell).
 template <class S, int MODEL, bool IO>
-__device__ __forceinline__ void march_cell(const Params& p, uint8_t fl, uint32_t n,
+__device__ __forceinline__ void march_cell(const Params& p, uint8_t fl, uint32_t n, float alpha,
                                            const IoValues<typename S::R>& v, typename S::R* g,
                                            typename S::R& rho, typename S::R& ux,
-                                           typename S::R& uy) {
+                                           typename S::R& uy, typename S::R* tr) {
 #pragma clang fp contract(off)
   using R = typename S::R;
   if (fl & (kGas | kWall)) {
@@ -199,6 +246,9 @@ __device__ __forceinline__ void march_cell(const Params& p, uint8_t fl, uint32_t
     mx = (g[1] - g[2] + g[5] - g[6] + g[7] - g[8]) * (R(1) / unit);
     my = (g[3] - g[4] + g[5] - g[6] + g[8] - g[7]) * (R(1) / unit);
   }
+  tr[0] = rho;
+  tr[1] = io ? ux : mx;
+  tr[2] = io ? uy : my;
   const Quotient<R> over_rho(rho);
   if (!io) {
     ux = over_rho(mx);
@@ -206,13 +256,14 @@ __device__ __forceinline__ void march_cell(const Params& p, uint8_t fl, uint32_t
   }
   R fi[9], fe[9];
   bool forced = false;
-  if (MODEL == kMarchForced || MODEL == kMarchGeneral) {
-    const bool brinkman = MODEL == kMarchGeneral && p.alpha && !io;
-    forced = apply_force<R>(p, MODEL == kMarchForced || p.use_force != 0, brinkman,
-                            brinkman ? R(at(p.alpha, n)) : R(0), rho, over_rho, ux, uy, fi, unit);
+  if (MODEL != kMarchPlain && MODEL != kMarchUnforced) {
+    const bool brinkman = MODEL != kMarchForced && p.alpha && !io;
+    if (MODEL == kMarchGeneral && brinkman) alpha = at(p.alpha, n);
+    forced = apply_force<R>(p, MODEL == kMarchForced || p.use_force != 0, brinkman, R(alpha), rho,
+                            over_rho, ux, uy, fi, unit);
   }
   equilibrium_shifted<R>(rho, rho1, ux, uy, fe, unit);
-  const bool any = MODEL >= kMarchUnforced;
+  const bool any = MODEL == kMarchUnforced || MODEL == kMarchGeneral;
   relax<R>(p, any ? p.collision : 0, any && p.smagorinsky != 0, io != 0, forced, over_rho, fe,
            fi, g, unit);
 }
@@ -221,7 +272,7 @@ struct Fill { static constexpr bool value = false; };
 struct Steady { static constexpr bool value = true; };
 
 // The pass over one chunk of one strip: rows [ya, yb).
-template <class S, int T, int MODEL, bool IO>
+template <class S, int T, int MODEL, bool IO, bool TRACE = false>
 __device__ __forceinline__ void march_rows(const Params& p, const March& a, uint32_t strip,
                                            uint32_t ya, uint32_t yb) {
   static_assert(T >= 2 && T <= 4, "a lane keeps the flags of the T rows in one word");
@@ -245,6 +296,7 @@ __device__ __forceinline__ void march_rows(const Params& p, const March& a, uint
 
   E raw[9];
   uint8_t raw_fl;
+  float raw_alpha = 0.0f;
   IoValues<R> raw_io{};
   auto load_row = [&](uint32_t y) {
     const uint64_t rc = uint64_t(y) * pitch, ru = uint64_t(up(y)) * pitch,
@@ -261,6 +313,7 @@ __device__ __forceinline__ void march_rows(const Params& p, const March& a, uint
     raw[7] = at(here(7) + rc, x);
     raw[8] = at(there(7) + rd, xr);
     raw_fl = at(p.flags + rc, x);
+    if (MODEL == kMarchDrag && p.alpha) raw_alpha = at(p.alpha + rc, x);
     if (IO) {  // the neighbours' too: the end lanes have none to take them from
       const R* const r = fld<R>(const_cast<float*>(a.pub_rho_in)) + rc;
       const R* const u = fld<R>(const_cast<float*>(a.pub_u_in)) + rc;
@@ -300,6 +353,7 @@ __device__ __forceinline__ void march_rows(const Params& p, const March& a, uint
     pr[s] = pu[s] = pv[s] = R(0);
   }
   uint32_t fls = 0;  // flags of the rows of steps 1 .. T, a byte each
+  float alpha[T] = {};  // solid fractions of these rows (kMarchDrag)
 
   uint32_t y1 = ya >= uint32_t(H) ? ya - H : ya + ny - H;  // row of step 1 (ny >= T)
   load_row(y1);
@@ -309,6 +363,11 @@ __device__ __forceinline__ void march_rows(const Params& p, const March& a, uint
 #pragma unroll
     for (int i = 0; i < 9; i++) g[i] = Held<S>::in(raw[i]);
     fls = fls << 8 | raw_fl;
+    if (MODEL == kMarchDrag) {
+#pragma unroll
+      for (int s = T - 1; s > 0; s--) alpha[s] = alpha[s - 1];
+      alpha[0] = raw_alpha;
+    }
     const IoValues<R> io_now = raw_io;
     const uint32_t y = y1;
     y1 = up(y1);
@@ -330,8 +389,21 @@ __device__ __forceinline__ void march_rows(const Params& p, const March& a, uint
             v.uy_prev = from_left(v.uy);
           }
         }
-        march_cell<S, MODEL, IO>(p, fl, n, v, g, rho, ux, uy);
+        R tr[3];
+        march_cell<S, MODEL, IO>(p, fl, n, alpha[s - 1], v, g, rho, ux, uy, tr);
         const bool solid = fl & (kGas | kWall);
+        // The row is in the chunk (the halo rows are another wavefront's).
+        if (TRACE && it - uint32_t(H + s - 1) < yb - ya && own) {
+          if (!solid && a.trace) {
+            R* const to = static_cast<R*>(a.trace) + uint64_t(s - 1) * 3u * p.N;
+            at(to, n) = tr[0];
+            at(to + p.N, n) = tr[1];
+            at(to + 2 * p.N, n) = tr[2];
+          }
+          if ((a.window >> (s - 1) & 1u) && x == a.column)
+            a.discharge[uint64_t(s - 1) * ny + ys] =
+                solid ? 0.0 : double(rho) * double(IO && (fl & kInlet) ? tr[1] : ux);
+        }
         if (s < T) {
           Held<S>::round(g);
         } else {
