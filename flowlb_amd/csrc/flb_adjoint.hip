@@ -4,7 +4,7 @@
 // column with respect to the Brinkman solid fraction and the inlet velocity.
 // No reference counterpart: FlowLB has no adjoint.
 //
-// Reverse of one step, per cell and in place: the forward step of a cell
+// Reverse of one step, per cell and, where steps go singly, in place: the forward step of a cell
 // loads nine slots and stores nine results into the same slot set (esoteric
 // pull), so the adjoint kernel reads the adjoints of the stored results from
 // the store slots and writes the adjoints of the loaded populations to the
@@ -19,7 +19,8 @@
 // checkpoint of the populations and the inlet/outlet publication buffers every
 // `ckpt` steps and are recomputed, with their trace, during the reverse sweep.
 // The adjoint state (9 population planes, the adjoints of the published
-// inlet/outlet values) and its arithmetic are FP64: over 2000 reverse steps an
+// inlet/outlet values; the planes twice where the reverse steps go in passes)
+// and its arithmetic are FP64: over 2000 reverse steps an
 // FP32 adjoint lost about 2e-4 (relative) on cells with small gradients.  The
 // trace is what the forward computed: FP32 for an FP32 handle, FP64 for an
 // FP64 handle (FP64 forward and trace: the gradient of the FP64 discrete
@@ -29,6 +30,7 @@
 
 #include "flb_cell.h"
 #include "flb_internal.h"
+#include "flb_march.h"
 
 namespace flb {
 
@@ -64,6 +66,7 @@ struct Moments {
 };
 template <class T>
 __device__ __forceinline__ Moments moments(const double* v) {
+#pragma clang fp contract(on)
   const double w0 = double(wgt_r<T>(0)), w1 = double(wgt_r<T>(1)), w5 = double(wgt_r<T>(5));
   const double h = v[1] + v[2], k = v[3] + v[4], p = v[5] + v[6], m = v[7] + v[8];
   const double d = p + m;
@@ -80,6 +83,7 @@ __device__ __forceinline__ Moments moments(const double* v) {
 // Adjoint of feq(rho, u) from the moments of the adjoints of its nine values.
 __device__ __forceinline__ void feq_adjoint(const Moments& m, double rho, double ux, double uy,
                                             double& rb, double& ubx, double& uby) {
+#pragma clang fp contract(on)
   const double qx = ux * m.xx + uy * m.xy, qy = ux * m.xy + uy * m.yy;
   rb = m.s * (1.0 - 1.5 * (ux * ux + uy * uy)) + 3.0 * (ux * m.x + uy * m.y) +
        4.5 * (ux * qx + uy * qy);
@@ -87,21 +91,33 @@ __device__ __forceinline__ void feq_adjoint(const Moments& m, double rho, double
   uby = rho * (3.0 * (m.y - uy * m.s) + 9.0 * qy);
 }
 
+// 1 / v for a density or 1 + alpha / 2, to the last place: the hardware's estimate
+// and two Newton steps, half the instructions of a division, which also scales
+// operands near the ends of the range.
+__device__ __forceinline__ double reciprocal(double v) {
+  double r = __builtin_amdgcn_rcp(v);
+  r = fma(r, fma(-v, r, 1.0), r);
+  return fma(r, fma(-v, r, 1.0), r);
+}
+__device__ __forceinline__ double drag_scale(double al) { return reciprocal(fma(0.5, al, 1.0)); }
+
 // Reverse of one cell's step.  v: adjoints of the populations it emitted;
 // rb, ubx, uby: adjoints of its density and velocity as published (0 where none);
-// t0, t1, t2: its trace.  gb: adjoints of the populations it received; ab: of
-// its solid fraction.  For an inlet or outlet cell (io) gb is zero and rb, ubx,
+// al: its solid fraction, sa = drag_scale(al); t0, t1, t2: its trace.  gb:
+// adjoints of the populations it received; ab: of its solid fraction.  For an inlet or outlet cell (io) gb is zero and rb, ubx,
 // uby become the adjoints of the density and velocity it read.  `in_window`:
-// the objective takes the discharge here at this step.
+// the objective takes the discharge here at this step.  Contractions are the
+// source's, not the optimiser's: the single step and the passes agree bit for bit.
 template <class T>
-__device__ __forceinline__ void adjoint_cell(const Params& p, bool io, double al, double t0,
-                                             double t1, double t2, bool in_window, double qbar,
-                                             const double* v, double* gb, double& rb, double& ubx,
-                                             double& uby, double& ab) {
+__device__ __forceinline__ void adjoint_cell(const Params& p, bool io, double al, double sa,
+                                             double t0, double t1, double t2, bool in_window,
+                                             double qbar, const double* v, double* gb, double& rb,
+                                             double& ubx, double& uby, double& ab) {
+#pragma clang fp contract(on)
   const double Fx = p.use_force ? p.fx : 0.0f, Fy = p.use_force ? p.fy : 0.0f;
   const Moments m = moments<T>(v);
   double r, x, y;
-  const double rho = t0, inv = 1.0 / rho;
+  const double rho = t0, inv = reciprocal(rho);
   if (io) {
     // populations = feq(rho, u_read + F/(2 rho)): no dependence on the loaded ones
     const double ux = t1 + 0.5 * inv * Fx, uy = t2 + 0.5 * inv * Fy;
@@ -114,7 +130,7 @@ __device__ __forceinline__ void adjoint_cell(const Params& p, bool io, double al
     ab = 0.0;
     return;
   }
-  const double sa = 1.0 / (1.0 + 0.5 * al), si = sa * inv;
+  const double si = sa * inv;
   const double ux = (t1 + 0.5 * Fx) * si, uy = (t2 + 0.5 * Fy) * si;
   // The forward's SRT weights are float constants (also in FP64).
   const double om = p.inv_tau, omc = 1.0f - p.inv_tau, tl = 1.0f - 0.5f * p.inv_tau;
@@ -225,7 +241,8 @@ __global__ void __launch_bounds__(256) k_adjoint_step(const Params p, const AdjP
       const T* const tr = static_cast<const T*>(a.trace);
       const uint8_t io = fl & (kInlet | kOutlet);
       double gb[9], ab;
-      adjoint_cell<T>(p, io != 0, p.alpha ? p.alpha[n] : 0.0f, tr[n], tr[N + n], tr[2 * N + n],
+      const double al = p.alpha ? p.alpha[n] : 0.0f;
+      adjoint_cell<T>(p, io != 0, al, drag_scale(al), tr[n], tr[N + n], tr[2 * N + n],
                       a.in_window && x == a.column, a.qbar, v, gb, rb, ubx, uby, ab);
       if (io & kInlet) {
         a.rbar[ODD ^ 1][lin.next] += rb;
@@ -241,6 +258,234 @@ __global__ void __launch_bounds__(256) k_adjoint_step(const Params p, const AdjP
     }
   }
   block_add(duin, a.duin);
+}
+
+// Reverse of K steps, from the one at time t down to t - K + 1, in one pass over
+// the adjoint state: the forward pass (march_rows) mirrored.  A wavefront owns
+// 64 - 2 (K - 1) columns of a strip and marches up its chunk of rows; the reverse
+// of step t - s takes the row below that of step t - s + 1.  Since a population i
+// that cell n emits is received at n + c_i, the adjoint cell n needs is the one
+// of the cell it sent to: those above come from the row just done, those
+// beside from one iteration ago, those below from two.  A wall, which emits what
+// it received in the opposite direction, exchanges the adjoints.  A single step
+// moves 196 bytes per cell, 144 of them the adjoint populations, which a pass of
+// three moves once; 1024 x 256, FP32: 10.2 us per step one by one, 5.9 in passes
+// (140 FP64 instructions of about 200 per step-row, halo rows included: the
+// vector units bind, except on grids beyond the caches).
+struct AdjMarch {
+  const double* in;   // adjoint populations after step t
+  double* out;        // before step t - K + 1
+  // Adjoints of the densities and velocities published at step t, and those
+  // at step t - K.  Cells no inlet or outlet reads hold zero.
+  const double* rb_in;
+  const double* ub_in;
+  double* rb_out;
+  double* ub_out;
+  double* galpha;
+  double* duin;
+  const void* trace;  // of step t; that of step t - s is 3 s N values before it
+  int32_t odd;        // t % 2
+  uint32_t column, window;  // bit s of window: step t - s is averaged
+  double qbar;
+  MarchGrid grid;
+};
+
+template <class T, int K, bool IO>
+__device__ __forceinline__ void adjoint_rows(const Params& p, const AdjMarch& a, uint32_t strip,
+                                             uint32_t ya, uint32_t yb) {
+  constexpr int H = K - 1;  // halo
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t nx = p.nx, ny = p.ny, pitch = p.pitch;
+  const uint32_t xs = strip * march_columns(K) + lane;  // column + H
+  const bool own = lane >= H && lane < 64 - H && xs - H < nx;
+  const uint32_t x = (xs + H * (nx - 1)) % nx;
+  const uint32_t xr = x + 1 == nx ? 0u : x + 1;
+  const bool odd = a.odd != 0, odd_last = odd != ((K & 1) == 0);
+  const uint64_t Np = p.Np;
+  auto up = [&](uint32_t y) { return y + 1 == ny ? 0u : y + 1; };
+  auto down = [&](uint32_t y) { return y == 0 ? ny - 1 : y - 1; };
+
+  double raw[9], raw_ga = 0.0, raw_rb = 0.0, raw_ub = 0.0, raw_vb = 0.0;
+  T raw_tr[K][3];
+  uint8_t raw_fl;
+  float raw_al = 0.0f;
+  auto load_row = [&](uint32_t y) {
+    const uint64_t rc = uint64_t(y) * pitch, ru = uint64_t(up(y)) * pitch,
+                   rd = uint64_t(down(y)) * pitch;
+    auto here = [&](int i) { return a.in + (odd ? i : i + 1) * Np; };
+    auto there = [&](int i) { return a.in + (odd ? i + 1 : i) * Np; };
+    raw[0] = at(a.in + rc, x);
+    raw[1] = at(there(1) + rc, xr);
+    raw[2] = at(here(1) + rc, x);
+    raw[3] = at(there(3) + ru, x);
+    raw[4] = at(here(3) + rc, x);
+    raw[5] = at(there(5) + ru, xr);
+    raw[6] = at(here(5) + rc, x);
+    raw[7] = at(there(7) + rd, xr);
+    raw[8] = at(here(7) + rc, x);
+    raw_fl = at(p.flags + rc, x);
+    if (p.alpha) raw_al = at(p.alpha + rc, x);
+    if (a.galpha) raw_ga = at(a.galpha + rc, x);
+    if (IO) {
+      raw_rb = at(a.rb_in + rc, x);
+      raw_ub = at(a.ub_in + rc, x);
+      raw_vb = at(a.ub_in + p.N + rc, x);
+    }
+    uint32_t ys = y;  // each step's row of the next iteration
+#pragma unroll
+    for (int s = 0; s < K; s++) {
+      const T* const tr = static_cast<const T*>(a.trace) - uint64_t(s) * 3u * p.N +
+                          uint64_t(ys) * pitch;
+#pragma unroll
+      for (int k = 0; k < 3; k++) raw_tr[s][k] = at(tr + k * p.N, x);
+      ys = down(ys);
+    }
+  };
+  auto store_row = [&](uint32_t y, const double* g) {
+    const uint64_t rc = uint64_t(y) * pitch, ru = uint64_t(up(y)) * pitch,
+                   rd = uint64_t(down(y)) * pitch;
+    auto here = [&](int i) { return a.out + (odd_last ? i : i + 1) * Np; };
+    auto there = [&](int i) { return a.out + (odd_last ? i + 1 : i) * Np; };
+    at(a.out + rc, x) = g[0];
+    at(here(1) + rc, x) = g[1];
+    at(there(1) + rc, xr) = g[2];
+    at(here(3) + rc, x) = g[3];
+    at(there(3) + ru, x) = g[4];
+    at(here(5) + rc, x) = g[5];
+    at(there(5) + ru, xr) = g[6];
+    at(here(7) + rc, x) = g[7];
+    at(there(7) + rd, xr) = g[8];
+  };
+
+  // Between two steps (index of the first), already shifted to the lane that
+  // takes them: 0, 1, 2 of the row the second takes next; 4, 6, 7 of that row
+  // and of the one below it; the published values' adjoints of that row (IO).
+  double flat[H][3] = {}, fall0[H][3] = {}, fall1[H][3] = {};
+  double pr[H] = {}, pu[H] = {}, pv[H] = {};
+  uint32_t fls = 0;
+  float al[K] = {};  // solid fractions of the rows under way
+  double sa[K] = {};  // drag_scale of them
+  double ga[K] = {};  // dJ/dalpha
+  double duin = 0.0;
+
+  uint32_t y1 = ya >= uint32_t(H) ? ya - H : ya + ny - H;
+  load_row(y1);
+  const uint32_t iterations = yb - ya + 2 * H;
+  const auto iterate = [&](uint32_t it, auto steady) {
+    double g[9];
+#pragma unroll
+    for (int i = 0; i < 9; i++) g[i] = raw[i];
+    fls = fls << 8 | raw_fl;
+#pragma unroll
+    for (int s = K - 1; s > 0; s--) {
+      al[s] = al[s - 1];
+      sa[s] = sa[s - 1];
+      ga[s] = ga[s - 1];
+    }
+    al[0] = raw_al;
+    sa[0] = drag_scale(raw_al);
+    ga[0] = raw_ga;
+    double rb = raw_rb, ubx = raw_ub, uby = raw_vb;
+    T tr[K][3];
+#pragma unroll
+    for (int s = 0; s < K; s++)
+#pragma unroll
+      for (int k = 0; k < 3; k++) tr[s][k] = raw_tr[s][k];
+    uint32_t ys = y1;
+    y1 = up(y1);
+    load_row(y1);  // one row past the last is loaded and not used
+#pragma unroll
+    for (int s = 0; s < K; s++) {
+      if (decltype(steady)::value || it >= 2u * uint32_t(s)) {
+        const uint8_t fl = uint8_t(fls >> (8 * s));
+        const bool solid = fl & (kGas | kWall);
+        const uint8_t io = IO ? fl & (kInlet | kOutlet) : 0;
+        if (solid) {
+#pragma unroll
+          for (int i = 1; i < 9; i += 2) {
+            const double t = g[i];
+            g[i] = g[i + 1];
+            g[i + 1] = t;
+          }
+        } else {
+          if (!IO) rb = ubx = uby = 0.0;
+          if (IO && (fl & kInlet)) ubx = uby = 0.0;
+          double gb[9], ab;
+          adjoint_cell<T>(p, io != 0, al[s], sa[s], tr[s][0], tr[s][1], tr[s][2],
+                          (a.window >> s & 1u) && x == a.column, a.qbar, g, gb, rb, ubx, uby, ab);
+#pragma unroll
+          for (int i = 0; i < 9; i++) g[i] = gb[i];
+          if (!io) ga[s] += ab;
+        }
+        const bool inlet = IO && !solid && (fl & kInlet);
+        const bool outlet = IO && !solid && !inlet && (fl & kOutlet);
+        // The row is in the chunk (the halo rows are another wavefront's).
+        if (inlet && own && it - uint32_t(H + s) < yb - ya) duin += ubx;
+        if (s < K - 1) {
+          constexpr int last = K > 1 ? H - 1 : 0;
+          const int b = s < last ? s : last;
+          double v[9];
+          v[0] = flat[b][0];
+          v[1] = flat[b][1];
+          v[2] = flat[b][2];
+          v[4] = fall1[b][0];
+          v[6] = fall1[b][1];
+          v[7] = fall1[b][2];
+          v[3] = g[3];
+          v[5] = from_right(g[5]);
+          v[8] = from_left(g[8]);
+          flat[b][0] = g[0];
+          flat[b][1] = from_right(g[1]);
+          flat[b][2] = from_left(g[2]);
+#pragma unroll
+          for (int k = 0; k < 3; k++) fall1[b][k] = fall0[b][k];
+          fall0[b][0] = g[4];
+          fall0[b][1] = from_left(g[6]);
+          fall0[b][2] = from_right(g[7]);
+          if (IO) {
+            const double r = from_left(inlet ? rb : 0.0);
+            const double q = from_right(outlet ? ubx : 0.0), w = from_right(outlet ? uby : 0.0);
+            rb = pr[b];
+            ubx = pu[b];
+            uby = pv[b];
+            pr[b] = r;
+            pu[b] = q;
+            pv[b] = w;
+          }
+#pragma unroll
+          for (int i = 0; i < 9; i++) g[i] = v[i];
+          ys = down(ys);
+        } else if (own) {
+          const uint64_t rc = uint64_t(ys) * pitch;
+          store_row(ys, g);
+          if (a.galpha && !solid && !io) at(a.galpha + rc, x) = ga[s];
+          if (inlet) at(a.rb_out + rc, x + 1) = rb;
+          if (outlet) {
+            at(a.ub_out + rc, x - 1) = ubx;
+            at(a.ub_out + p.N + rc, x - 1) = uby;
+          }
+        }
+      }
+    }
+    if (!IO) __builtin_amdgcn_s_barrier();  // a block's strips keep to the same row
+  };
+  for (uint32_t it = 0; it < 2 * H; ++it) iterate(it, Fill{});
+#pragma unroll 2
+  for (uint32_t it = 2 * H; it < iterations; ++it) iterate(it, Steady{});
+  if (IO) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) duin += __shfl_down(duin, o, 64);
+    if (lane == 0 && duin != 0.0) atomicAdd(a.duin, duin);
+  }
+}
+
+template <class T, int K>
+__global__ void __launch_bounds__(64 * kMarchWaves) __attribute__((amdgpu_waves_per_eu(2)))
+k_adjoint_march(const Params p, const AdjMarch a) {
+  const MarchWork w = march_work(a.grid, p.ny);
+  if (w.ya >= w.yb) return;
+  if (w.io) adjoint_rows<T, K, true>(p, a, w.strip, w.ya, w.yb);
+  else adjoint_rows<T, K, false>(p, a, w.strip, w.ya, w.yb);
 }
 
 // The initial populations of inlet cells, feq(rho0, u0) stored with the odd
@@ -386,6 +631,12 @@ int check_adjoint_state(flb_handle* h, const flb_adjoint_spec* sp) {
 
 using flb::kDischargeSteps;
 
+using AdjMarchFn = void (*)(const flb::Params, const flb::AdjMarch);
+AdjMarchFn adjoint_march(bool fp64, int steps) {
+  if (fp64) return steps == 2 ? flb::k_adjoint_march<double, 2> : flb::k_adjoint_march<double, 3>;
+  return steps == 2 ? flb::k_adjoint_march<float, 2> : flb::k_adjoint_march<float, 3>;
+}
+
 // Forward steps [t, t+count) with the objective accumulated into d_j; with a
 // trace buffer, step t + k records its trace at trace + k * 3 N values.  In
 // passes of several steps where the handle has them: the averaged steps record
@@ -525,7 +776,7 @@ int flb_adjoint(flb_handle* h, const flb_adjoint_spec* sp, double* J, float* dj_
   using W = flb::Workspace;
   TrimWork trim{h};
   uint8_t *ckpt = nullptr, *fields0 = nullptr, *trace_res = nullptr, *trace_tmp = nullptr;
-  double *abar = nullptr, *rbar = nullptr, *ubar = nullptr, *galpha = nullptr, *d_acc = nullptr;
+  double *abar = nullptr, *abar_alt = nullptr, *rbar = nullptr, *ubar = nullptr, *galpha = nullptr, *d_acc = nullptr;
   auto buffers = [&]() {
     flb::Workspace& w = h->work;
     return (!first_res || ((ckpt = w.get<uint8_t>(W::kCheckpoints, first_res * ck_bytes)) &&
@@ -543,6 +794,10 @@ int flb_adjoint(flb_handle* h, const flb_adjoint_spec* sp, double* J, float* dj_
     if (!buffers())
       return flb::set_error(h, FLB_ERR_MEMORY, "adjoint buffers (checkpoints, trace, adjoint state)");
   }
+  // Passes need a second adjoint state; without room for it, single steps.
+  flb::MarchShape shape = flb::adjoint_shape(h);
+  if (std::min(K, T) < 2 || !h->f_alt) shape.steps = 0;
+  if (shape.steps && !(abar_alt = h->work.get<double>(W::kAdjointAlt, 9 * Np))) shape.steps = 0;
   auto seg_trace = [&](uint64_t s) {
     return s >= first_res ? trace_res + (s - first_res) * seg_bytes : trace_tmp;
   };
@@ -574,6 +829,8 @@ int flb_adjoint(flb_handle* h, const flb_adjoint_spec* sp, double* J, float* dj_
   if (galpha) ADJ_HIP(h, hipMemsetAsync(galpha, 0, N * sizeof(double), h->stream));
   const int abx = 256;
   float recompute_ms = 0.0f;
+  double *rb[2] = {rbar, rbar + N}, *ub[2] = {ubar, ubar + 2 * N};  // by parity
+  bool stale = false;  // the other parity's hold values a pass has used
   for (uint64_t s = nseg; s-- > 0 && !rc;) {
     const uint64_t ts = s * K, te = std::min(ts + K, T);
     uint8_t* trace = seg_trace(s);
@@ -585,15 +842,55 @@ int flb_adjoint(flb_handle* h, const flb_adjoint_spec* sp, double* J, float* dj_
       ADJ_HIP(h, hipEventRecord(ev[3], h->stream));
     }
     for (uint64_t t = te; t-- > ts;) {
+      const uint8_t* const tr = trace + (t - ts) * 3 * N * h->field_bytes;
       flb::Params p = flb::make_params(h, abx);
+      const int steps = shape.steps ? flb::march_steps_next(t + 1 - ts, shape.steps) : 0;
+      if (steps) {
+        const int par = int(t & 1), to = par ^ (steps & 1);
+        // Published values' adjoints go to the parity of the step below the pass;
+        // an even pass would write what it reads, so the buffers change places.
+        if (!(steps & 1)) {
+          std::swap(rb[0], rb[1]);
+          std::swap(ub[0], ub[1]);
+        }
+        flb::AdjMarch a{};
+        a.in = abar;
+        a.out = abar_alt;
+        a.rb_in = rb[steps & 1 ? par : par ^ 1];
+        a.ub_in = ub[steps & 1 ? par : par ^ 1];
+        a.rb_out = rb[to];
+        a.ub_out = ub[to];
+        a.galpha = galpha;
+        a.duin = d_acc + 1;
+        a.trace = tr;
+        a.odd = par;
+        a.column = sp->column;
+        for (int k = 0; k < steps; ++k)
+          if (t - k >= sp->t0 && t - k <= sp->t1) a.window |= 1u << k;
+        a.qbar = qs;
+        a.grid = flb::march_grid(h, steps, shape.rows, (shape.rows + 1) / 2);
+        hipLaunchKernelGGL(adjoint_march(fp64, steps), dim3(a.grid.blocks),
+                           dim3(64 * flb::kMarchWaves), 0, h->stream, p, a);
+        ADJ_HIP(h, hipGetLastError());
+        std::swap(abar, abar_alt);
+        stale = true;
+        t -= uint64_t(steps - 1);
+        continue;
+      }
+      if (stale) {  // a single step adds to what it publishes for the step below
+        const int to = int(t & 1) ^ 1;
+        ADJ_HIP(h, hipMemsetAsync(rb[to], 0, N * sizeof(double), h->stream));
+        ADJ_HIP(h, hipMemsetAsync(ub[to], 0, 2 * N * sizeof(double), h->stream));
+        stale = false;
+      }
       flb::AdjParams a{};
       a.abar = abar;
-      a.rbar[0] = rbar;
-      a.rbar[1] = rbar + N;
-      a.ubar[0] = ubar;
-      a.ubar[1] = ubar + 2 * N;
+      for (int k = 0; k < 2; ++k) {
+        a.rbar[k] = rb[k];
+        a.ubar[k] = ub[k];
+      }
       a.galpha = galpha;
-      a.trace = trace + (t - ts) * 3 * N * h->field_bytes;
+      a.trace = tr;
       a.duin = d_acc + 1;
       a.column = sp->column;
       a.in_window = t >= sp->t0 && t <= sp->t1;

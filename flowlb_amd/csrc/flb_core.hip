@@ -778,7 +778,8 @@ static int enqueue_march(flb_handle* h, int T, bool moments, const flb::MarchTra
   a.pub_u_out = h->pub_u[last ^ 1];
   a.odd = int32_t(h->t & 1u);
   a.moments = moments;
-  a.grid = flb::march_grid(h, T);
+  const uint32_t rows = march_shape(h).rows;
+  a.grid = flb::march_grid(h, T, rows, (rows + flb::kMarchWaves - 1) / flb::kMarchWaves);
   if (trace) {
     a.trace = trace->trace;
     a.discharge = trace->discharge;
@@ -820,8 +821,10 @@ uint32_t march_strips(uint32_t nx, int steps, const std::vector<uint8_t>& io,
   for (uint32_t s = 0; s < order.size(); ++s) order[s] = s;
   const auto split = std::stable_partition(order.begin(), order.end(), [&](uint32_t s) {
     uint8_t any = 0;
-    for (uint32_t l = 0; l < kMarchLanes; ++l)
-      any |= io[(uint64_t(s) * cols + l + uint64_t(steps - 1) * (nx - 1)) % nx];
+    // One column more on each side: the reverse pass (adjoint) takes values an
+    // inlet or outlet beside the first or last lane's cell hands it.
+    for (uint32_t l = 0; l < kMarchLanes + 2; ++l)
+      any |= io[(uint64_t(s) * cols + l + uint64_t(steps) * (nx - 1)) % nx];
     return any != 0;
   });
   return uint32_t(split - order.begin());
@@ -991,20 +994,39 @@ int enqueue_march_ex(flb_handle* h, int T, bool moments, const MarchTrace* trace
   return enqueue_march(h, T, moments, trace);
 }
 int march_most(const flb_handle* h) { return h->f_alt ? ::march_shape(h).steps : 0; }
-MarchGrid march_grid(const flb_handle* h, int T) {
+MarchGrid march_grid(const flb_handle* h, int T, uint32_t rows, uint32_t io_rows) {
   const uint32_t cols = march_columns(T);
   constexpr uint32_t G = kMarchWaves;
   MarchGrid g{};
   g.strips = (h->nx + cols - 1) / cols;
   g.io_strips = h->march_io[T];
   g.order = h->march_order[T];
-  g.rows = ::march_shape(h).rows;
+  g.rows = rows;
   g.chunks = (h->ny + g.rows - 1) / g.rows;
-  g.io_rows = (g.rows + G - 1) / G;
+  g.io_rows = io_rows;
+  g.io_chunks = (h->ny + g.io_rows * G - 1) / (g.io_rows * G);
   g.groups = (g.strips - g.io_strips + G - 1) / G;
   g.group_magic = div_magic(g.groups);
-  g.blocks = g.io_strips * g.chunks + (g.groups * g.chunks + 7u) / 8u * 8u;
+  g.blocks = g.io_strips * g.io_chunks + (g.groups * g.chunks + 7u) / 8u * 8u;
   return g;
+}
+// A reverse pass is bound by its FP64 instructions, about 6 cycles each with one
+// wavefront on a SIMD and no less with two, so its time is the longest SIMD's.
+// Blocks that share a CU then cost more than longer chunks, as long as the grid
+// is small: of the chunks of up to 8 rows, the shortest whose blocks take a CU
+// each.  1024 x 256, us per step in reverse, 3 steps: 7.7, 5.9, 6.3, 7.2 with 4, 5,
+// 6, 8 rows (320, 252, 216, 160 blocks; single steps 10.2).  Larger grids are bound by
+// memory and want the wavefronts: 2048 x 512 19.7, 17.5, 20.4 with 8, 12, 16
+// rows (single steps 35.6).  Where two or three rows do, a pass of 2 steps has
+// the shorter chain: 256 x 64 3.4, against 4.0 with 3 steps (single steps 5.4).
+MarchShape adjoint_shape(const flb_handle* h) {
+  for (uint32_t r = 2; r <= 8; ++r) {
+    const MarchShape s{r < 4 ? 2 : 3, r};
+    if (march_grid(h, s.steps, r, (r + 1) / 2).blocks <= uint32_t(h->cus)) return s;
+  }
+  const uint64_t waves = uint64_t(h->cus) * 6;  // 1.5 per SIMD
+  const uint64_t rows = (march_grid(h, 3, 1, 1).strips * uint64_t(h->ny) + waves - 1) / waves;
+  return MarchShape{3, uint32_t(std::min<uint64_t>(std::max<uint64_t>(rows, 5), 16))};
 }
 int copy_cells_in(flb_handle* h, void* dev, const void* host, size_t elem, int planes) {
   return cells_in(h, dev, host, elem, planes);

@@ -236,7 +236,8 @@ struct MarchTrace {
   uint32_t column, window;
 };
 int enqueue_march_ex(flb_handle* h, int T, bool moments, const MarchTrace* trace);
-MarchGrid march_grid(const flb_handle* h, int T);
+MarchGrid march_grid(const flb_handle* h, int T, uint32_t rows, uint32_t io_rows);
+MarchShape adjoint_shape(const flb_handle* h);  // of the adjoint's passes
 int march_most(const flb_handle* h);  // steps per pass of a long run, 0: no passes
 // Copies `planes` planes of cells of `elem` bytes between a host array
 // (planes of nx * ny, row-major) and a pitched device array (planes of Nd),

@@ -37,8 +37,8 @@ constexpr uint32_t kMarchLanes = 64;
 constexpr int kMarchWaves = 4;  // wavefronts per block
 constexpr uint32_t march_columns(int steps) { return kMarchLanes - 2u * uint32_t(steps - 1); }
 
-// Blocks of a pass over a single domain.  The first io_strips * chunks blocks take
-// a chunk of an inlet/outlet strip each, split by rows between their wavefronts
+// Blocks of a pass over a single domain.  The first io_strips * io_chunks blocks
+// take rows of an inlet/outlet strip each, io_rows for each of their wavefronts
 // (such a strip costs two to three times the others: with whole chunks these
 // wavefronts ended last, alone).  The others take a chunk of kMarchWaves adjacent
 // strips, which stay within a row of each other (a barrier per row), so that
@@ -48,7 +48,8 @@ struct MarchGrid {
   uint32_t strips, io_strips;  // strips, and those whose 64 columns hold an inlet or outlet cell
   uint32_t chunks;             // chunks of rows
   uint32_t rows;               // rows per chunk
-  uint32_t io_rows;            // rows a wavefront takes of a chunk of such a strip
+  uint32_t io_chunks;          // blocks per inlet/outlet strip
+  uint32_t io_rows;            // rows a wavefront takes of such a strip
   uint32_t groups, group_magic;  // blocks per chunk of the other strips, div_magic of it
   uint32_t blocks;
   const uint32_t* order;       // strips, the io_strips ones first
@@ -59,14 +60,14 @@ struct MarchWork {
 };
 __device__ __forceinline__ MarchWork march_work(const MarchGrid& g, uint32_t ny) {
   const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(threadIdx.x / 64u));
-  const uint32_t io_blocks = g.io_strips * g.chunks;
+  const uint32_t io_blocks = g.io_strips * g.io_chunks;
   MarchWork w{};
   if (blockIdx.x < io_blocks) {
     const uint32_t chunk = blockIdx.x / g.io_strips;
     w.io = true;
     w.strip = g.order[blockIdx.x - chunk * g.io_strips];
-    w.ya = chunk * g.rows + wave * g.io_rows;
-    w.yb = min(w.ya + g.io_rows, min((chunk + 1u) * g.rows, ny));
+    w.ya = (chunk * uint32_t(kMarchWaves) + wave) * g.io_rows;
+    w.yb = min(w.ya + g.io_rows, ny);
     return w;
   }
   const uint32_t b = blockIdx.x - io_blocks, per = (gridDim.x - io_blocks) / 8u;
