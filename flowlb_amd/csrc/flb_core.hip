@@ -525,7 +525,7 @@ int flb_create(const flb_options* opt, const uint8_t* flags, uint32_t nx, uint32
     }
     {
       void* hb = nullptr;
-      if (hipHostMalloc(&hb, 2 * sizeof(unsigned long long),
+      if (hipHostMalloc(&hb, 3 * sizeof(unsigned long long),
                         hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
         (void)hipGetLastError();
         return bail(FLB_ERR_MEMORY);
@@ -699,6 +699,37 @@ void stream_collide_window(const flb_handle* h, flb::Params& p, int bx) {
   flb::set_walk(p, uint32_t(rows), p.ncols);
 }
 
+// Grids of the free-surface kernels that walk a list: its published length and
+// a quarter more (the surface grows), or the most blocks if none is known.
+// chunks: blocks of four wavefronts, one chunk each; pass1: every eighth block
+// classifies a tile per thread, the others take chunks; update: a block per tile
+// and one that publishes.
+struct ListGrids {
+  uint32_t chunks, pass1, update;
+};
+static ListGrids list_grids(const flb_handle* h) {
+  const uint32_t cus = uint32_t(h->cus), tiles = h->work_x * h->tile_rows;
+  uint64_t nt = tiles, nc = uint64_t(h->work_x) * h->ny;
+  if (h->box_host) {
+    const volatile unsigned long long* bh = h->box_host;
+    if (const unsigned long long s = bh[1]; s != ~0ull && s <= h->t) {
+      const unsigned long long n = bh[2];
+      nt = n & 0xffffffffu;
+      nc = n >> 32;
+    }
+  }
+  nt = std::min<uint64_t>(nt + nt / 4 + 2, tiles + 1);
+  nc = nc + nc / 4 + 2;
+  const uint64_t list = uint64_t(flb::kListBlocksPerCU) * cus;
+  constexpr uint64_t waves = flb::kListThreads / 64;
+  ListGrids g;
+  g.chunks = uint32_t(std::min(list, (nc + waves - 1) / waves));
+  g.pass1 = uint32_t(std::min(list, 8 * std::max<uint64_t>((tiles + flb::kListThreads - 1) / flb::kListThreads,
+                                                 (nc + 7 * waves - 1) / (7 * waves))));
+  g.update = uint32_t(std::min<uint64_t>(uint64_t(flb::kUpdateBlocksPerCU) * cus, nt));
+  return g;
+}
+
 // One lattice step on the handle's stream.  ev (optional) receives per-kernel
 // event pairs: ev[2k], ev[2k+1] around kernel k.
 static int enqueue_step(flb_handle* h, bool moments, hipEvent_t* ev) {
@@ -724,8 +755,9 @@ static int enqueue_step(flb_handle* h, bool moments, hipEvent_t* ev) {
     p.counts_out = h->counts + 4 * wr;
     p.tile_count = h->tile_counts + rd;
     p.tile_count_next = h->tile_counts + wr;
+    const ListGrids grids = list_grids(h);
     flb::Params q = p;  // pass 1: a grid of resident blocks walks the list
-    q.nblocks = uint32_t(flb::kListBlocksPerCU * h->cus);
+    q.nblocks = grids.pass1;
     if ((rc = run(FLB_K_FS1, flb::get_fs1(st, odd), q, flb::kListThreads))) return rc;
     if (h->opt.mass_mode != FLB_MASS_CONSERVATIVE) {
       if ((rc = run(FLB_K_STREAM_COLLIDE, flb::get_stream_collide(st, odd, true, moments), p, bx)))
@@ -746,13 +778,14 @@ static int enqueue_step(flb_handle* h, bool moments, hipEvent_t* ev) {
       if (ev) FLB_HIP(h, hipEventRecord(ev[2 * FLB_K_STREAM_COLLIDE], h->stream));
       if (w.nblocks && (rc = launch(h, flb::get_stream_collide_dense(st, odd, moments), w, bx)))
         return rc;
+      q.nblocks = grids.chunks;
       if ((rc = launch(h, flb::get_stream_collide_surface(st, odd, moments), q, flb::kListThreads)))
         return rc;
       if (ev) FLB_HIP(h, hipEventRecord(ev[2 * FLB_K_STREAM_COLLIDE + 1], h->stream));
     }
     q = p;  // passes 2-4: blocks of kFsTileW x kFsTileH threads walk the tile list
     q.tiles_x = h->work_x;
-    q.nblocks = uint32_t(flb::kUpdateBlocksPerCU * h->cus);
+    q.nblocks = grids.update;
     if ((rc = run(FLB_K_FS_UPDATE, flb::get_fs_update(st, odd, h->nx, h->ny), q,
                   flb::kFsTileW * flb::kFsTileH)))
       return rc;

@@ -581,8 +581,8 @@ __device__ __forceinline__ void update_tile(const Params& p, uint32_t tx, uint32
 }
 
 // One block of the update reduces the per-wavefront boxes pass 1 wrote this
-// step and sends the result to the host (mapped memory): first the box, then
-// -- after a system-scope fence, so that a host that reads the step and then
+// step and sends the result to the host (mapped memory), with the lengths of
+// this step's tile and chunk lists: first these, then -- after a system-scope fence, so that a host that reads the step and then
 // the box gets a box at least as new -- the step.  Every thread of the block
 // calls it.
 __device__ __forceinline__ void publish_box(const Params& p, uint32_t* red) {
@@ -621,6 +621,8 @@ __device__ __forceinline__ void publish_box(const Params& p, uint32_t* red) {
         (unsigned long long)(ylo & 0xffffu) | (unsigned long long)(yhi & 0xffffu) << 16 |
         (unsigned long long)(xlo & 0xffffu) << 32 | (unsigned long long)(xhi & 0xffffu) << 48;
     p.box_host[0] = packed;
+    p.box_host[2] = (unsigned long long)*p.tile_count |
+                    (unsigned long long)p.counts_in[kListFS1] << 32;
     __threadfence_system();
     p.box_host[1] = (unsigned long long)p.step;
   }
