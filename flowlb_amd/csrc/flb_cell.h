@@ -178,9 +178,10 @@ __device__ __forceinline__ Cell locate_window(const Params& p, uint32_t b = bloc
 // is one row segment that starts at a multiple of 64), so its tile word is a
 // scalar load.
 // Returns the work bits of the chunk (bit kWorkSC: stream-collide, bit
-// kWorkFS1: pass 1, kChunkBody: the tile is a body of fluid, Params::tile_body),
+// kWorkFS1: pass 1, kChunkBody: the tile is a body of fluid, Params::tile_body; kChunkFresh),
 // 0 for a wavefront past the row's end.
 constexpr uint32_t kChunkBody = 1u << 30;
+constexpr uint32_t kChunkFresh = 1u << 29;  // with kChunkBody: not a body in the last step
 __device__ __forceinline__ uint32_t chunk_work(const Params& p, const Cell& c, bool with_pub,
                                                bool with_body) {
   const uint32_t tx = uint32_t(__builtin_amdgcn_readfirstlane(c.x)) / kFsTileW;
@@ -190,7 +191,8 @@ __device__ __forceinline__ uint32_t chunk_work(const Params& p, const Cell& c, b
   const int r = int(y % kFsTileH);
   const uint32_t w = p.tile_work[i];
   const uint32_t sc = (w | (with_pub ? p.tile_pub[i] : 0u)) >> (kWorkSC + r);
-  const uint32_t body = with_body && p.tile_body[i] ? kChunkBody : 0u;
+  const uint32_t b = with_body ? p.tile_body[i] : kBodyNot;
+  const uint32_t body = b == kBodyNot ? 0u : (b == kBodyFresh ? kChunkBody | kChunkFresh : kChunkBody);
   return (sc & 1u) << kWorkSC | ((w >> (kWorkFS1 + r)) & 1u) << kWorkFS1 | body;
 }
 
@@ -472,12 +474,18 @@ __device__ __forceinline__ void relax(const Params& p, int collision, bool smago
 // bodies of fluid to fewer registers.
 // BODY (with DENSE): the cell's tile and its halo are plain fluid
 // (Params::tile_body) and the update kernel will not visit it, so the cell
-// also does the update's body-of-fluid step: mass = rho, its excess (the
-// deviation) shared by eight receivers into excess_out, flag kept.  Its flag
+// also does the update's body-of-fluid step: its excess (the deviation) shared by
+// eight receivers into excess_out.  Of the rest, mass = rho is read by no kernel
+// -- a cell takes its mass from its deviation in the first step that its tile is
+// not a body -- and stored at readback steps (MOM), and the flag is stored in the
+// tile's first step as a body (fresh), after which both buffers hold it: 5 of the
+// 90 (FP32) or 58 (16-bit) bytes a cell moved (8192 x 2048 dam break: 79.1 -> 76.0
+// us per step; 4096 x 1024 FP16S, bound by latency, as before).  Its flag
 // is known (plain fluid, no inlet/outlet neighbour role: such tiles are never
 // bodies), so the wavefront goes straight to the population loads.
 template <class S, int ODD, bool FS, bool MOM, bool TRACE, bool DENSE = false, bool BODY = false>
-__device__ __forceinline__ void stream_collide_cell(const Params& p, const Cell c) {
+__device__ __forceinline__ void stream_collide_cell(const Params& p, const Cell c,
+                                                    bool fresh = false) {
   constexpr bool body = DENSE && BODY;
   using R = typename S::R;
   R* const rho_f = fld<R>(p.rho);
@@ -625,9 +633,9 @@ __device__ __forceinline__ void stream_collide_cell(const Params& p, const Cell 
       dev = R(m);
     }
     if (body) {
-      at(fld<R>(p.mass), n) = rho;
+      if (MOM) at(fld<R>(p.mass), n) = rho;
       at(fld<R>(p.excess_out), n) = dev / R(8.0f);
-      p.flags_next[n] = fl;
+      if (fresh) p.flags_next[n] = fl;
     } else {
       at(fld<R>(p.mass), n) = dev;
     }

@@ -217,7 +217,7 @@ struct Params {
   uint32_t* tile_count;
   uint32_t* tile_count_next;
   // Per tile, written by pass 1: the tile and its three-cell halo are plain
-  // fluid, so stream-collide also does the update's work for its cells.
+  // fluid, so stream-collide also does the update's work for its cells (BodyKind).
   uint32_t* tile_body;
   // Free surface: bounding box, in tiles (row lo, row hi, column lo, column
   // hi), of the chunks with stream-collide work.  Pass 1 writes one box per
@@ -245,6 +245,9 @@ inline void set_relaxation(Params& p, float inv_tau) {
   p.tau = 1.0f / inv_tau;
   p.trt_minus = 1.0f / (0.25f / (p.tau - 0.5f) + 0.5f);
 }
+
+// Params::tile_body: no body of fluid, one since this step, one since an earlier step.
+enum BodyKind : uint32_t { kBodyNot = 0, kBodyFresh = 1, kBodyKept = 2 };
 
 enum : int { kListFS1 = 0 };
 constexpr int kListThreads = 256;  // block size of the list-driven pass 1

@@ -43,7 +43,7 @@ __global__ void __launch_bounds__(1024) k_stream_collide(const Params p) {
   }
   if (!c.valid) return;
   if (DENSE && (work & kChunkBody))
-    stream_collide_cell<S, ODD, FS, MOM, TRACE, DENSE, true>(p, c);
+    stream_collide_cell<S, ODD, FS, MOM, TRACE, DENSE, true>(p, c, work & kChunkFresh);
   else
     stream_collide_cell<S, ODD, FS, MOM, TRACE, DENSE>(p, c);
 }
@@ -65,7 +65,7 @@ k_stream_collide_all(const Params p) {
   if (work & (1u << kWorkFS1))
     stream_collide_cell<S, ODD, true, MOM, false, false>(p, c);
   else if (work & kChunkBody)
-    stream_collide_cell<S, ODD, true, MOM, false, true, true>(p, c);
+    stream_collide_cell<S, ODD, true, MOM, false, true, true>(p, c, work & kChunkFresh);
   else
     stream_collide_cell<S, ODD, true, MOM, false, true>(p, c);
 }
@@ -738,7 +738,7 @@ __global__ void __launch_bounds__(kListThreads) k_fs1(const Params p) {
       const uint32_t xm = tx > 0 ? tx - 1 : p.work_x - 1, xp = tx + 1 < p.work_x ? tx + 1 : 0;
       const uint32_t ym = ty > 0 ? ty - 1 : p.tile_rows - 1;
       const uint32_t yp = ty + 1 < p.tile_rows ? ty + 1 : 0;
-      const uint32_t pub = at(p.tile_pub, t);
+      const uint32_t pub = at(p.tile_pub, t), was = at(p.tile_body, t);
       uint32_t w[9];
       const uint32_t rows[3] = {ym * p.work_x, ty * p.work_x, yp * p.work_x};
 #pragma unroll
@@ -765,7 +765,8 @@ __global__ void __launch_bounds__(kListThreads) k_fs1(const Params p) {
         // and sets their mass, as the update's body-of-fluid path would.
         body = p.mass_mode != 0 && (all & kWorkFluid) && !(own & (0xffu << kWorkFS1));
       }
-      at(p.tile_body, t) = body;
+      const uint32_t kind = !body ? kBodyNot : (was == kBodyNot ? kBodyFresh : kBodyKept);
+      if (kind != was) at(p.tile_body, t) = kind;
       need = !skip && !body;
     }
     // Bounding box of this wavefront's tiles with stream-collide work (empty:
