@@ -40,19 +40,18 @@ def active_counts(solver):
 def algorithmic_bytes(active, inactive, s, free_surface):
     """Per-launch bytes of stream-collide and per-step bytes of the whole step.
     Stream-collide: 18 s (nine loads, nine stores) + 1 flag byte per active cell,
-    + 13 in (conservative) free-surface runs, as a body-of-fluid cell -- whose
+    + 8 in (conservative) free-surface runs, as a body-of-fluid cell -- whose
     update stream-collide does -- moves them: the excess shares pulled from
     the neighbours (each share is read by 8 neighbours, 4 bytes per cell
-    once), the mass store, its new excess share and flag (a surface cell
-    stores its density instead of the share and flag: 1 byte less); the
-    interface cells' extra velocity store and reconstructed populations
-    (< 0.2 % of the cells) are left out; 1 flag byte per inactive cell.  With
-    16-bit storage a free-surface cell also reads and writes its 2-byte
-    rounding residual (the mass the population stores rounded away).
-    Free-surface step: 18 s + 38 per active cell (+ 4 with 16-bit storage)."""
+    once) and its new excess share (a surface cell stores its mass or density
+    instead); the interface cells' extra velocity store and reconstructed
+    populations (< 0.2 % of the cells) are left out; 1 flag byte per inactive
+    cell.  With 16-bit storage a free-surface cell also reads and writes its
+    2-byte rounding residual (the mass the population stores rounded away).
+    Free-surface step: 18 s + 33 per active cell (+ 4 with 16-bit storage)."""
     resid = 4 if free_surface and s < 4 else 0
-    sc = active * (18 * s + 1 + (13 if free_surface else 0) + resid) + inactive
-    step = active * (18 * s + (38 if free_surface else 1) + resid) + inactive
+    sc = active * (18 * s + 1 + (8 if free_surface else 0) + resid) + inactive
+    step = active * (18 * s + (33 if free_surface else 1) + resid) + inactive
     return sc, step
 
 
@@ -364,6 +363,8 @@ def bench_batch(args):
                        "unit": "GB/s", "frac": round(out["achieved_GBs"] / HBM_PEAK_GBS, 4),
                        "traffic": traffic, "kernel": "batched stream-collide",
                        "algorithmic_bytes_per_launch": alg_bytes,
+                       "bytes_of": "steps one by one; runs of steps move them once per pass "
+                                   "of several",
                        "timing": "HIP events around the timed steps (graph replays)"}
     if k > 0:
         out.update({"one_at_a_time_ms_per_step": round(per_sync * 1e3, 4),
@@ -569,7 +570,9 @@ def main():
         "mlups_active_cells": round(r["active"] / (ms_step * 1e-3) / 1e6, 1),
         "step_roofline": {"algorithmic_bytes_per_step": int(r["step_bytes"]),
                           "achieved_GBs": round(r["step_bytes"] / (ms_step * 1e-3) / 1e9, 1),
-                          "frac": round(r["step_bytes"] / (ms_step * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)},
+                          "frac": round(r["step_bytes"] / (ms_step * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
+                          "bytes_of": "steps one by one" + ("" if case.free_surface else
+                                      "; runs of steps move them once per pass of several")},
         "kernel_ms": {k: round(v, 5) for k, v in zip(core.KERNEL_NAMES, r["per_kernel_ms"])},
         "wall_s_timed_region": round(r["wall"], 4),
     }

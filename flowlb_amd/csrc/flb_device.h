@@ -264,8 +264,9 @@ constexpr int kUpdateBlocksPerCU = 16;  // at most
 // Both grids follow the list lengths the last update published (a few steps
 // old; a longer list is walked in more rounds): a block without an item still
 // takes its turn to be dispatched and to read the length.  us per step with the
-// most blocks / with the lists' lengths: 101 x 101 17.4 / 15.4, 4096 x 1024 FP16S
-// 25.4 / 24.2, 8192 x 2048 FP32 80.4 / 79.1.
+// most blocks / with the lists' lengths: 4096 x 1024 FP16S 25.4 / 24.3, 8192 x 2048
+// FP32 80.4 / 79.1; 101 x 101 and 1024 x 256 the same (their idle blocks ran beside
+// the chain of the few with an item).
 
 constexpr int kWorkSC = 0, kWorkFS1 = 8;  // bit offsets in a tile_work word
 constexpr uint32_t kWorkQuiet = 1u << 16;  // the update found the tile quiet
