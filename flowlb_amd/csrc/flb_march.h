@@ -21,10 +21,11 @@
 //
 // What bounds it: a single step moves 18 values per cell (72 bytes in FP32) and is
 // bound by memory on large grids and by the launch on small ones.  T = 4 steps in
-// one pass move 18 x 61 / 58 values in all, a quarter, and the vector units become
-// the bound: about 110 instructions per step and row of 64 columns, 10 % of them
-// for halo columns.  Measured, us per step, single steps / passes: 8192 x 2048
-// FP32 226 / 77 (4.0 TB/s, 0.7 of the vector rate), FP16S 118 / 62, 2001 x 401
+// one pass move about a third of that and the vector units become the bound: about
+// 110 instructions per step and row of 64 columns, 10 % of them for halo columns.
+// A pass of four over 8192 x 2048 in FP32 reads 966 MB, 1.6 times the populations
+// (22 rows for a chunk of 16, 64 columns for 58), and writes 628 MB.  Measured, us per step, single steps / passes: 8192 x 2048
+// FP32 226 / 77 (4.7 TB/s of that traffic, 0.7 of the vector rate), FP16S 118 / 62, 2001 x 401
 // FP64 16.4 / 10.0; 512 x 128 FP32 3.8 / 3.3 for one handle alone and 3.7 / 1.3 with
 // three handles stepping side by side.
 #pragma once
