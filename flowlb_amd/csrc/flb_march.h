@@ -8,7 +8,7 @@
 // comes from registers: the populations along x of the row itself (kept one
 // iteration), those moving up of the row below (kept two) and those moving down
 // of the row above (just computed), each shifted by a lane for its x component
-// (DPP wavefront shift).  No LDS, no barrier; wavefronts are independent.
+// (DPP wavefront shift).  No LDS; no wavefront waits for another's values.
 //
 // Dependencies reach one cell per step, so of the 64 columns a wavefront loads
 // the 64 - 2 (T - 1) inner ones are its own, and it starts T - 1 rows below its
@@ -24,9 +24,10 @@
 // one pass move about a third of that and the vector units become the bound: about
 // 110 instructions per step and row of 64 columns, 10 % of them for halo columns.
 // A pass of four over 8192 x 2048 in FP32 reads 966 MB, 1.6 times the populations
-// (22 rows for a chunk of 16, 64 columns for 58), and writes 628 MB.  Measured, us per step, single steps / passes: 8192 x 2048
-// FP32 226 / 77 (4.7 TB/s of that traffic, 0.7 of the vector rate), FP16S 118 / 62, 2001 x 401
-// FP64 16.4 / 10.0; 512 x 128 FP32 3.8 / 3.3 for one handle alone and 3.7 / 1.3 with
+// (22 rows for a chunk of 16, 64 columns for 58), and writes 628 MB.  Measured, us
+// per step, single steps / passes: 8192 x 2048 FP32 226 / 77 (4.7 TB/s of that
+// traffic, 0.7 of the vector rate), FP16S 118 / 62, 2001 x 401 FP64 16.4 / 9.2;
+// 512 x 128 FP32 3.8 / 3.3 for one handle alone and 3.7 / 1.3 with
 // three handles stepping side by side.
 #pragma once
 
