@@ -238,6 +238,8 @@ struct flb_batch {
   flb::MarchBlock* march[flb::kMarchMax + 1] = {};
   uint32_t march_blocks[flb::kMarchMax + 1] = {};
   flb::MarchShape shape{0, 0};
+  flb::MarchShape rule_shape{0, 0};  // march_shape's choice
+  std::vector<std::vector<uint8_t>> io;  // per instance, its columns with inlet or outlet cells
   bool forced = false;
   flb::Tile* tiles = nullptr;
   uint32_t ntiles = 0;
@@ -270,6 +272,14 @@ int balloc(flb_batch* b, T** p, size_t count) {
   b->owned.push_back(v);
   *p = static_cast<T*>(v);
   return FLB_OK;
+}
+
+template <class T>
+void release(flb_batch* b, T** p) {
+  if (!*p) return;
+  (void)hipFree(*p);
+  b->owned.erase(std::remove(b->owned.begin(), b->owned.end(), static_cast<void*>(*p)), b->owned.end());
+  *p = nullptr;
 }
 
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
@@ -321,12 +331,7 @@ int build_tiles(flb_batch* b, int bx) {
       }
     }
   }
-  if (b->tiles) {
-    (void)hipFree(b->tiles);
-    b->owned.erase(std::remove(b->owned.begin(), b->owned.end(), static_cast<void*>(b->tiles)),
-                   b->owned.end());
-    b->tiles = nullptr;
-  }
+  release(b, &b->tiles);
   // The odd steps take the list's bands (runs of tiles of one instance and one
   // 32-row band) last to first, each band's tiles in their order, so that a
   // step starts on the tiles the previous one wrote last, which are still in
@@ -365,13 +370,13 @@ void use_set(flb_batch* b, int set) {
 // Block list of the passes of T steps: the inlet/outlet strips first (they take
 // longest), the others in an order that gives each XCD (block index mod 8)
 // consecutive groups of strips.
-int build_march(flb_batch* b, int T, const std::vector<std::vector<uint8_t>>& io) {
+int build_march(flb_batch* b, int T) {
   constexpr uint32_t G = flb::kMarchWaves;
   std::vector<flb::MarchBlock> first, rest;
   std::vector<uint32_t> order;
   for (uint32_t i = 0; i < b->host_inst.size(); ++i) {
     const flb::Params& p = b->host_inst[i];
-    const uint32_t nio = flb::march_strips(p.nx, T, io[i], order);
+    const uint32_t nio = flb::march_strips(p.nx, T, b->io[i], order);
     for (uint32_t ya = 0; ya < p.ny; ya += b->shape.rows) {
       flb::MarchBlock d{};
       d.inst = i;
@@ -397,6 +402,7 @@ int build_march(flb_batch* b, int T, const std::vector<std::vector<uint8_t>>& io
     const size_t w = (q % 8) * per + q / 8;
     first.push_back(w < rest.size() ? rest[w] : none);
   }
+  release(b, &b->march[T]);
   int rc = balloc(b, &b->march[T], first.size());
   if (rc) return rc;
   const size_t bytes = first.size() * sizeof(flb::MarchBlock);
@@ -405,18 +411,27 @@ int build_march(flb_batch* b, int T, const std::vector<std::vector<uint8_t>>& io
   return FLB_OK;
 }
 
+// Shape of the passes and their block lists.
+int set_shape(flb_batch* b, flb::MarchShape shape) {
+  b->shape = shape;
+  if (!shape.steps) return FLB_OK;
+  int rc = FLB_OK;
+  for (int T = flb::kMarchMin; T <= flb::kMarchMax && !rc; ++T) rc = build_march(b, T);
+  if (rc) b->shape = flb::MarchShape{0, 0};
+  return rc;
+}
+
 // The second population array, the four sets of parameters and the block lists
 // of the passes; single steps only where an instance does not fit the passes'
 // rules or the array would take more than a quarter of the memory left.
 int prepare_march(flb_batch* b, const flb_instance* in, size_t f_bytes) {
   const size_t count = b->host_inst.size();
-  int rc;
-  std::vector<std::vector<uint8_t>> io(count);
+  b->io.resize(count);
   uint64_t strip_rows = 0;
   bool fits = true;
   const uint32_t cols = flb::march_columns(flb::kMarchMax);
   for (size_t i = 0; i < count && fits; ++i) {
-    fits = flb::march_columns_io(in[i].flags, in[i].nx, in[i].ny, io[i]);
+    fits = flb::march_columns_io(in[i].flags, in[i].nx, in[i].ny, b->io[i]);
     strip_rows += uint64_t((in[i].nx + cols - 1) / cols) * in[i].ny;
     b->forced = b->forced || in[i].use_force;
   }
@@ -444,11 +459,8 @@ int prepare_march(flb_batch* b, const flb_instance* in, size_t f_bytes) {
   const size_t bytes = sets.size() * sizeof(flb::Params);
   BAT_HIP(b, b->staging.to_device(b->stream, b->inst_sets, sets.data(), bytes, bytes, 1));
   if (!alt) return FLB_OK;
-  const flb::MarchShape shape = flb::march_shape(b->ncu, strip_rows, b->storage == 0 ? 4 : 2, false);
-  b->shape = shape;
-  for (int T = flb::kMarchMin; T <= flb::kMarchMax; ++T)
-    if ((rc = build_march(b, T, io))) return rc;
-  return FLB_OK;
+  b->rule_shape = flb::march_shape(b->ncu, strip_rows, b->storage == 0 ? 4 : 2, false);
+  return set_shape(b, b->rule_shape);
 }
 
 int launch_step(flb_batch* b, int odd, bool mom) {
@@ -472,7 +484,7 @@ int launch_march(flb_batch* b, int T, int odd, bool mom) {
 
 // The next steps of a run with `left` to go: a pass, or a single step.
 int advance(flb_batch* b, uint64_t t, uint64_t left, bool mom, int* done) {
-  const int T = b->shape.steps ? flb::march_steps_next(left, b->shape.steps) : 0;
+  const int T = flb::march_steps_next(left, b->shape.steps);
   *done = T ? T : 1;
   const bool last = mom && left == uint64_t(*done);
   return T ? launch_march(b, T, int(t & 1), last) : launch_step(b, int(t & 1), last);
@@ -737,6 +749,14 @@ int flb_batch_step(flb_batch* b, uint64_t nsteps) {
     }
   }
   return rc;
+}
+
+int flb_test_batch_pass_shape(flb_batch* b, int32_t steps, uint32_t rows) {
+  if (!b || !b->rule_shape.steps || steps == 1 || steps > flb::kMarchMax || (steps > 1 && rows == 0))
+    return FLB_ERR_ARGUMENT;
+  BAT_HIP(b, hipStreamSynchronize(b->stream));
+  drop_graph(b);
+  return set_shape(b, steps < 0 ? b->rule_shape : flb::MarchShape{steps, rows});
 }
 
 int flb_batch_sync(flb_batch* b) {

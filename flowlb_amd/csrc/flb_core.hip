@@ -365,6 +365,7 @@ int prepare_march(flb_handle* h, const uint8_t* flags) {
 }
 
 flb::MarchShape march_shape(const flb_handle* h) {
+  if (h->pass_shape.steps >= 0) return h->pass_shape;
   const uint32_t cols = flb::march_columns(flb::kMarchMax);
   return flb::march_shape(h->cus, uint64_t((h->nx + cols - 1) / cols) * h->ny, h->elem_bytes,
                           h->opt.smagorinsky != 0);
@@ -1053,6 +1054,7 @@ MarchGrid march_grid(const flb_handle* h, int T, uint32_t rows, uint32_t io_rows
 // rows (single steps 35.6).  Where two or three rows do, a pass of 2 steps has
 // the shorter chain: 256 x 64 3.4, against 4.0 with 3 steps (single steps 5.4).
 MarchShape adjoint_shape(const flb_handle* h) {
+  if (h->reverse_shape.steps >= 0) return h->reverse_shape;
   for (uint32_t r = 2; r <= 8; ++r) {
     const MarchShape s{r < 4 ? 2 : 3, r};
     if (march_grid(h, s.steps, r, (r + 1) / 2).blocks <= uint32_t(h->cus)) return s;
@@ -1077,9 +1079,8 @@ int flb_step(flb_handle* h, uint64_t nsteps) {
   constexpr uint64_t G = flb_handle::kGroup, R = flb_handle::kRing;
   for (uint64_t k = 0; k < nsteps;) {
     const uint64_t left = nsteps - k;
-    if (h->f_alt && left > 1) {
-      // Passes of the shape's steps; a single step is not left over.
-      const int T = flb::march_steps_next(left, march_shape(h).steps);
+    // Passes of the shape's steps; a single step is not left over.
+    if (const int T = h->f_alt ? flb::march_steps_next(left, march_shape(h).steps) : 0) {
       const int rc = enqueue_march(h, T, left == uint64_t(T));
       if (rc) return rc;
       k += uint64_t(T);
@@ -1100,6 +1101,16 @@ int flb_step(flb_handle* h, uint64_t nsteps) {
     ++k;
     if (throttle && t % G == G - 1) FLB_HIP(h, hipEventRecord(h->in_flight[g % R], h->stream));
   }
+  return FLB_OK;
+}
+
+int flb_test_pass_shape(flb_handle* h, int32_t steps, uint32_t rows, int32_t reverse_steps,
+                        uint32_t reverse_rows) {
+  if (!h || !h->f_alt || steps == 1 || steps > flb::kMarchMax || (steps > 1 && rows == 0) ||
+      reverse_steps == 1 || reverse_steps > 3 || (reverse_steps > 1 && reverse_rows == 0))
+    return FLB_ERR_ARGUMENT;
+  h->pass_shape = flb::MarchShape{steps, rows};
+  h->reverse_shape = flb::MarchShape{reverse_steps, reverse_rows};
   return FLB_OK;
 }
 

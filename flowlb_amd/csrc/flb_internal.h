@@ -57,7 +57,7 @@ struct MarchShape {
 MarchShape march_shape(int cus, uint64_t strip_rows, int elem_bytes, bool heavy);
 // Steps of the next pass of a run with `left` steps to go; 0: a single step.
 inline int march_steps_next(uint64_t left, int most) {
-  if (left < 2) return 0;
+  if (left < 2 || most < kMarchMin) return 0;
   return int(left == uint64_t(most) + 1 ? (left + 1) / 2 : (left < uint64_t(most) ? left : most));
 }
 // Strips of a domain of nx columns for passes of `steps` steps, those whose 64
@@ -172,6 +172,8 @@ struct flb_handle {
   void* f_alt = nullptr;
   uint32_t* march_order[flb::kMarchMax + 1] = {};
   uint32_t march_io[flb::kMarchMax + 1] = {};
+  // Shapes set by flb_test_pass_shape; steps < 0: by march_shape, adjoint_shape.
+  flb::MarchShape pass_shape{-1, 0}, reverse_shape{-1, 0};
   uint8_t* flags[2] = {nullptr, nullptr};
   int cur = 0;
   float* rho = nullptr;
@@ -248,3 +250,12 @@ int copy_cells_out(flb_handle* h, void* host, const void* dev, size_t elem, int 
 void host_initial_populations(uint32_t nx, uint32_t ny, const float* rho0, const float* u0,
                               std::vector<float>& fs);
 }  // namespace flb
+
+// For tests and measurements, on handles whose domain fits the passes: the steps
+// (0: single steps only; 2 to 4, in reverse 2 or 3) and rows per chunk of the
+// passes in place of the rules' choice; steps < 0 returns to the rules.
+extern "C" {
+int flb_test_pass_shape(flb_handle* h, int32_t steps, uint32_t rows, int32_t reverse_steps,
+                        uint32_t reverse_rows);
+int flb_test_batch_pass_shape(struct flb_batch* b, int32_t steps, uint32_t rows);
+}
