@@ -134,6 +134,9 @@ k_batch_march(const MarchBlock* __restrict__ blocks, const Params* __restrict__ 
   a.pub_u_in = q.pub_u[odd ^ 1];
   a.pub_rho_out = q.pub_rho[odd];
   a.pub_u_out = q.pub_u[odd];
+  // A program cannot reach an instance's fields, so these hold the same values.
+  a.own_rho = a.pub_rho_in;
+  a.own_u = a.pub_u_in;
   a.odd = odd;
   a.moments = moments;
   if (d->io) {

@@ -810,6 +810,8 @@ static int enqueue_march(flb_handle* h, int T, bool moments, const flb::MarchTra
   a.pub_u_in = h->pub_u[last];
   a.pub_rho_out = h->pub_rho[last ^ 1];
   a.pub_u_out = h->pub_u[last ^ 1];
+  a.own_rho = h->rho;
+  a.own_u = h->u;
   a.odd = int32_t(h->t & 1u);
   a.moments = moments;
   const uint32_t rows = march_shape(h).rows;

@@ -93,6 +93,11 @@ struct March {
   const float* pub_u_in;
   float* pub_rho_out;
   float* pub_u_out;
+  // Where inlet cells find the velocity they prescribe and outlet cells the density
+  // they keep: the readback fields of a handle, which its program may write to.  The
+  // pass leaves those values as they are.
+  const float* own_rho;
+  const float* own_u;
   int32_t odd;        // t % 2
   int32_t moments;    // write the readback fields of the last step
   // TRACE: the trace of step t + k at trace + k * 3 N elements of R; and, where
@@ -125,6 +130,28 @@ __device__ __forceinline__ double from_right(double v) {
   const uint32_t lo = __builtin_amdgcn_update_dpp(0, int(uint32_t(b)), 0x130, 0xf, 0xf, true);
   const uint32_t hi = __builtin_amdgcn_update_dpp(0, int(uint32_t(b >> 32)), 0x130, 0xf, 0xf, true);
   return __builtin_bit_cast(double, uint64_t(hi) << 32 | lo);
+}
+
+__device__ __forceinline__ uint32_t left_flags(uint32_t fl) {
+  return uint32_t(__builtin_amdgcn_update_dpp(0, int(fl), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ uint32_t right_flags(uint32_t fl) {
+  return uint32_t(__builtin_amdgcn_update_dpp(0, int(fl), 0x130, 0xf, 0xf, true));
+}
+
+// In the flags a pass keeps of its rows (where the bit says nothing a pass uses):
+// an inlet beside a wall it reads the density of, or an outlet beside a wall or an
+// inlet it reads the velocity of.  Walls publish nothing and inlets no velocity;
+// what the publication buffers were filled with stands there.
+constexpr uint32_t kFilled = kFluid;
+
+// A loaded value that is waited for here, in the branch that loads it: waited for
+// where the branches meet, it would hold up every wavefront until the loads of the
+// row ahead are in as well (1.5 % of a gradient of 1024 x 256).
+template <class R>
+__device__ __forceinline__ R arrived(R v) {
+  asm volatile("" : "+v"(v));
+  return v;
 }
 
 // How the pass holds populations between memory and the collision: in the
@@ -196,15 +223,13 @@ constexpr int march_occupancy() {
   return S::kBytes > 4 ? 2 : (MODEL >= kMarchUnforced ? 3 : 4);
 }
 
-// What an inlet or outlet cell reads (stream_collide_cell): the published
-// density of the cell at x + 1 and velocity of the cell at x - 1, of the step
-// before, and its own published values.  An inlet cell never publishes a
-// velocity and an outlet cell's density never changes, so these hold the
-// velocity the inlet prescribes and the density the outlet keeps.
+// The density and velocity an inlet or outlet cell takes (stream_collide_cell): an
+// inlet the published density of the cell at x + 1, of the step before, and the
+// velocity it prescribes; an outlet the published velocity of the cell at x - 1 and
+// the density it keeps.
 template <class R>
 struct IoValues {
   R rho, ux, uy;
-  R rho_next, ux_prev, uy_prev;
 };
 
 // One step of one cell: g holds its incoming populations and receives the
@@ -230,16 +255,11 @@ __device__ __forceinline__ void march_cell(const Params& p, uint8_t fl, uint32_t
   constexpr R unit = Held<S>::kUnit;
   const uint8_t io = IO ? fl & (kInlet | kOutlet) : 0;
   R rho1, mx = R(0), my = R(0);
-  if (IO && (io & kInlet)) {
-    rho = v.rho_next;
+  if (IO && io) {
+    rho = v.rho;
     rho1 = rho - R(1);
     ux = v.ux;
     uy = v.uy;
-  } else if (IO && (io & kOutlet)) {
-    rho = v.rho;
-    rho1 = rho - R(1);
-    ux = v.ux_prev;
-    uy = v.uy_prev;
   } else {
     rho1 = g[0];
 #pragma unroll
@@ -297,8 +317,13 @@ __device__ __forceinline__ void march_rows(const Params& p, const March& a, uint
   auto up = [&](uint32_t y) { return y + 1 == ny ? 0u : y + 1; };
   auto down = [&](uint32_t y) { return y == 0 ? ny - 1 : y - 1; };
 
+  const R* const pub_rho = fld<R>(const_cast<float*>(a.pub_rho_in));
+  const R* const pub_u = fld<R>(const_cast<float*>(a.pub_u_in));
+  const R* const own_rho = fld<R>(const_cast<float*>(a.own_rho));
+  const R* const own_u = fld<R>(const_cast<float*>(a.own_u));
   E raw[9];
   uint8_t raw_fl;
+  uint8_t next_fl = 0;  // IO: flags of the row after, which say what it loads
   float raw_alpha = 0.0f;
   IoValues<R> raw_io{};
   auto load_row = [&](uint32_t y) {
@@ -315,17 +340,21 @@ __device__ __forceinline__ void march_rows(const Params& p, const March& a, uint
     raw[6] = at(there(5) + ru, xr);
     raw[7] = at(here(7) + rc, x);
     raw[8] = at(there(7) + rd, xr);
-    raw_fl = at(p.flags + rc, x);
     if (MODEL == kMarchDrag && p.alpha) raw_alpha = at(p.alpha + rc, x);
-    if (IO) {  // the neighbours' too: the end lanes have none to take them from
-      const R* const r = fld<R>(const_cast<float*>(a.pub_rho_in)) + rc;
-      const R* const u = fld<R>(const_cast<float*>(a.pub_u_in)) + rc;
-      raw_io.rho = at(r, x);
-      raw_io.ux = at(u, x);
-      raw_io.uy = at(u + p.N, x);
-      raw_io.rho_next = at(r, xr);
-      raw_io.ux_prev = at(u, xl);
-      raw_io.uy_prev = at(u + p.N, xl);
+    if (IO) {
+      raw_fl = next_fl;
+      next_fl = at(p.flags + ru, x);
+      if (raw_fl & kInlet) {
+        raw_io.rho = at(pub_rho + rc, xr);
+        raw_io.ux = at(own_u + rc, x);
+        raw_io.uy = at(own_u + p.N + rc, x);
+      } else if (raw_fl & kOutlet) {
+        raw_io.rho = at(own_rho + rc, x);
+        raw_io.ux = at(pub_u + rc, xl);
+        raw_io.uy = at(pub_u + p.N + rc, xl);
+      }
+    } else {
+      raw_fl = at(p.flags + rc, x);
     }
   };
   auto store_row = [&](uint32_t y, const R* g) {
@@ -359,6 +388,7 @@ __device__ __forceinline__ void march_rows(const Params& p, const March& a, uint
   float alpha[T] = {};  // solid fractions of these rows (kMarchDrag)
 
   uint32_t y1 = ya >= uint32_t(H) ? ya - H : ya + ny - H;  // row of step 1 (ny >= T)
+  if (IO) next_fl = at(p.flags + uint64_t(y1) * pitch, x);
   load_row(y1);
   const uint32_t iterations = yb - ya + 2 * H;
   const auto iterate = [&](uint32_t it, auto steady) {
@@ -366,6 +396,12 @@ __device__ __forceinline__ void march_rows(const Params& p, const March& a, uint
 #pragma unroll
     for (int i = 0; i < 9; i++) g[i] = Held<S>::in(raw[i]);
     fls = fls << 8 | raw_fl;
+    if (IO) {
+      const uint32_t left = left_flags(raw_fl), right = right_flags(raw_fl);
+      const bool filled = (raw_fl & kInlet) ? (right & (kGas | kWall))
+                                            : (raw_fl & kOutlet) && (left & (kGas | kWall | kInlet));
+      fls = (fls & ~uint32_t(kFilled)) | (filled ? kFilled : 0u);
+    }
     if (MODEL == kMarchDrag) {
 #pragma unroll
       for (int s = T - 1; s > 0; s--) alpha[s] = alpha[s - 1];
@@ -384,17 +420,26 @@ __device__ __forceinline__ void march_rows(const Params& p, const March& a, uint
         const uint8_t fl = uint8_t(fls >> (8 * (s - 1)));
         const uint32_t n = ys * pitch + x;
         IoValues<R> v{};
+        const bool solid = fl & (kGas | kWall);
         if (IO) {
           v = kept;
           if (s > 1) {
-            v.rho_next = from_right(v.rho);
-            v.ux_prev = from_left(v.ux);
-            v.uy_prev = from_left(v.uy);
+            const R next = from_right(v.rho), px = from_left(v.ux), py = from_left(v.uy);
+            if (fl & kInlet) {
+              v.rho = next;
+              if (fl & kFilled) v.rho = arrived(at(pub_rho + uint64_t(ys) * pitch, xr));
+            } else {
+              v.ux = px;
+              v.uy = py;
+              if (fl & kFilled) {
+                v.ux = arrived(at(pub_u + uint64_t(ys) * pitch, xl));
+                v.uy = arrived(at(pub_u + p.N + uint64_t(ys) * pitch, xl));
+              }
+            }
           }
         }
         R tr[3];
         march_cell<S, MODEL, IO>(p, fl, n, alpha[s - 1], v, g, rho, ux, uy, tr);
-        const bool solid = fl & (kGas | kWall);
         // The row is in the chunk (the halo rows are another wavefront's).
         if (TRACE && it - uint32_t(H + s - 1) < yb - ya && own) {
           if (!solid && a.trace) {
@@ -421,8 +466,7 @@ __device__ __forceinline__ void march_rows(const Params& p, const March& a, uint
             }
           }
           if (IO) {
-            const uint32_t left = uint32_t(__builtin_amdgcn_update_dpp(0, int(fl), 0x138, 0xf, 0xf, true));
-            const uint32_t right = uint32_t(__builtin_amdgcn_update_dpp(0, int(fl), 0x130, 0xf, 0xf, true));
+            const uint32_t left = left_flags(fl), right = right_flags(fl);
             if (own && !solid && (left & kInlet)) at(fld<R>(a.pub_rho_out), n) = rho;
             if (own && !solid && (right & kOutlet) && !(fl & kInlet)) {
               at(fld<R>(a.pub_u_out), n) = ux;
@@ -457,9 +501,9 @@ __device__ __forceinline__ void march_rows(const Params& p, const March& a, uint
             kept.rho = pr[b];
             kept.ux = pu[b];
             kept.uy = pv[b];
-            pr[b] = solid ? v.rho : rho;
-            pu[b] = solid || (fl & kInlet) ? v.ux : ux;
-            pv[b] = solid || (fl & kInlet) ? v.uy : uy;
+            pr[b] = rho;
+            pu[b] = (fl & kInlet) ? v.ux : ux;
+            pv[b] = (fl & kInlet) ? v.uy : uy;
           }
 #pragma unroll
           for (int i = 0; i < 9; i++) g[i] = in[i];
