@@ -903,7 +903,17 @@ hipError_t Staging::init() {
   hipError_t e = hipSuccess;
   for (hipEvent_t& d : done)
     if (e == hipSuccess) e = hipEventCreateWithFlags(&d, hipEventDisableTiming);
+  (void)reserve(kSmall);  // without it the runtime copies
   return e;
+}
+
+bool Staging::known(const void* host) {
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, host) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type != hipMemoryTypeUnregistered;
 }
 
 void Staging::release() {
@@ -957,9 +967,12 @@ hipError_t Staging::to_host(hipStream_t s, void* host, const void* dev, size_t p
   const size_t total = row_bytes * rows;
   if (!total) return hipStreamSynchronize(s);
   const bool flat = pitch == row_bytes;
-  if ((!flat && row_bytes > kBytes) || !reserve(total)) {  // rows longer than a buffer
+  const bool pinned = known(host);
+  const bool direct = pinned || (flat ? total > kSmall && total < kLargeIn
+                                      : row_bytes > kBytes);  // rows longer than a buffer
+  if (direct || !reserve(total)) {
     const hipError_t e =
-        flat ? hipMemcpyAsync(host, dev, total, hipMemcpyDeviceToHost, s)
+        flat && (!pinned || rows == 1) ? hipMemcpyAsync(host, dev, total, hipMemcpyDeviceToHost, s)
              : hipMemcpy2DAsync(host, row_bytes, dev, pitch, row_bytes, rows, hipMemcpyDeviceToHost, s);
     return e == hipSuccess ? hipStreamSynchronize(s) : e;
   }
@@ -992,9 +1005,11 @@ hipError_t Staging::to_device(hipStream_t s, void* dev, const void* host, size_t
   const size_t total = row_bytes * rows;
   if (!total) return hipStreamSynchronize(s);
   const bool flat = pitch == row_bytes;
-  if ((!flat && row_bytes > kBytes) || !reserve(total)) {
+  const bool pinned = known(host);
+  const bool direct = pinned || (flat ? total <= kLargeOut : row_bytes > kBytes);
+  if (direct || !reserve(total)) {
     const hipError_t e =
-        flat ? hipMemcpyAsync(dev, host, total, hipMemcpyHostToDevice, s)
+        flat && (!pinned || rows == 1) ? hipMemcpyAsync(dev, host, total, hipMemcpyHostToDevice, s)
              : hipMemcpy2DAsync(dev, pitch, host, row_bytes, row_bytes, rows, hipMemcpyHostToDevice, s);
     return e == hipSuccess ? hipStreamSynchronize(s) : e;
   }

@@ -74,14 +74,27 @@ MarchFn get_march(int storage, int steps, int model, bool trace);
 }  // namespace flb
 
 namespace flb {
-// Pinned buffers a handle's host copies go through (two, so that one is filled
-// while the other is copied), allocated by the first copy and freed with the
-// handle.  A strided copy to or from pageable memory is done row by row by the
-// runtime, 7 us each: 7.2 ms for 1000 rows of 8 KB against 0.25 ms through the
-// buffers (54 GB/s over the bus, 70 GB/s for the host's copy).  One copy at a
-// time, as all calls on a handle.
+// Pinned buffers a handle's copies to and from pageable memory go through (two,
+// so that one is filled while the other is copied): a small one from the start, so
+// that short readbacks never allocate, larger ones by the first copy that takes
+// them; freed with the handle.  A strided copy to or from pageable memory is done
+// row by row by the runtime, 7 us each: 7.2 ms for 1000 rows of 8 KB against 0.25 ms
+// through the buffers (54 GB/s over the bus, 70 GB/s for the host's copy).
+//
+// The runtime copies by itself (direct) where that is the faster way:
+//  - memory the driver knows, as a caller's pinned buffers, needs no second copy:
+//    u and rho of 1024 x 512 cells 0.13 ms, through the buffers 0.34 (as a strided
+//    copy also where the rows have no padding: 64 x 16 18 us, as a plain one 25);
+//  - contiguous copies of middling size, which the runtime stages as well: to the
+//    host 8 KiB 23 us, 16 by the buffers, 32 KiB 30 / 35, 590 KB 48 / 55, 1.2 MB 92 / 90,
+//    19 MB 1100 / 840; to the device, with what the caller does before, 150 KB 36 / 42,
+//    9.4 MB 527 / 600, 38 MB 9320 / 9320.
+// One copy at a time, as all calls on a handle.
 struct Staging {
   static constexpr size_t kBytes = 8u << 20;
+  static constexpr size_t kSmall = 16u << 10;        // direct above, to the host
+  static constexpr size_t kLargeIn = 1u << 20;       // direct below, to the host
+  static constexpr size_t kLargeOut = 2 * kBytes;    // direct up to, to the device
   void* buf[2] = {nullptr, nullptr};
   size_t size = 0;
   hipEvent_t done[2] = {nullptr, nullptr};
@@ -100,6 +113,7 @@ struct Staging {
  private:
   bool reserve(size_t bytes);
   void release();
+  static bool known(const void* host);  // to the driver
 };
 }  // namespace flb
 
