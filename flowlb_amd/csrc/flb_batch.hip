@@ -26,6 +26,7 @@
 #include <hip/hip_cooperative_groups.h>
 
 #include "flb_cell.h"
+#include "flb_cost.h"
 #include "flb_internal.h"
 #include "flb_march.h"
 
@@ -242,6 +243,10 @@ struct flb_batch {
   uint32_t march_blocks[flb::kMarchMax + 1] = {};
   flb::MarchShape shape{0, 0};
   flb::MarchShape rule_shape{0, 0};  // march_shape's choice
+  bool any_shape = false;            // set by flb_test_batch_pass_shape: taken always
+  flb::StepModel model{};            // flb_cost.h
+  flb::PassRows pass_rows[flb::kMarchMax + 1];
+  double mb = 0.0;                   // populations, megabytes
   std::vector<std::vector<uint8_t>> io;  // per instance, its columns with inlet or outlet cells
   bool forced = false;
   flb::Tile* tiles = nullptr;
@@ -377,9 +382,12 @@ int build_march(flb_batch* b, int T) {
   constexpr uint32_t G = flb::kMarchWaves;
   std::vector<flb::MarchBlock> first, rest;
   std::vector<uint32_t> order;
+  b->pass_rows[T] = flb::PassRows{};
   for (uint32_t i = 0; i < b->host_inst.size(); ++i) {
     const flb::Params& p = b->host_inst[i];
     const uint32_t nio = flb::march_strips(p.nx, T, b->io[i], order);
+    b->pass_rows[T].add(uint32_t(order.size()) - nio, nio, p.ny, T, b->shape.rows,
+                        (b->shape.rows + G - 1) / G, true);
     for (uint32_t ya = 0; ya < p.ny; ya += b->shape.rows) {
       flb::MarchBlock d{};
       d.inst = i;
@@ -462,6 +470,10 @@ int prepare_march(flb_batch* b, const flb_instance* in, size_t f_bytes) {
   const size_t bytes = sets.size() * sizeof(flb::Params);
   BAT_HIP(b, b->staging.to_device(b->stream, b->inst_sets, sets.data(), bytes, bytes, 1));
   if (!alt) return FLB_OK;
+  b->model.storage = b->storage;
+  b->model.force = b->forced;
+  b->model.kernel = b->forced ? flb::kMarchGeneral : flb::kMarchPlain;
+  b->mb = 1e-6 * double(f_bytes);
   b->rule_shape = flb::march_shape(b->ncu, strip_rows, b->storage == 0 ? 4 : 2, false);
   return set_shape(b, b->rule_shape);
 }
@@ -485,9 +497,18 @@ int launch_march(flb_batch* b, int T, int odd, bool mom) {
   return FLB_OK;
 }
 
+// Whether a pass of T steps takes less time than T single steps in the batch's
+// tile order (flb_cost.h).
+bool pass_pays(const flb_batch* b, int T) {
+  return b->any_shape ||
+         flb::faster(flb::pass_time(b->model, T, b->pass_rows[T], b->mb, b->ncu),
+                     flb::batch_single_time(b->model, b->mb, b->order == FLB_BATCH_ORDER_ROWS));
+}
+
 // The next steps of a run with `left` to go: a pass, or a single step.
 int advance(flb_batch* b, uint64_t t, uint64_t left, bool mom, int* done) {
-  const int T = flb::march_steps_next(left, b->shape.steps);
+  int T = flb::march_steps_next(left, b->shape.steps);
+  if (T && !(pass_pays(b, b->shape.steps) && pass_pays(b, T))) T = 0;
   *done = T ? T : 1;
   const bool last = mom && left == uint64_t(*done);
   return T ? launch_march(b, T, int(t & 1), last) : launch_step(b, int(t & 1), last);
@@ -759,6 +780,7 @@ int flb_test_batch_pass_shape(flb_batch* b, int32_t steps, uint32_t rows) {
     return FLB_ERR_ARGUMENT;
   BAT_HIP(b, hipStreamSynchronize(b->stream));
   drop_graph(b);
+  b->any_shape = steps >= 0;
   return set_shape(b, steps < 0 ? b->rule_shape : flb::MarchShape{steps, rows});
 }
 

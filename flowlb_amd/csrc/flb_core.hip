@@ -24,6 +24,7 @@
 #include "../../include/flb_core.h"
 #include "flb_device.h"
 
+#include "flb_cost.h"
 #include "flb_internal.h"
 #include "flb_march.h"
 
@@ -369,6 +370,29 @@ flb::MarchShape march_shape(const flb_handle* h) {
   const uint32_t cols = flb::march_columns(flb::kMarchMax);
   return flb::march_shape(h->cus, uint64_t((h->nx + cols - 1) / cols) * h->ny, h->elem_bytes,
                           h->opt.smagorinsky != 0);
+}
+
+uint32_t march_io_rows(uint32_t rows) { return (rows + flb::kMarchWaves - 1) / flb::kMarchWaves; }
+
+// Whether a pass of T steps takes less time than T single steps (flb_cost.h).
+bool pass_pays(const flb_handle* h, int T) {
+  if (h->pass_shape.steps >= 0) return true;
+  flb::StepModel m{};
+  m.storage = h->opt.storage;
+  m.force = h->opt.use_force != 0;
+  m.drag = h->alpha != nullptr;
+  m.trt = h->opt.collision != FLB_SRT;
+  m.guo = h->opt.collision == FLB_TRT_GUO && (m.force || m.drag);
+  m.smagorinsky = h->opt.smagorinsky != 0;
+  m.kernel = march_model(h);
+  const uint32_t rows = march_shape(h).rows, io_rows = march_io_rows(rows);
+  const flb::MarchGrid g = flb::march_grid(h, T, rows, io_rows);
+  flb::PassRows r;
+  r.add(g.strips - g.io_strips, g.io_strips, h->ny, T, rows, io_rows);
+  const double mb = 9e-6 * double(h->Nd) * h->elem_bytes;
+  const uint32_t tiles = (h->nx + uint32_t(block_x(h)) - 1) / uint32_t(block_x(h));
+  const bool same_xcd = uint64_t(flb::last_band_rows(h->ny)) * tiles % 8 == 0;
+  return flb::faster(flb::pass_time(m, T, r, mb, h->cus), flb::single_time(m, mb, same_xcd));
 }
 
 }  // namespace
@@ -815,7 +839,7 @@ static int enqueue_march(flb_handle* h, int T, bool moments, const flb::MarchTra
   a.odd = int32_t(h->t & 1u);
   a.moments = moments;
   const uint32_t rows = march_shape(h).rows;
-  a.grid = flb::march_grid(h, T, rows, (rows + flb::kMarchWaves - 1) / flb::kMarchWaves);
+  a.grid = flb::march_grid(h, T, rows, march_io_rows(rows));
   if (trace) {
     a.trace = trace->trace;
     a.discharge = trace->discharge;
@@ -1094,10 +1118,15 @@ int flb_step(flb_handle* h, uint64_t nsteps) {
   if (!h) return FLB_ERR_ARGUMENT;
   const bool throttle = h->box_host != nullptr;
   constexpr uint64_t G = flb_handle::kGroup, R = flb_handle::kRing;
+  // Passes of the shape's steps, and of what is left of them at the end, where they
+  // take less time than single steps.
+  const int most = h->f_alt && nsteps > 1 ? march_shape(h).steps : 0;
+  bool pays[flb::kMarchMax + 1] = {};
+  for (int T = flb::kMarchMin; T <= most; ++T) pays[T] = pass_pays(h, T);
   for (uint64_t k = 0; k < nsteps;) {
     const uint64_t left = nsteps - k;
-    // Passes of the shape's steps; a single step is not left over.
-    if (const int T = h->f_alt ? flb::march_steps_next(left, march_shape(h).steps) : 0) {
+    const int T = most && pays[most] ? flb::march_steps_next(left, most) : 0;
+    if (pays[T]) {
       const int rc = enqueue_march(h, T, left == uint64_t(T));
       if (rc) return rc;
       k += uint64_t(T);
