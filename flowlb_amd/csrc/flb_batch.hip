@@ -604,8 +604,11 @@ int flb_batch_create(const flb_instance* in, uint32_t count, int32_t storage, in
   };
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, device) == hipSuccess) b->ncu = prop.multiProcessorCount;
+  size_t largest = 0;  // velocities
+  for (uint32_t i = 0; i < count; ++i)
+    largest = std::max(largest, 2 * sizeof(float) * in[i].nx * in[i].ny);
   if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess ||
-      b->staging.init() != hipSuccess)
+      b->staging.init(largest) != hipSuccess)
     return bail(FLB_ERR_DEVICE);
   const size_t eb = storage == 0 ? 4 : 2;
   // Offsets of every instance in the shared allocations (elements).

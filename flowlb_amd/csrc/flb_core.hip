@@ -497,7 +497,7 @@ int flb_create(const flb_options* opt, const uint8_t* flags, uint32_t nx, uint32
           hipSuccess || h->cus <= 0)
     h->cus = 256;
   if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess ||
-      h->staging.init() != hipSuccess)
+      h->staging.init(2 * N * h->field_bytes) != hipSuccess)
     return bail(FLB_ERR_DEVICE);
 
   int rc = FLB_OK;
@@ -923,11 +923,11 @@ MarchShape march_shape(int cus, uint64_t strip_rows, int elem_bytes, bool heavy)
                     uint32_t(std::min<uint64_t>(std::max<uint64_t>(rows, least), most))};
 }
 
-hipError_t Staging::init() {
+hipError_t Staging::init(size_t bytes) {
   hipError_t e = hipSuccess;
   for (hipEvent_t& d : done)
     if (e == hipSuccess) e = hipEventCreateWithFlags(&d, hipEventDisableTiming);
-  (void)reserve(kSmall);  // without it the runtime copies
+  (void)reserve(std::min(std::max(bytes, kSmall), kBytes));  // without it the runtime copies
   return e;
 }
 

@@ -75,9 +75,9 @@ MarchFn get_march(int storage, int steps, int model, bool trace);
 
 namespace flb {
 // Pinned buffers a handle's copies to and from pageable memory go through (two,
-// so that one is filled while the other is copied): a small one from the start, so
-// that short readbacks never allocate, larger ones by the first copy that takes
-// them; freed with the handle.  A strided copy to or from pageable memory is done
+// so that one is filled while the other is copied): one for the largest field from
+// the start, so that short readbacks never allocate, the other by the first copy
+// of more than 8 MiB; freed with the handle.  A strided copy to or from pageable memory is done
 // row by row by the runtime, 7 us each: 7.2 ms for 1000 rows of 8 KB against 0.25 ms
 // through the buffers (54 GB/s over the bus, 70 GB/s for the host's copy).
 //
@@ -102,7 +102,9 @@ struct Staging {
   Staging(const Staging&) = delete;
   Staging& operator=(const Staging&) = delete;
   ~Staging();
-  hipError_t init();  // with the handle's device current
+  // With the handle's device current.  bytes: the largest field to be copied (each
+  // pinned allocation takes 0.2 to 0.6 ms).
+  hipError_t init(size_t bytes);
   // `rows` rows of row_bytes: contiguous on the host, `pitch` bytes apart on
   // the device.  Returns when the host memory may be used.
   hipError_t to_host(hipStream_t s, void* host, const void* dev, size_t pitch, size_t row_bytes,
