@@ -244,6 +244,8 @@ struct flb_batch {
   flb::MarchShape shape{0, 0};
   flb::MarchShape rule_shape{0, 0};  // march_shape's choice
   bool any_shape = false;            // set by flb_test_batch_pass_shape: taken always
+  // Runs of several steps: by flb_cost.h, or what flb_batch_autotune measured.
+  enum Way { kEstimated, kSingle, kPasses } way = kEstimated;
   flb::StepModel model{};            // flb_cost.h
   flb::PassRows pass_rows[flb::kMarchMax + 1];
   double mb = 0.0;                   // populations, megabytes
@@ -497,10 +499,11 @@ int launch_march(flb_batch* b, int T, int odd, bool mom) {
   return FLB_OK;
 }
 
-// Whether a pass of T steps takes less time than T single steps in the batch's
-// tile order (flb_cost.h).
+// Whether to take a pass of T steps: where it takes less time than T single steps
+// in the batch's tile order (flb_cost.h).
 bool pass_pays(const flb_batch* b, int T) {
-  return b->any_shape ||
+  if (b->way == flb_batch::kSingle) return false;
+  return b->any_shape || (b->way == flb_batch::kPasses && T == b->shape.steps) ||
          flb::faster(flb::pass_time(b->model, T, b->pass_rows[T], b->mb, b->ncu),
                      flb::batch_single_time(b->model, b->mb, b->order == FLB_BATCH_ORDER_ROWS));
 }
@@ -712,6 +715,7 @@ int flb_batch_configure(flb_batch* b, int32_t block_x, int32_t grid, int32_t gra
       graph_chunk % 2)
     return FLB_ERR_ARGUMENT;
   drop_graph(b);
+  b->way = flb_batch::kEstimated;
   b->mode = FLB_BATCH_LAUNCH;
   b->grid = grid;
   b->graph_chunk = graph_chunk;
@@ -723,6 +727,7 @@ int flb_batch_set_order(flb_batch* b, int32_t order) {
   if (!b || order < FLB_BATCH_ORDER_ROWS || order > FLB_BATCH_ORDER_BANDS) return FLB_ERR_ARGUMENT;
   if (order == b->order) return FLB_OK;
   drop_graph(b);
+  b->way = flb_batch::kEstimated;
   b->order = order;
   return build_tiles(b, b->block_x);
 }
@@ -742,6 +747,7 @@ int flb_batch_configure_persistent(flb_batch* b, int32_t block_x, int32_t blocks
   }
   drop_graph(b);
   if (block_x != b->block_x && (rc = build_tiles(b, block_x))) return rc;
+  b->way = flb_batch::kEstimated;
   b->mode = FLB_BATCH_PERSISTENT;
   b->persist_per_cu = blocks_per_cu;
   b->persist_chunk = chunk;
@@ -813,21 +819,28 @@ int flb_batch_step_timed(flb_batch* b, uint64_t nsteps, float* ms) {
 // For each tile order, times block sizes {64, 128, 256, 512} x {4, 16, 64
 // blocks per CU, one block per tile} with one launch per step, and the
 // persistent kernel at block sizes {256, 512} with 1, 2 or 4 resident blocks
-// per CU (as far as they fit), over `steps` steps each (the state advances),
-// and keeps the fastest.
+// per CU (as far as they fit), over `steps` steps each (the state advances); then
+// the passes, which none of these settings change, and keeps the fastest.
 // best_grid reports blocks of the launch (0: one per tile); a persistent
-// winner reports -(blocks per CU).
+// winner reports -(blocks per CU).  Where the passes win, the settings are the
+// fastest ones of the single steps that are left: calls of one step.
 int flb_batch_autotune(flb_batch* b, uint32_t steps, int32_t* best_block, int32_t* best_grid,
                        float* best_ms) {
   if (!b || steps == 0) return FLB_ERR_ARGUMENT;
   const int blocks[4] = {64, 128, 256, 512};
   const int per_cu[4] = {4, 16, 64, 0};
   const int chunk = b->graph_chunk;
-  float best = 1e30f;
-  int bb = b->block_x, bg = b->grid, bo = b->order;
-  bool bp = false;
+  struct Setting {
+    float ms = 1e30f;
+    int block, grid, order;
+    bool persistent = false;
+  } best, launched;
+  best.block = launched.block = b->block_x;
+  best.grid = launched.grid = b->grid;
+  best.order = launched.order = b->order;
   int rc = FLB_OK;
-  auto time_it = [&](float* ms) -> int {
+  auto time_it = [&](flb_batch::Way way, float* ms) -> int {
+    b->way = way;
     int r = flb_batch_step(b, 2);  // warm
     if (!r) r = flb_batch_step_timed(b, steps, ms);
     return r;
@@ -838,14 +851,8 @@ int flb_batch_autotune(flb_batch* b, uint32_t steps, int32_t* best_block, int32_
       for (int pc : per_cu) {
         if ((rc = flb_batch_configure(b, bx, pc * b->ncu, 0))) return rc;
         float ms = 0.0f;
-        if ((rc = time_it(&ms))) return rc;
-        if (ms < best) {
-          best = ms;
-          bb = bx;
-          bg = pc * b->ncu;
-          bo = order;
-          bp = false;
-        }
+        if ((rc = time_it(flb_batch::kSingle, &ms))) return rc;
+        if (ms < launched.ms) launched = Setting{ms, bx, pc * b->ncu, order, false};
       }
     for (int bx : {256, 512})
       for (int pc : {1, 2, 4}) {
@@ -854,25 +861,35 @@ int flb_batch_autotune(flb_batch* b, uint32_t steps, int32_t* best_block, int32_
         if (pc > cap) continue;
         if ((rc = flb_batch_configure_persistent(b, bx, pc, int(steps)))) return rc;
         float ms = 0.0f;
-        if ((rc = time_it(&ms))) return rc;
-        if (ms < best) {
-          best = ms;
-          bb = bx;
-          bg = pc;
-          bo = order;
-          bp = true;
-        }
+        if ((rc = time_it(flb_batch::kSingle, &ms))) return rc;
+        if (ms < best.ms) best = Setting{ms, bx, pc, order, true};
       }
   }
-  if ((rc = flb_batch_set_order(b, bo))) return rc;
-  if (bp) {
-    if ((rc = flb_batch_configure_persistent(b, bb, bg, chunk > 0 ? chunk : 100))) return rc;
-  } else if ((rc = flb_batch_configure(b, bb, bg, chunk))) {
+  if (launched.ms <= best.ms) best = launched;
+  flb_batch::Way way = flb_batch::kSingle;
+  if (b->shape.steps && steps > 1) {
+    if ((rc = flb_batch_set_order(b, launched.order)) ||
+        (rc = flb_batch_configure(b, launched.block, launched.grid, 0)))
+      return rc;
+    float ms = 0.0f;
+    if ((rc = time_it(flb_batch::kPasses, &ms))) return rc;
+    if (ms < best.ms) {
+      best = launched;
+      best.ms = ms;
+      way = flb_batch::kPasses;
+    }
+  }
+  if ((rc = flb_batch_set_order(b, best.order))) return rc;
+  if (best.persistent) {
+    if ((rc = flb_batch_configure_persistent(b, best.block, best.grid, chunk > 0 ? chunk : 100))) return rc;
+  } else if ((rc = flb_batch_configure(b, best.block, best.grid, chunk))) {
     return rc;
   }
-  if (best_block) *best_block = bb;
-  if (best_grid) *best_grid = bp ? -bg : bg;
-  if (best_ms) *best_ms = best / float(steps);
+  // Timed by calls of one step, the tuning says nothing of longer runs.
+  b->way = steps > 1 ? way : flb_batch::kEstimated;
+  if (best_block) *best_block = best.block;
+  if (best_grid) *best_grid = best.persistent ? -best.grid : best.grid;
+  if (best_ms) *best_ms = best.ms / float(steps);
   return FLB_OK;
 }
 

@@ -316,9 +316,10 @@ int flb_adjoint(flb_handle* h, const flb_adjoint_spec* spec, double* J, float* d
                 double* dj_duin, float* phase_ms);
 
 /* ------------------------------------------------------------ batch */
-/* Many independent monofluid SRT domains of uneven sizes advanced together, one
-   kernel launch per step for all of them, runs of steps replayed from HIP
-   graphs.  No reference counterpart (FlowLB runs one domain per process, each
+/* Many independent monofluid SRT domains of uneven sizes advanced together: one
+   kernel launch for all of them, per step or, in runs of two or more steps where
+   that is the faster way and every domain has four rows or more, per pass of two
+   to four steps; runs of steps replayed from HIP graphs.  No reference counterpart (FlowLB runs one domain per process, each
    step being launch + device synchronisation, src/cuda/runCuda.cu:473-490). */
 typedef struct flb_instance {
   uint32_t nx, ny;
@@ -342,7 +343,8 @@ enum { FLB_BATCH_ORDER_ROWS = 0, FLB_BATCH_ORDER_INSTANCE = 1, FLB_BATCH_ORDER_B
 int flb_batch_set_order(flb_batch* b, int32_t order);
 /* FLB_BATCH_LAUNCH: threads per block (multiple of 64), blocks of the
    grid-stride launch (0 = one block per tile), steps per captured graph (even;
-   0 = plain launches). */
+   0 = plain launches).  Block size, grid and tile order are those of single steps;
+   passes of several steps have their own. */
 int flb_batch_configure(flb_batch* b, int32_t block_x, int32_t grid, int32_t graph_chunk);
 /* FLB_BATCH_PERSISTENT: one cooperative launch runs up to `chunk` steps, its
    blocks_per_cu resident blocks per CU walking the tile list and meeting at a
@@ -351,10 +353,12 @@ int flb_batch_configure(flb_batch* b, int32_t block_x, int32_t grid, int32_t gra
    FLB_ERR_ARGUMENT when that many blocks cannot be resident together. */
 int flb_batch_configure_persistent(flb_batch* b, int32_t block_x, int32_t blocks_per_cu,
                                    int32_t chunk);
-/* Times tile orders x block sizes x grid sizes of both modes over `steps`
-   steps each (the state advances) and keeps the fastest (flb_batch_order
-   reports the order).  best_grid: blocks of the launch
-   (0 = one per tile), or -(blocks per CU) when the persistent mode won. */
+/* Times tile orders x block sizes x grid sizes of both modes, and the passes of
+   several steps, over `steps` steps each (the state advances) and keeps the
+   fastest (flb_batch_order reports the order).  best_grid: blocks of the launch
+   (0 = one per tile), or -(blocks per CU) when the persistent mode won.  Where the
+   passes won, the settings are the fastest of the single steps.  flb_batch_set_order
+   and the two configure calls end what it chose. */
 int flb_batch_autotune(flb_batch* b, uint32_t steps, int32_t* best_block, int32_t* best_grid,
                        float* best_ms_per_step);
 int flb_batch_step(flb_batch* b, uint64_t nsteps);
