@@ -571,9 +571,9 @@ namespace {
       return flb::set_error((h), FLB_ERR_DEVICE, std::string(#call) + ": " + hipGetErrorString(e_)); \
   } while (0)
 
-// Bounds what a handle keeps of its buffers after a call, a sixteenth of the
-// device's memory (18 GB of 288; a gradient of 2000 steps of 1024 x 256 takes
-// 6.3 GB in FP32, 12.6 GB in FP64).
+// Bounds what the handles of a device keep of their buffers after a call, a
+// thirty-second of its memory together (9 GB of 288; a gradient of 2000 steps of 1024 x
+// 256 takes 6.3 GB in FP32).
 struct TrimWork {
   flb_handle* h;
   ~TrimWork() {
@@ -582,7 +582,8 @@ struct TrimWork {
       (void)hipGetLastError();
       total = 0;
     }
-    h->work.trim(total / 16);
+    const size_t most = total / 32, others = flb::idle_elsewhere(h);
+    h->work.trim(most > others ? most - others : 0);
   }
 };
 
@@ -723,7 +724,7 @@ int flb_set_brinkman(flb_handle* h, const float* alpha) {
     return flb::set_error(h, FLB_ERR_UNSUPPORTED, "Brinkman drag needs a monofluid handle");
   if (!h->alpha) {
     void* v = nullptr;
-    ADJ_HIP(h, hipMalloc(&v, h->Nd * sizeof(float)));
+    ADJ_HIP(h, flb::device_malloc(&v, h->Nd * sizeof(float), h->device, nullptr));
     h->owned.push_back(v);
     h->alpha = static_cast<float*>(v);
     ADJ_HIP(h, hipMemsetAsync(v, 0, h->Nd * sizeof(float), h->stream));
@@ -734,11 +735,19 @@ int flb_set_brinkman(flb_handle* h, const float* alpha) {
 int flb_objective(flb_handle* h, const flb_adjoint_spec* sp, double* J) {
   int rc = check_adjoint_state(h, sp);
   if (rc) return rc;
+  const std::lock_guard<std::recursive_mutex> lock(h->in_use);
   using W = flb::Workspace;
   TrimWork trim{h};
-  uint8_t* saved = h->work.get<uint8_t>(W::kState, state_bytes(h, true));
-  double* d_j = h->work.get<double>(W::kSums, 2);
-  if (!saved || !d_j) return flb::set_error(h, FLB_ERR_MEMORY, "objective buffers");
+  uint8_t* saved = nullptr;
+  double* d_j = nullptr;
+  auto buffers = [&]() {
+    return (saved = h->work.get<uint8_t>(W::kState, state_bytes(h, true))) &&
+           (d_j = h->work.get<double>(W::kSums, 2));
+  };
+  if (!buffers()) {
+    h->work.trim(0);  // buffers of an earlier call may be what is in the way
+    if (!buffers()) return flb::set_error(h, FLB_ERR_MEMORY, "objective buffers");
+  }
   if ((rc = copy_state(h, saved, false, true))) return rc;
   ADJ_HIP(h, hipMemsetAsync(d_j, 0, sizeof(double), h->stream));
   rc = run_forward(h, sp->nsteps, sp, 1.0 / double(sp->t1 - sp->t0 + 1), d_j);
@@ -757,6 +766,7 @@ int flb_adjoint(flb_handle* h, const flb_adjoint_spec* sp, double* J, float* dj_
                 double* dj_duin, float* phase_ms) {
   int rc = check_adjoint_state(h, sp);
   if (rc) return rc;
+  const std::lock_guard<std::recursive_mutex> lock(h->in_use);
   const size_t N = h->Nd, Np = h->Np;  // device planes
   const uint64_t K = sp->ckpt, T = sp->nsteps;
   const uint64_t nseg = (T + K - 1) / K;
@@ -769,7 +779,10 @@ int flb_adjoint(flb_handle* h, const flb_adjoint_spec* sp, double* J, float* dj_
   if (budget == 0) {
     size_t free_b = 0, total_b = 0;
     ADJ_HIP(h, hipMemGetInfo(&free_b, &total_b));
-    budget = (free_b + h->work.held()) / 2;  // what the handle kept counts as free
+    // What handles keep between calls counts as free.
+    budget = (free_b + h->work.held() + flb::idle_elsewhere(h)) / 2;
+  } else if (h->work.size[flb::Workspace::kTrace] > budget) {
+    h->work.drop(flb::Workspace::kTrace);  // an earlier call's, larger than this one allows
   }
   const uint64_t resident = std::min<uint64_t>(nseg, budget / seg_bytes);
   const uint64_t first_res = nseg - resident;  // segments [0, first_res) are recomputed

@@ -218,7 +218,7 @@ PersistFn get_persistent(int storage) {
 
 }  // namespace flb
 
-struct flb_batch {
+struct flb_batch : flb::Kept {
   int storage = 0;
   int block_x = 256;
   int grid = 0;            // blocks of the grid-stride launch
@@ -254,10 +254,12 @@ struct flb_batch {
   flb::Tile* tiles = nullptr;
   uint32_t ntiles = 0;
   std::vector<void*> owned;
+  void* pops[2] = {nullptr, nullptr};  // the population arrays; the second for the passes
   hipGraphExec_t graph[4] = {};  // by the set it starts from
   int graph_set[4] = {};         // the set it ends at
   uint64_t t = 0;
   std::string err;
+  bool give_back() override;
 };
 
 namespace {
@@ -274,8 +276,7 @@ namespace {
 template <class T>
 int balloc(flb_batch* b, T** p, size_t count) {
   void* v = nullptr;
-  if (hipMalloc(&v, std::max<size_t>(count, 1) * sizeof(T)) != hipSuccess) {
-    (void)hipGetLastError();
+  if (flb::device_malloc(&v, std::max<size_t>(count, 1) * sizeof(T), b->device, b) != hipSuccess) {
     b->err = "hipMalloc of " + std::to_string(count * sizeof(T)) + " bytes failed";
     return FLB_ERR_MEMORY;
   }
@@ -455,7 +456,7 @@ int prepare_march(flb_batch* b, const flb_instance* in, size_t f_bytes) {
     (void)hipGetLastError();
     alt = nullptr;
   }
-  if (alt) b->owned.push_back(alt);
+  b->pops[1] = alt;
   const uint8_t* const base = static_cast<const uint8_t*>(b->host_inst[0].f);
   std::vector<flb::Params> sets;
   sets.reserve(4 * count);
@@ -477,7 +478,8 @@ int prepare_march(flb_batch* b, const flb_instance* in, size_t f_bytes) {
   b->model.kernel = b->forced ? flb::kMarchGeneral : flb::kMarchPlain;
   b->mb = 1e-6 * double(f_bytes);
   b->rule_shape = flb::march_shape(b->ncu, strip_rows, b->storage == 0 ? 4 : 2, false);
-  return set_shape(b, b->rule_shape);
+  if (set_shape(b, b->rule_shape)) b->rule_shape = flb::MarchShape{0, 0};  // no room: single steps
+  return FLB_OK;
 }
 
 int launch_step(flb_batch* b, int odd, bool mom) {
@@ -516,6 +518,22 @@ int advance(flb_batch* b, uint64_t t, uint64_t left, bool mom, int* done) {
   const bool last = mom && left == uint64_t(*done);
   return T ? launch_march(b, T, int(t & 1), last) : launch_step(b, int(t & 1), last);
 }
+
+}  // namespace
+
+// The population array that the current set does not name.
+bool flb_batch::give_back() {
+  if (!pops[1] || !pops[0]) return false;
+  (void)hipStreamSynchronize(stream);
+  drop_graph(this);
+  shape = rule_shape = flb::MarchShape{0, 0};
+  void*& other = pops[(set & 1) ^ 1];
+  (void)hipFree(other);
+  other = nullptr;
+  return true;
+}
+
+namespace {
 
 // Resident blocks per CU the persistent kernel can have at block size bx.
 int persistent_capacity(flb_batch* b, int bx, int* per_cu) {
@@ -571,10 +589,13 @@ const char* flb_batch_last_error(const flb_batch* b) { return b ? b->err.c_str()
 
 void flb_batch_destroy(flb_batch* b) {
   if (!b) return;
+  flb::forget(b);
   if (b->stream) (void)hipStreamSynchronize(b->stream);
   drop_graph(b);
   if (b->stream) (void)hipStreamDestroy(b->stream);
   for (void* v : b->owned) (void)hipFree(v);
+  for (void* v : b->pops)
+    if (v) (void)hipFree(v);
   delete b;
 }
 
@@ -601,6 +622,7 @@ int flb_batch_create(const flb_instance* in, uint32_t count, int32_t storage, in
   if (hipSetDevice(device) != hipSuccess) return FLB_ERR_DEVICE;
   flb_batch* b = new flb_batch();
   b->storage = storage;
+  b->device = device;
   auto bail = [&](int rc) {
     flb_batch_destroy(b);
     return rc;
@@ -635,10 +657,14 @@ int flb_batch_create(const flb_instance* in, uint32_t count, int32_t storage, in
       (rc = balloc(b, &pu0, 2 * tot_c)) || (rc = balloc(b, &pu1, 2 * tot_c)) ||
       (rc = balloc(b, &b->inst_sets, 4 * size_t(count))))
     return bail(rc);
+  b->pops[0] = f;
+  b->owned.erase(b->owned.begin());  // f, the first
   float* staging = nullptr;
   size_t max_n = 0;
   for (uint32_t i = 0; i < count; ++i) max_n = std::max(max_n, size_t(in[i].nx) * in[i].ny);
-  if (hipMalloc(&staging, 9 * max_n * sizeof(float)) != hipSuccess) return bail(FLB_ERR_MEMORY);
+  if (flb::device_malloc(reinterpret_cast<void**>(&staging), 9 * max_n * sizeof(float), device, b) !=
+      hipSuccess)
+    return bail(FLB_ERR_MEMORY);
   b->host_inst.resize(count);
   use_set(b, 0);
   std::vector<float> fs, hr, hu;
@@ -705,12 +731,14 @@ int flb_batch_create(const flb_instance* in, uint32_t count, int32_t storage, in
   if ((rc = prepare_march(b, in, tot_f * eb))) return bail(rc);
   b->grid = 8 * b->ncu;
   if ((rc = build_tiles(b, 256))) return bail(rc);
+  flb::keep(b);
   *out = b;
   return FLB_OK;
 }
 
 int flb_batch_configure(flb_batch* b, int32_t block_x, int32_t grid, int32_t graph_chunk) {
   if (!b) return FLB_ERR_ARGUMENT;
+  const std::lock_guard<std::recursive_mutex> lock(b->in_use);
   if (block_x % 64 || block_x < 64 || block_x > 1024 || grid < 0 || graph_chunk < 0 ||
       graph_chunk % 2)
     return FLB_ERR_ARGUMENT;
@@ -725,6 +753,7 @@ int flb_batch_configure(flb_batch* b, int32_t block_x, int32_t grid, int32_t gra
 
 int flb_batch_set_order(flb_batch* b, int32_t order) {
   if (!b || order < FLB_BATCH_ORDER_ROWS || order > FLB_BATCH_ORDER_BANDS) return FLB_ERR_ARGUMENT;
+  const std::lock_guard<std::recursive_mutex> lock(b->in_use);
   if (order == b->order) return FLB_OK;
   drop_graph(b);
   b->way = flb_batch::kEstimated;
@@ -735,6 +764,7 @@ int flb_batch_set_order(flb_batch* b, int32_t order) {
 int flb_batch_configure_persistent(flb_batch* b, int32_t block_x, int32_t blocks_per_cu,
                                    int32_t chunk) {
   if (!b) return FLB_ERR_ARGUMENT;
+  const std::lock_guard<std::recursive_mutex> lock(b->in_use);
   if (block_x % 64 || block_x < 64 || block_x > 1024 || blocks_per_cu < 1 || chunk < 1)
     return FLB_ERR_ARGUMENT;
   int cap = 0, rc;
@@ -756,6 +786,7 @@ int flb_batch_configure_persistent(flb_batch* b, int32_t block_x, int32_t blocks
 
 int flb_batch_step(flb_batch* b, uint64_t nsteps) {
   if (!b) return FLB_ERR_ARGUMENT;
+  const std::lock_guard<std::recursive_mutex> lock(b->in_use);
   int rc = FLB_OK;
   uint64_t left = nsteps;
   while (left > 0 && !rc) {
@@ -785,7 +816,9 @@ int flb_batch_step(flb_batch* b, uint64_t nsteps) {
 }
 
 int flb_test_batch_pass_shape(flb_batch* b, int32_t steps, uint32_t rows) {
-  if (!b || !b->rule_shape.steps || steps == 1 || steps > flb::kMarchMax || (steps > 1 && rows == 0))
+  if (!b) return FLB_ERR_ARGUMENT;
+  const std::lock_guard<std::recursive_mutex> lock(b->in_use);
+  if (!b->rule_shape.steps || steps == 1 || steps > flb::kMarchMax || (steps > 1 && rows == 0))
     return FLB_ERR_ARGUMENT;
   BAT_HIP(b, hipStreamSynchronize(b->stream));
   drop_graph(b);
@@ -827,6 +860,7 @@ int flb_batch_step_timed(flb_batch* b, uint64_t nsteps, float* ms) {
 int flb_batch_autotune(flb_batch* b, uint32_t steps, int32_t* best_block, int32_t* best_grid,
                        float* best_ms) {
   if (!b || steps == 0) return FLB_ERR_ARGUMENT;
+  const std::lock_guard<std::recursive_mutex> lock(b->in_use);
   const int blocks[4] = {64, 128, 256, 512};
   const int per_cu[4] = {4, 16, 64, 0};
   const int chunk = b->graph_chunk;
@@ -907,7 +941,7 @@ int flb_batch_read_populations(flb_batch* b, uint32_t i, float* f) {
   if (!b || !f || i >= b->host_inst.size()) return FLB_ERR_ARGUMENT;
   const flb::Params& p = b->host_inst[i];
   float* tmp = nullptr;
-  BAT_HIP(b, hipMalloc(&tmp, 9 * p.NL * sizeof(float)));
+  BAT_HIP(b, flb::device_malloc(reinterpret_cast<void**>(&tmp), 9 * p.NL * sizeof(float), b->device, nullptr));
   void (*conv)(const flb::Params*, uint32_t, float*) =
       b->storage == 1 ? flb::k_batch_to_f32<flb::StoreF16S>
                       : (b->storage == 2 ? flb::k_batch_to_f32<flb::StoreBF16S>

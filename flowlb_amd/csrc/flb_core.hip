@@ -140,9 +140,8 @@ template <class T>
 int dev_alloc(flb_handle* h, T** ptr, size_t count) {
   void* v = nullptr;
   const size_t bytes = std::max<size_t>(count, 1) * sizeof(T);
-  hipError_t e = hipMalloc(&v, bytes);
+  hipError_t e = flb::device_malloc(&v, bytes, h->device, nullptr);
   if (e != hipSuccess) {
-    (void)hipGetLastError();
     return fail(h, FLB_ERR_MEMORY, std::string("hipMalloc of ") + std::to_string(count * sizeof(T)) +
                                        " bytes failed: " + hipGetErrorString(e));
   }
@@ -339,30 +338,31 @@ int march_model(const flb_handle* h) {
 }
 
 // Sets a single-phase handle up for the multi-step pass.  It is left to single
-// steps (f_alt null) where the pass's rules do not hold (march_columns_io) or
-// the second population array would take more than a quarter of the memory
-// left (a program that fills the device with handles keeps its room).
-int prepare_march(flb_handle* h, const uint8_t* flags) {
+// steps (f_alt null) where the pass's rules do not hold (march_columns_io), where
+// the second population array would take more than a quarter of the memory left,
+// or where there is none (a program that fills the device with handles keeps its
+// room: device_malloc takes the array back).
+void prepare_march(flb_handle* h, const uint8_t* flags) {
   std::vector<uint8_t> io;
-  if (!flb::march_columns_io(flags, h->nx, h->ny, io)) return FLB_OK;
+  if (!flb::march_columns_io(flags, h->nx, h->ny, io)) return;
   const size_t bytes = 9 * h->Np * h->elem_bytes;
   size_t left = 0, total = 0;
   void* v = nullptr;
   if (hipMemGetInfo(&left, &total) != hipSuccess || bytes > left / 4 ||
       hipMalloc(&v, bytes) != hipSuccess) {
     (void)hipGetLastError();
-    return FLB_OK;
+    return;
   }
-  h->owned.push_back(v);
-  int rc;
   for (int T = flb::kMarchMin; T <= flb::kMarchMax; ++T) {
     std::vector<uint32_t> order;
     h->march_io[T] = flb::march_strips(h->nx, T, io, order);
-    if ((rc = dev_alloc(h, &h->march_order[T], order.size()))) return rc;
-    if ((rc = upload(h, h->march_order[T], order.data(), order.size() * sizeof(uint32_t)))) return rc;
+    if (dev_alloc(h, &h->march_order[T], order.size()) ||
+        upload(h, h->march_order[T], order.data(), order.size() * sizeof(uint32_t))) {
+      (void)hipFree(v);
+      return;
+    }
   }
   h->f_alt = v;
-  return FLB_OK;
 }
 
 flb::MarchShape march_shape(const flb_handle* h) {
@@ -442,11 +442,14 @@ int flb_get_layout(const flb_handle* h, uint32_t* pitch, uint64_t* plane) {
 
 void flb_destroy(flb_handle* h) {
   if (!h) return;
+  flb::forget(h);
   if (h->stream) {
     (void)hipStreamSynchronize(h->stream);
     (void)hipStreamDestroy(h->stream);
   }
   for (void* v : h->owned) (void)hipFree(v);
+  if (h->f) (void)hipFree(h->f);
+  if (h->f_alt) (void)hipFree(h->f_alt);
   if (h->box_host) (void)hipHostFree(h->box_host);
   for (hipEvent_t e : h->in_flight)
     if (e) (void)hipEventDestroy(e);
@@ -469,6 +472,7 @@ int flb_create(const flb_options* opt, const uint8_t* flags, uint32_t nx, uint32
   flb_handle* h = new (std::nothrow) flb_handle();
   if (!h) return FLB_ERR_MEMORY;
   h->opt = *opt;
+  h->device = opt->device;
   h->nx = nx;
   h->ny = ny;
   h->N = N;
@@ -503,6 +507,7 @@ int flb_create(const flb_options* opt, const uint8_t* flags, uint32_t nx, uint32
   int rc = FLB_OK;
   uint8_t* fbytes = nullptr;
   if ((rc = dev_alloc(h, &fbytes, 9 * h->Np * h->elem_bytes))) return bail(rc);
+  h->owned.pop_back();
   h->f = fbytes;
   const bool fs = opt->problem == FLB_FREE_SURFACE;
   const uint64_t Nd = h->Nd;
@@ -590,7 +595,7 @@ int flb_create(const flb_options* opt, const uint8_t* flags, uint32_t nx, uint32
     if ((rc = upload(h, h->tile_pub, pub.data(), tiles * sizeof(uint32_t)))) return bail(rc);
     if ((rc = reset_work(h))) return bail(rc);
   }
-  if (!fs && (rc = prepare_march(h, flags))) return bail(rc);
+  if (!fs) prepare_march(h, flags);
   if ((rc = dev_alloc(h, &h->rho_init, Nd))) return bail(rc);
   if ((rc = dev_alloc(h, &h->u_init, 2 * Nd))) return bail(rc);
   const flb::Params pu = params(h, kUtilBlock);
@@ -622,10 +627,8 @@ int flb_create(const flb_options* opt, const uint8_t* flags, uint32_t nx, uint32
     else initial_populations(nx, ny, rho0, u0, fsf);
     const size_t bytes = f64 ? fsd.size() * sizeof(double) : fsf.size() * sizeof(float);
     void* staging = nullptr;
-    if (hipMalloc(&staging, bytes) != hipSuccess) {
-      (void)hipGetLastError();
+    if (flb::device_malloc(&staging, bytes, h->device, nullptr) != hipSuccess)
       return bail(FLB_ERR_MEMORY);
-    }
     int r2 = upload(h, staging, f64 ? static_cast<const void*>(fsd.data()) : fsf.data(), bytes);
     if (!r2) {
       const flb::Params p = params(h, kUtilBlock);
@@ -642,6 +645,7 @@ int flb_create(const flb_options* opt, const uint8_t* flags, uint32_t nx, uint32
     (void)hipFree(staging);
     if (r2) return bail(r2);
   }
+  flb::keep(h);
   *out = h;
   return FLB_OK;
 }
@@ -862,6 +866,15 @@ static int enqueue_march(flb_handle* h, int T, bool moments, const flb::MarchTra
 
 }  // extern "C"
 
+bool flb_handle::give_back() {
+  if (!f_alt && !work.held()) return false;
+  (void)hipStreamSynchronize(stream);
+  work.trim(0);
+  if (f_alt) (void)hipFree(f_alt);
+  f_alt = nullptr;
+  return true;
+}
+
 namespace flb {
 bool march_columns_io(const uint8_t* flags, uint32_t nx, uint32_t ny, std::vector<uint8_t>& io) {
   if (ny < uint32_t(kMarchMax)) return false;
@@ -921,6 +934,57 @@ MarchShape march_shape(int cus, uint64_t strip_rows, int elem_bytes, bool heavy)
     return MarchShape{2, uint32_t(std::min<uint64_t>(std::max<uint64_t>(rows, least), most))};
   return MarchShape{rows < least ? 3 : 4,
                     uint32_t(std::min<uint64_t>(std::max<uint64_t>(rows, least), most))};
+}
+
+namespace {
+// Never destroyed: a program may destroy its last handles after its statics.
+struct KeptList {
+  std::mutex lock;
+  std::vector<Kept*> all;
+};
+KeptList& kept_list() {
+  static KeptList* const list = new KeptList;
+  return *list;
+}
+}  // namespace
+
+void keep(Kept* k) {
+  KeptList& l = kept_list();
+  const std::lock_guard<std::mutex> lock(l.lock);
+  l.all.push_back(k);
+}
+
+void forget(Kept* k) {
+  KeptList& l = kept_list();
+  const std::lock_guard<std::mutex> lock(l.lock);
+  l.all.erase(std::remove(l.all.begin(), l.all.end(), k), l.all.end());
+}
+
+size_t idle_elsewhere(const Kept* self) {
+  KeptList& l = kept_list();
+  const std::lock_guard<std::mutex> lock(l.lock);
+  size_t n = 0;
+  for (const Kept* k : l.all)
+    if (k != self && k->device == self->device) n += k->idle;
+  return n;
+}
+
+hipError_t device_malloc(void** p, size_t bytes, int device, const Kept* self) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipSuccess) return e;
+  (void)hipGetLastError();
+  KeptList& l = kept_list();
+  const std::lock_guard<std::mutex> lock(l.lock);
+  bool any = false;
+  for (Kept* k : l.all) {
+    if (k == self || k->device != device || !k->in_use.try_lock()) continue;
+    any = k->give_back() || any;
+    k->in_use.unlock();
+  }
+  if (!any) return e;
+  e = hipMalloc(p, bytes);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
 }
 
 hipError_t Staging::init(size_t bytes) {
@@ -1116,6 +1180,7 @@ extern "C" {
 
 int flb_step(flb_handle* h, uint64_t nsteps) {
   if (!h) return FLB_ERR_ARGUMENT;
+  const std::lock_guard<std::recursive_mutex> lock(h->in_use);
   const bool throttle = h->box_host != nullptr;
   constexpr uint64_t G = flb_handle::kGroup, R = flb_handle::kRing;
   // Passes of the shape's steps, and of what is left of them at the end, where they
@@ -1261,7 +1326,7 @@ template <class T>
 int read_pops(flb_handle* h, T* f) {
   if (!h || !f) return FLB_ERR_ARGUMENT;
   T* tmp = nullptr;
-  FLB_HIP(h, hipMalloc(&tmp, 9 * h->N * sizeof(T)));
+  FLB_HIP(h, flb::device_malloc(reinterpret_cast<void**>(&tmp), 9 * h->N * sizeof(T), h->device, nullptr));
   const flb::Params p = params(h, kUtilBlock);
   if (std::is_same<T, double>::value)
     hipLaunchKernelGGL(flb::get_pop_to_f64(h->opt.storage), dim3(p.nblocks), dim3(kUtilBlock), 0,
@@ -1309,7 +1374,7 @@ int write_pops(flb_handle* h, const T* f) {
     for (size_t n = 0; n < N; ++n) fsh[q * N + n] = f[q * N + n] - w;
   }
   T* tmp = nullptr;
-  FLB_HIP(h, hipMalloc(&tmp, 9 * N * sizeof(T)));
+  FLB_HIP(h, flb::device_malloc(reinterpret_cast<void**>(&tmp), 9 * N * sizeof(T), h->device, nullptr));
   int rc = upload(h, tmp, fsh.data(), 9 * N * sizeof(T));
   if (!rc) {
     const flb::Params p = params(h, kUtilBlock);
@@ -1363,7 +1428,7 @@ int flb_mass(flb_handle* h, double* total) {
 int flb_flag_histogram(flb_handle* h, uint64_t* counts) {
   if (!h || !counts) return FLB_ERR_ARGUMENT;
   unsigned long long* d = nullptr;
-  FLB_HIP(h, hipMalloc(&d, 256 * sizeof(unsigned long long)));
+  FLB_HIP(h, flb::device_malloc(reinterpret_cast<void**>(&d), 256 * sizeof(unsigned long long), h->device, nullptr));
   int rc = FLB_OK;
   hipError_t e = hipMemsetAsync(d, 0, 256 * sizeof(unsigned long long), h->stream);
   if (e == hipSuccess) {

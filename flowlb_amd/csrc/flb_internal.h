@@ -2,6 +2,8 @@
 // of libflbcore.so (not part of the public ABI).
 #pragma once
 
+#include <atomic>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -120,15 +122,38 @@ struct Staging {
 }  // namespace flb
 
 namespace flb {
+// Device memory that a handle or batch holds for speed alone: the second population
+// array, the buffers of the last gradient.  Where an allocation of the library
+// finds no room, the others on that device give theirs back (device_malloc), so
+// that what fits without such memory still fits.  Any thread may ask for it: calls
+// that use it hold in_use, and who uses it keeps it.
+struct Kept {
+  std::recursive_mutex in_use;
+  int device = 0;
+  std::atomic<size_t> idle{0};  // bytes held between calls (Workspace)
+  // With in_use held.  Waits for the work on the memory; returns whether any was freed.
+  virtual bool give_back() = 0;
+
+ protected:
+  ~Kept() = default;
+};
+void keep(Kept* k);    // from now on others may ask
+void forget(Kept* k);  // from now on they do not; waits for one who is asking
+size_t idle_elsewhere(const Kept* self);  // on self's device
+// hipMalloc; without room, after the others on the device, and owner unless its
+// calling thread holds in_use (self), gave back what they keep.
+hipError_t device_malloc(void** p, size_t bytes, int device, const Kept* self);
+
 // Device buffers a handle keeps between calls that need the same ones
 // (objective, gradient), by slot.  Allocating and freeing 2 GB takes 0.6 ms, and
-// now and then 60 to 200 ms.  Freed with the handle; after each call
-// trim() gives back what exceeds its bound.
+// now and then 60 to 200 ms.  After each call trim() gives back what exceeds a
+// thirty-second of the device's memory (9 GB of 288) for all handles together.
 struct Workspace {
   enum Slot { kCheckpoints, kState, kTrace, kTraceOnce, kAdjoint, kAdjointAlt, kDensity, kVelocity,
               kAlpha, kSums, kColumn, kSlots };
   void* ptr[kSlots] = {};
   size_t size[kSlots] = {};
+  Kept* owner = nullptr;
   Workspace() = default;
   Workspace(const Workspace&) = delete;
   Workspace& operator=(const Workspace&) = delete;
@@ -138,17 +163,19 @@ struct Workspace {
   T* get(Slot s, size_t count) {
     const size_t bytes = (count ? count : 1) * sizeof(T);
     if (size[s] < bytes) {
-      if (ptr[s]) (void)hipFree(ptr[s]);
-      ptr[s] = nullptr;
-      size[s] = 0;
-      if (hipMalloc(&ptr[s], bytes) != hipSuccess) {
-        (void)hipGetLastError();
+      drop(s);
+      if (device_malloc(&ptr[s], bytes, owner->device, owner) != hipSuccess) {
         ptr[s] = nullptr;
         return nullptr;
       }
       size[s] = bytes;
     }
     return static_cast<T*>(ptr[s]);
+  }
+  void drop(Slot s) {
+    if (ptr[s]) (void)hipFree(ptr[s]);
+    ptr[s] = nullptr;
+    size[s] = 0;
   }
   size_t held() const {
     size_t n = 0;
@@ -161,15 +188,14 @@ struct Workspace {
       int big = 0;
       for (int s = 1; s < kSlots; ++s)
         if (size[s] > size[big]) big = s;
-      (void)hipFree(ptr[big]);
-      ptr[big] = nullptr;
-      size[big] = 0;
+      drop(Slot(big));
     }
+    if (owner) owner->idle = held();
   }
 };
 }  // namespace flb
 
-struct flb_handle {
+struct flb_handle : flb::Kept {
   flb_options opt{};
   flb::Workspace work;
   flb::Staging staging;
@@ -181,7 +207,7 @@ struct flb_handle {
   int elem_bytes = 4;   // bytes per stored population
   int field_bytes = 4;  // bytes per element of the cell fields (8 for FP64)
   hipStream_t stream = nullptr;
-  void* f = nullptr;
+  void* f = nullptr;  // with f_alt not in `owned`: passes exchange the two
   // Single phase, the multi-step pass (flb_march.h): second population array
   // (null where the pass is not used) and, per number of steps, the strips with
   // those that hold an inlet or outlet column first and the number of these.
@@ -238,6 +264,9 @@ struct flb_handle {
   float inv_tau = 0.0f;
   std::vector<void*> owned;
   std::string err;
+
+  flb_handle() { work.owner = this; }
+  bool give_back() override;
 };
 
 

@@ -23,6 +23,15 @@
  * stream-collide launch from a bounding box the device published a few steps
  * earlier, so flb_step may wait for the step 8 back); the readback calls
  * (flb_read*, flb_mass) and flb_sync wait for it.
+ *
+ * Memory held for speed alone: single-phase handles and batches have a second
+ * population array, with which runs of several steps take fewer passes over
+ * memory, unless it would have taken more than a quarter of what was free at their
+ * creation; handles keep the buffers of their last flb_objective or flb_adjoint
+ * call, up to a thirty-second of the device's memory for all of them together.
+ * Where an allocation of this library finds no room, handles and batches of the
+ * process that are in no call of their own give both back, and go on by single
+ * steps with the same results.  flb_destroy and flb_batch_destroy free all.
  */
 #ifndef FLB_CORE_H
 #define FLB_CORE_H
