@@ -91,9 +91,9 @@ __device__ __forceinline__ void feq_adjoint(const Moments& m, double rho, double
   uby = rho * (3.0 * (m.y - uy * m.s) + 9.0 * qy);
 }
 
-// 1 / v for a density or 1 + alpha / 2, to the last place: the hardware's estimate
-// and two Newton steps, half the instructions of a division, which also scales
-// operands near the ends of the range.
+// 1 / v for a density or 1 + alpha / 2, to within a unit in the last place: the
+// hardware's estimate and two Newton steps, half the instructions of a division,
+// which rounds correctly and scales operands near the ends of the range.
 __device__ __forceinline__ double reciprocal(double v) {
   double r = __builtin_amdgcn_rcp(v);
   r = fma(r, fma(-v, r, 1.0), r);
@@ -269,7 +269,7 @@ __global__ void __launch_bounds__(256) k_adjoint_step(const Params p, const AdjP
 // beside from one iteration ago, those below from two.  A wall, which emits what
 // it received in the opposite direction, exchanges the adjoints.  A single step
 // moves 196 bytes per cell, 144 of them the adjoint populations, which a pass of
-// three moves once; 1024 x 256, FP32: 10.2 us per step one by one, 5.9 in passes
+// three moves once; 1024 x 256, FP32: 9.8 us per step one by one, 6.0 in passes
 // (140 FP64 instructions of about 200 per step-row, halo rows included: the
 // vector units bind, except on grids beyond the caches).
 struct AdjMarch {

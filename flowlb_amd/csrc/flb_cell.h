@@ -358,7 +358,7 @@ __device__ __forceinline__ bool apply_force(const Params& p, bool use_force, boo
 // Square root, correctly rounded (as sqrtf) for zero and normal x above 2^-100:
 // the hardware's value s is within one unit in the last place, and the sign of
 // x - s t for its neighbours t, exact in a fused multiply-add, tells which of the
-// three is nearest.  Nine instructions; sqrtf takes fifteen, scaling x first
+// three is nearest (Tuckerman's test).  Nine instructions; sqrtf takes fifteen, scaling x first
 // for the sake of smaller ones.
 __device__ __forceinline__ float root(float x) {
   const float s = __builtin_amdgcn_sqrtf(x);

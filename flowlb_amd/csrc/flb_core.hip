@@ -903,29 +903,30 @@ uint32_t march_strips(uint32_t nx, int steps, const std::vector<uint8_t>& io,
   return uint32_t(split - order.begin());
 }
 
-// Shape of the passes of a run of steps.
+// Shape of the passes of a run of steps (us per step of one handle alone, one run).
 //
 // Rows per chunk.  A wavefront's chunk of r rows takes r + 2 (T - 1)
 // iterations and T (r + T - 1) step-rows, so long chunks waste less, while the
-// chip needs wavefronts on its 1024 SIMDs.  Measured with T = 4, us per step: 2048 x 512
-// FP32 (36 strips) 8.3, 7.2, 7.2, 8.6, 9.2 with 4, 8, 12, 16, 24 rows: best near
-// 1.5 wavefronts per SIMD (12 rows).  Where that gives long chunks, the chip
-// runs several rounds of wavefronts anyway and FP32 wants them short, so that
-// fewer rows are in flight: 8192 x 2048 79.8, 83.2, 84.3, 90.5 with 16, 24, 36,
-// 64 rows; FP16S, which is bound by the vector units, 70.6, 68.6, 66.1, 74.6
-// (5001 x 1001: 32 rows 2 to 10 % ahead of 36 or 40, which end a round short).
-// Below four rows nothing is gained (512 x 128: 3.3 us with 1 to 4).
+// chip needs wavefronts on its 1024 SIMDs.  With T = 4, 2048 x 512 FP32 (36 strips) 9.5,
+// 8.3, 8.0, 9.3, 9.6 with 4, 8, 12, 16, 24 rows: best near 1.5 wavefronts per SIMD (12
+// rows).  Where that gives long chunks, the chip runs several rounds of wavefronts
+// anyway and FP32 wants them short, so that fewer rows are in flight: 8192 x 2048 79.6,
+// 83.3, 83.4, 90.1 with 16, 24, 36, 64 rows; FP64 150.6, 147.3, 149.1 with 8, 16, 32
+// (4096 x 1024 42.5, 40.4, 45.3); FP16S, which is bound by the vector units, 70.1, 65.5,
+// 65.2, 68.0, 69.6 with 16, 24, 32, 40, 64 (5001 x 1001 25.6, 23.8, 24.2, 29.1 with 16, 24,
+// 32, 40, which end a round short).  Below four rows little is gained (512 x 128: 3.0,
+// 3.0, 3.4 with 1, 2, 4, and 1.3, 1.3, 1.4 with three handles side by side).
 //
 // Steps per pass.  T = 4 moves the fewest bytes and was the fastest from
-// 2048 x 512 on (8192 x 2048 FP32 80 us per step, with T = 3 110, with T = 2
-// about 150; single steps 196).  Grids that give less than 1.5 wavefronts per
+// 2048 x 512 on (8192 x 2048 FP32 79.6, with T = 3 109.4, with T = 2 145.0; FP64 147.3
+// against 189.6 with T = 3, 4096 x 1024 40.4 against 51.5, with a force, where T = 3
+// spills nothing, 43.6 against 53.8).  Grids that give less than 1.5 wavefronts per
 // SIMD at four rows are bound by the chain of a wavefront, T (r + T - 1)
-// step-rows: T = 3 takes 3.1 us per step on 512 x 128 and 3.5 on 1024 x 256,
-// T = 4 3.4 and 4.0.  The subgrid model (heavy) adds two thirds to the
-// instructions of a step; in 16-bit storage, where the bytes were never the bound,
-// the halo then costs more than the bytes saved: 5001 x 1001 BF16S 30.7, 33.8, 34.4
-// with T = 2, 3, 4 (with TRT 36.6 with T = 2, single steps 42; FP32 keeps T = 4:
-// 46.9, 33.9, 33.2).
+// step-rows: T = 3 takes 3.4 on 512 x 128 and 4.4 on 1024 x 256, T = 4 3.8 and 4.5.  The
+// subgrid model (heavy) adds two thirds to the instructions of a step; in 16-bit
+// storage, where the bytes were never the bound, the halo then costs more than
+// the bytes saved: 5001 x 1001 BF16S 32.4, 34.2, 34.7 with T = 2, 3, 4, with TRT 38.3, 41.3,
+// 42.4 (FP32 keeps T = 4: with TRT 48.4, 40.2, 40.3).
 MarchShape march_shape(int cus, uint64_t strip_rows, int elem_bytes, bool heavy) {
   const uint64_t waves = uint64_t(cus) * 6;  // 1.5 per SIMD
   const uint32_t least = 4, most = elem_bytes == 2 && !heavy ? 32 : 16;
@@ -1126,9 +1127,6 @@ void host_initial_populations(uint32_t nx, uint32_t ny, const float* rho0, const
 int set_error(flb_handle* h, int code, const std::string& msg) { return fail(h, code, msg); }
 Params make_params(const flb_handle* h, int bx) { return params(h, bx); }
 int handle_block_x(const flb_handle* h) { return block_x(h); }
-int enqueue_step_ex(flb_handle* h, bool moments, hipEvent_t* ev) {
-  return enqueue_step(h, moments, ev);
-}
 int enqueue_march_ex(flb_handle* h, int T, bool moments, const MarchTrace* trace) {
   return enqueue_march(h, T, moments, trace);
 }
@@ -1153,11 +1151,11 @@ MarchGrid march_grid(const flb_handle* h, int T, uint32_t rows, uint32_t io_rows
 // wavefront on a SIMD and no less with two, so its time is the longest SIMD's.
 // Blocks that share a CU then cost more than longer chunks, as long as the grid
 // is small: of the chunks of up to 8 rows, the shortest whose blocks take a CU
-// each.  1024 x 256, us per step in reverse, 3 steps: 7.7, 5.9, 6.3, 7.2 with 4, 5,
-// 6, 8 rows (320, 252, 216, 160 blocks; single steps 10.2).  Larger grids are bound by
-// memory and want the wavefronts: 2048 x 512 19.7, 17.5, 20.4 with 8, 12, 16
-// rows (single steps 35.6).  Where two or three rows do, a pass of 2 steps has
-// the shorter chain: 256 x 64 3.4, against 4.0 with 3 steps (single steps 5.4).
+// each.  1024 x 256, us per step in reverse, 3 steps: 7.8, 6.0, 6.4, 7.3 with 4, 5,
+// 6, 8 rows (320, 252, 216, 160 blocks; single steps 9.8).  Larger grids are bound by
+// memory and want the wavefronts: 2048 x 512 20.3, 17.5, 20.4 with 8, 12, 16
+// rows (single steps 35.7).  Where two or three rows do, a pass of 2 steps has
+// the shorter chain: 256 x 64 3.5, against 4.2 with 3 steps (single steps 5.4).
 MarchShape adjoint_shape(const flb_handle* h) {
   if (h->reverse_shape.steps >= 0) return h->reverse_shape;
   for (uint32_t r = 2; r <= 8; ++r) {

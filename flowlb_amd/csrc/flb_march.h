@@ -24,11 +24,13 @@
 // one pass move about a third of that and the vector units become the bound: about
 // 110 instructions per step and row of 64 columns, 10 % of them for halo columns.
 // A pass of four over 8192 x 2048 in FP32 reads 966 MB, 1.6 times the populations
-// (22 rows for a chunk of 16, 64 columns for 58), and writes 628 MB.  Measured, us
-// per step, single steps / passes: 8192 x 2048 FP32 226 / 77 (4.7 TB/s of that
-// traffic, 0.7 of the vector rate), FP16S 118 / 62, 2001 x 401 FP64 16.4 / 9.2;
-// 512 x 128 FP32 3.8 / 3.3 for one handle alone and 3.7 / 1.3 with
-// three handles stepping side by side.
+// (22 rows for a chunk of 16, 64 columns for 58), and writes 628 MB.  Measured in
+// one run, us per step, single steps / passes of one handle alone, and in brackets
+// of three stepping side by side: 8192 x 2048 FP32 201 / 80 (5.0 TB/s of that traffic,
+// 0.7 of the vector rate) [233 / 76], FP16S 119 / 65 [116 / 57], FP64 432 / 148 [480 /
+// 153], 2001 x 401 FP64 with a force 18.7 / 12.3 [16.8 / 8.9], 1024 x 256 FP32 6.2 / 4.0
+// [3.3 / 2.1], 512 x 128 FP32 4.9 / 3.5 [3.3 / 1.4].  Where single steps are the faster
+// way they are taken: flb_cost.h.
 #pragma once
 
 #include "flb_cell.h"
@@ -217,7 +219,12 @@ struct Held<StoreBF16S> {
 // or drag, everything by the handle's options, and SRT with drag (TRACE too).
 enum : int { kMarchPlain = 0, kMarchForced = 1, kMarchUnforced = 2, kMarchGeneral = 3,
              kMarchDrag = 4 };
-// Wavefronts per SIMD the pass is compiled for (its registers: 128, 168, 256).
+// Wavefronts per SIMD the pass is compiled for (its registers: 128, 168, 256).  The
+// interior path fits these with no scratch memory; the inlet/outlet path in the same
+// kernel spills in passes of four in the plain model (10 to 14 registers in FP32 and
+// 16-bit storage), with a force (24 to 26, and 8 to 12 in passes of three) and in FP64
+// with drag or every option (10 to 22).  FP64 gains from four steps all the same
+// (march_shape).
 template <class S, int MODEL>
 constexpr int march_occupancy() {
   return S::kBytes > 4 ? 2 : (MODEL >= kMarchUnforced ? 3 : 4);

@@ -176,7 +176,10 @@ int flb_write_populations_f64(flb_handle* h, const double* f);
    element x + y * pitch of a plane of `plane` elements, and u holds the ux
    plane followed by the uy plane (flb_get_layout).  They stay valid until
    flb_destroy; the flag buffer of a free-surface handle alternates every
-   step, so query it again after stepping. */
+   step, so query it again after stepping.  At every step inlet cells take the
+   velocity they prescribe from u and outlet cells the density they keep from rho;
+   nothing else that is written there is read.  Which cells are inlets and outlets
+   is fixed by the flags given to flb_create. */
 int flb_device_fields(flb_handle* h, void** d_u, void** d_rho, void** d_flags, void** d_phi);
 
 /* Total fluid mass in FP64: stored mass plus the excess-mass shares that the
@@ -254,8 +257,10 @@ int flb_get_layout(const flb_handle* h, uint32_t* pitch, uint64_t* plane);
 
 /* Enqueue nsteps steps between two HIP events on the handle's stream and
    return the elapsed device time in ms.  With per_kernel_ms non-NULL (array of
-   FLB_NUM_KERNELS floats) each kernel launch is bracketed by its own events and
-   the summed device time per kernel is returned instead.  FLB_K_FS_UPDATE is
+   FLB_NUM_KERNELS floats) the steps go one by one, each kernel launch bracketed by
+   its own events, and the summed device time per kernel is returned instead (of a
+   single-phase handle the kernel of single steps, not that of the passes of
+   several that flb_step may run).  FLB_K_FS_UPDATE is
    the one launch that runs free-surface passes 2, 3 and 4
    (d_FreeSurface2D_2/_3/_4, src/cuda/lbmKernel2D.cu:123-303). */
 enum { FLB_K_STREAM_COLLIDE = 0, FLB_K_FS1 = 1, FLB_K_FS_UPDATE = 2, FLB_NUM_KERNELS = 3 };
