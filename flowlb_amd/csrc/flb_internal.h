@@ -84,7 +84,7 @@ namespace flb {
 // through the buffers (54 GB/s over the bus, 70 GB/s for the host's copy).
 //
 // The runtime copies by itself (direct) where that is the faster way:
-//  - memory the driver knows, as a caller's pinned buffers, needs no second copy:
+//  - memory the HIP runtime knows, as a caller's pinned buffers, needs no second copy:
 //    u and rho of 1024 x 512 cells 0.13 ms, through the buffers 0.34 (as a strided
 //    copy also where the rows have no padding: 64 x 16 18 us, as a plain one 25);
 //  - contiguous copies of middling size, which the runtime stages as well: to the
@@ -117,7 +117,7 @@ struct Staging {
  private:
   bool reserve(size_t bytes);
   void release();
-  static bool known(const void* host);  // to the driver
+  static bool known(const void* host);  // to the runtime
 };
 }  // namespace flb
 
